@@ -14,6 +14,7 @@ const SOURCES: [&str; 7] = [
     "lrq_quant.hip",
     "lrq_gemm.hip",
     "lrq_gemm_mid.hip",
+    "lrq_gemm_w8.hip",
     "lrq_skinny.hip",
     "lrq_lora.hip",
     "lrq_api.hip",

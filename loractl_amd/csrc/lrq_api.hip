@@ -437,7 +437,7 @@ int lrq_probe_stream_read(lrq_ctx* c, const void* data, int64_t bytes) {
 }
 
 int lrq_debug_gemm_path(int path) {
-  if (path < 0 || path > 5) return LRQ_EINVAL;
+  if (path < 0 || path > 7) return LRQ_EINVAL;
   set_gemm_path(path);
   return LRQ_OK;
 }
@@ -456,12 +456,13 @@ const char* lrq_last_error(const lrq_ctx* c) { return c ? c->err : "null context
 // partials (both jobs counted).
 static int64_t fold_fwd_floats(int64_t m, int64_t n, int64_t k, int rp) {
   const int64_t G = (m + 63) / 64, fs = (k + MID_FOLD_KT - 1) / MID_FOLD_KT;
-  return round_up(fs * G * 64 * rp, 64) + mid_split_plan(m, n, k).floats;
+  return round_up(fs * G * 64 * rp, 64) + mid_split_plan(m, n, k, SIDE_FWD).floats;
 }
 static int64_t fold_bwd_floats(int64_t m, int64_t n, int64_t k, int rp) {
   const int64_t G = (m + 63) / 64, fs = (n + MID_FOLD_KT - 1) / MID_FOLD_KT;
-  const LoraPlan tpb = mid_tn_plan(m, n, rp), tpa = mid_tn_plan(m, k, rp);
-  return round_up(fs * G * 64 * rp, 64) + round_up(mid_split_plan(m, k, n).floats, 64) +
+  const int lds = mid_tn_lds(m, k, n);
+  const LoraPlan tpb = mid_tn_plan(m, n, k, rp, lds), tpa = mid_tn_plan(m, k, n, rp, lds);
+  return round_up(fs * G * 64 * rp, 64) + round_up(mid_split_plan(m, k, n, SIDE_BWD).floats, 64) +
          (tpb.splits > 1 ? (int64_t)tpb.splits * n * rp : 0) + (tpa.splits > 1 ? (int64_t)tpa.splits * k * rp : 0);
 }
 
@@ -708,8 +709,8 @@ static int fwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t 
     const int64_t G = (m + 63) / 64, fs = (w->k + MID_FOLD_KT - 1) / MID_FOLD_KT;
     // (and the tiles' depth ranges, if any: partials after t's, counters
     // after the fold's)
-    const MidSplit ms = mid_split_plan(m, w->n, w->k);
-    if (r % 8 == 0 && r <= 32 && gemm_mid_tokens(m, w->n, w->k) > 0 && aligned16(a) && t_out && aligned16(t_out) &&
+    const MidSplit ms = mid_split_plan(m, w->n, w->k, SIDE_FWD);
+    if (r % 8 == 0 && r <= 32 && gemm_mid_tokens(m, w->n, w->k, SIDE_FWD) > 0 && aligned16(a) && t_out && aligned16(t_out) &&
         2 * G + ms.tiles <= SK_MAX_NB) {
       const int64_t fp = round_up(fs * G * 64 * rp, 64);
       LRQ_TRY(acquire_ws(c, src, (size_t)(fp + ms.floats) * 4, &ws, &cnt));
@@ -838,16 +839,18 @@ static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const ui
     // launch by workgroups ahead of the tiles (partials after the LoRA
     // workspace)
     const int64_t G = (m + 63) / 64, fs = (w->n + MID_FOLD_KT - 1) / MID_FOLD_KT;
-    const bool fold = !few && dx && r % 8 == 0 && r <= 32 && gemm_mid_tokens(m, w->k, w->n) > 0 && aligned16(a) &&
-                      2 * G + mid_split_plan(m, w->k, w->n).tiles <= SK_MAX_NB;
+    const bool fold = !few && dx && r % 8 == 0 && r <= 32 && gemm_mid_tokens(m, w->k, w->n, SIDE_BWD) > 0 && aligned16(a) &&
+                      2 * G + mid_split_plan(m, w->k, w->n, SIDE_BWD).tiles <= SK_MAX_NB;
     // and the weight gradients by workgroups after its tiles, in token
     // slices that fit its LDS (their counters after the fold's, partials
     // after u's)
-    const LoraPlan tpb = fold ? mid_tn_plan(m, w->n, rp) : LoraPlan{}, tpa = fold ? mid_tn_plan(m, w->k, rp) : LoraPlan{};
+    const int tlds = mid_tn_lds(m, w->k, w->n);
+    const LoraPlan tpb = fold ? mid_tn_plan(m, w->n, w->k, rp, tlds) : LoraPlan{};
+    const LoraPlan tpa = fold ? mid_tn_plan(m, w->k, w->n, rp, tlds) : LoraPlan{};
     const int64_t tb_floats = (db && tpb.splits > 1) ? (int64_t)tpb.splits * w->n * rp : 0;
     const int64_t ta_floats = (da && tpa.splits > 1) ? (int64_t)tpa.splits * w->k * rp : 0;
     // the tiles' depth ranges, if any (their partials and counters first)
-    const MidSplit ms = fold ? mid_split_plan(m, w->k, w->n) : MidSplit{1, 0, 0, 0};
+    const MidSplit ms = fold ? mid_split_plan(m, w->k, w->n, SIDE_BWD) : MidSplit{1, 0, 0, 0};
     const bool fold_tn = fold && (da || db) && tpb.splits > 0 && tpa.splits > 0 &&
                          2 * G + ms.tiles + TN_WAVES * ((db ? tpb.tiles : 0) + (da ? tpa.tiles : 0)) <= SK_MAX_NB;
     const int64_t fp_floats = round_up(fs * G * 64 * rp, 64);

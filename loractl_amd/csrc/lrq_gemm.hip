@@ -652,51 +652,75 @@ hipError_t run_fmt(hipStream_t st, int fmt, bool r192, const GemmArgs& a) {
 }
 
 // Which GEMM kernel a shape takes: the 256-token tiles above (split in
-// depth when they are too few), or lrq_gemm_mid.hip's 64-row tiles of 64 or
-// 128 tokens over the whole depth, two workgroups per CU. The choice is the
-// smaller modelled time, in microseconds, with constants measured on MI355X
-// (fwd and input gradient of the C1, C3, C5 and north-star shapes, every
-// path forced in turn):
-//   - a 256 x 256 x 64 step of the large tiles takes 1.86 us (0.8 of that
+// depth when they are too few), lrq_gemm_mid.hip's 64-row x 64-token tiles,
+// two workgroups per CU, or lrq_gemm_w8.hip's 128-token tiles of 128 or 256
+// rows, one workgroup per CU. The choice is the smallest modelled time, in
+// microseconds, with constants measured on MI355X (every path forced in turn
+// over the shapes of the 3072-wide MMDiT and the 2560-wide decoder):
+//   - a 256 x 256 x 64 step of the large tiles takes 1.75 us (0.8 of that
 //     for 192-row tiles); a split shape adds its f32 partials, written and
 //     read once at about 4 TB/s, and the reduction launch;
-//   - a 64-wide depth block of a mid tile takes MID_T1 us when its
-//     workgroup has the CU to itself and MID_T2 us each when two share it
-//     (64 tokens: 0.342 / 0.423, 128 tokens: 0.441 / 0.696); the tiles are
-//     dealt over the CUs, two at a time;
-//   - a mid tile may split its depth into S <= MID_MAX_SPLIT ranges (one
-//     workgroup each, whole rounds of MID_MST stages) when its tiles leave
-//     CUs idle; the ranges' accumulators meet in the launch, about
-//     MID_FINISH_US more, and S > 1 must model at least a tenth faster.
-constexpr double LARGE_STEP_US = 1.86;
-// per variant MID_64, MID_128: tile tokens, block us alone and shared, and
-// a fixed cost per round of tiles
-constexpr int MID_T[3] = {0, 64, 128};
-constexpr double MID_T1[3] = {0, 0.342, 0.441}, MID_T2[3] = {0, 0.423, 0.696};
-constexpr double MID_FIX[3] = {0, 2.0, 2.0};
-constexpr int MID_SD[3] = {0, 2, 1};  // 64-deep blocks per pipeline stage
-constexpr double MID_FINISH_US = 5.0;
+//   - a 64-wide depth block of a 64-token tile takes MID_T1 us when its
+//     workgroup has the CU to itself and MID_T2 us each when two share it;
+//     the tiles are dealt over the CUs, two at a time, MID_ROUND_US for each
+//     further round (400 tokens, 512 -> 8192: 24 us in two rounds);
+//   - a stage of a 128-token tile (256 deep with 128 rows, 128 deep with
+//     256: the same matrix-core work) takes 1.3 us with a third of the CUs at
+//     work and 1.75 us with all of them (the power limit), the tile's start and
+//     end MID_FIX us: 1024 tokens, 3072 -> 3072, 192 tiles of 12 stages
+//     25 us; 777 tokens, 3072 -> 9216, 252 tiles of 24 stages 45 us;
+//   - a tile may split its depth into ranges (one workgroup each, whole
+//     rounds of stages) when the tiles leave CUs idle; the ranges'
+//     accumulators meet in the launch, and S > 1 must model a tenth faster;
+//   - `side`: what forming the LoRA factors beside the product adds. The
+//     large tiles need a launch for t, or for u and for dA and dB (8 and 20
+//     us plus their streams at 6 TB/s); the others form them in their own
+//     launch: the factor slices' workgroups hold up tiles, and weight-gradient
+//     blocks beyond half a round of workgroups follow the tiles (4096 tokens,
+//     3072 -> 12288, rank 32: 100 us, where 1999 tokens, 2560 -> 4096 add 4).
+constexpr double LARGE_STEP_US = 1.75;
+// per variant MID_64, MID_128, MID_256: tile tokens and rows, a fixed cost
+// per round of tiles, 64-deep blocks per pipeline stage, stages a depth range
+// is a multiple of, and the most ranges
+constexpr int MID_T[4] = {0, 64, W8_TOKENS, W8_TOKENS}, MID_R[4] = {0, 64, 128, 256};
+constexpr double MID_T1 = 0.342, MID_T2 = 0.423;
+constexpr double W8_STAGE_US = 1.0, W8_STAGE_FULL_US = 0.75;  // W8_STAGE_US + the share of the CUs at work x the other
+constexpr double MID_FIX[4] = {0, 2.0, 7.0, 6.0};
+constexpr int MID_SD[4] = {0, 2, 4, 2};
+constexpr int MID_ROUND[4] = {0, MID_MST, 1, 1};
+constexpr int MID_MAXS[4] = {0, MID_MAX_SPLIT, W8_MAX_SPLIT, W8_MAX_SPLIT};
+constexpr double MID_FINISH_US = 4.5;  // depth ranges of a 64-token tile
+constexpr double W8_FINISH_US = 2.0;   // and of the others, with 0.5 a range and the partials at 8 TB/s
+constexpr double MID_ROUND_US = 6.0;   // a further round of 64-token tiles
 // lrq_debug_gemm_path: 0 planned, 1 large tiles, 2 + (variant - 1) a mid
-// variant, 4 + (variant - 1) a mid variant with at least two depth ranges
-// where the depth has them
+// variant (MID_64, MID_128), 4 + (variant - 1) one with at least two depth
+// ranges where the depth has them; 6 and 7 the same for MID_256
 int g_gemm_path = 0;
 
-double large_us(int64_t m, int64_t e, int64_t depth) {
+// microseconds that a product's bytes take beside a launch's fixed cost
+double stream_us(double bytes) { return bytes / 6.0e6; }
+
+double large_us(int64_t m, int64_t e, int64_t depth, int side) {
   const SplitPlan p = plan_split(m, e, depth);
   const int64_t cus = get_num_cus();
   const int64_t RA = p.r192 ? 192 : 256;
   const int64_t tiles = (m + RB - 1) / RB * ((e + RA - 1) / RA);
   const double f = p.r192 ? 0.8 : 1.0;
-  if (p.S <= 1) return (double)((tiles + cus - 1) / cus) * (double)((depth + 63) / 64) * LARGE_STEP_US * f + 3.0;
+  const double act = 2.0 * (double)m * (double)depth;
+  const double extra = side == SIDE_FWD ? 8.0 + stream_us(act)
+                       : side == SIDE_BWD ? 20.0 + stream_us(2.0 * act + 2.0 * (double)m * (double)e)
+                                          : 0.0;
+  if (p.S <= 1)
+    return (double)((tiles + cus - 1) / cus) * (double)((depth + 63) / 64) * LARGE_STEP_US * f + 3.0 + extra;
   const double part = 4.0 * (double)p.S * (double)m * (double)e;
-  return (double)p.spl * LARGE_STEP_US * f + 2.0 * part / 4.0e6 + 8.0;
+  return (double)p.spl * LARGE_STEP_US * f + 2.0 * part / 4.0e6 + 8.0 + extra;
 }
 
 // stages per range (whole rounds) for S ranges of a depth, and the ranges
 // that gives
 int mid_spl(int64_t depth, int v, int S) {
   const int64_t nst = ((depth + 63) / 64 + MID_SD[v] - 1) / MID_SD[v];
-  return (int)(((nst + S - 1) / S + MID_MST - 1) / MID_MST * MID_MST);
+  return (int)(((nst + S - 1) / S + MID_ROUND[v] - 1) / MID_ROUND[v] * MID_ROUND[v]);
 }
 int mid_ranges(int64_t depth, int v, int S) {
   const int64_t nst = ((depth + 63) / 64 + MID_SD[v] - 1) / MID_SD[v];
@@ -704,14 +728,27 @@ int mid_ranges(int64_t depth, int v, int S) {
   return (int)((nst + spl - 1) / spl);
 }
 
-double mid_us(int64_t m, int64_t e, int64_t depth, int v, int S = 1) {
+double mid_us(int64_t m, int64_t e, int64_t depth, int side, int v, int S = 1) {
   const int64_t T = MID_T[v], cus = get_num_cus();
-  const int64_t tiles = (m + T - 1) / T * ((e + 63) / 64) * S;
+  const int64_t tiles = (m + T - 1) / T * ((e + MID_R[v] - 1) / MID_R[v]) * S;
   const int64_t n = (tiles + cus - 1) / cus;
+  if (v != MID_64) {
+    const int64_t nst = ((depth + 63) / 64 + MID_SD[v] - 1) / MID_SD[v];
+    const double part = S > 1 ? W8_FINISH_US + 0.5 * S + 0.75 * stream_us(2.0 * 4.0 * (double)(tiles * T * MID_R[v])) : 0.0;
+    const double stage = W8_STAGE_US + W8_STAGE_FULL_US * std::min(1.0, (double)tiles / (double)cus);
+    double extra = 0.0;
+    if (side != SIDE_NONE)  // factor slices, two a workgroup, about 10 us a round with what they hold up
+      extra = 10.0 * (double)((m + 63) / 64 * ((depth + MID_FOLD_KT - 1) / MID_FOLD_KT)) / (2.0 * (double)cus);
+    if (side == SIDE_BWD) {
+      const LoraPlan pa = mid_tn_plan(m, e, depth, 32, W8_TN_LDS), pb = mid_tn_plan(m, depth, e, 32, W8_TN_LDS);
+      extra += 45.0 * std::max(0.0, (double)(pa.tiles * pa.splits + pb.tiles * pb.splits) / (2.0 * (double)cus) - 0.5);
+    }
+    return (double)n * ((double)(S > 1 ? mid_spl(depth, v, S) : nst) * stage + MID_FIX[v]) + part + extra;
+  }
   const int64_t nb = S > 1 ? std::min<int64_t>((int64_t)mid_spl(depth, v, S) * MID_SD[v], (depth + 63) / 64)
                            : (depth + 63) / 64;
-  return (double)nb * ((double)(n / 2) * MID_T2[v] + (double)(n % 2) * MID_T1[v]) +
-         MID_FIX[v] * (double)((n + 1) / 2) + (S > 1 ? MID_FINISH_US : 0.0);
+  return (double)nb * ((double)(n / 2) * MID_T2 + (double)(n % 2) * MID_T1) +
+         MID_FIX[v] + MID_ROUND_US * (double)((n + 1) / 2 - 1) + (S > 1 ? MID_FINISH_US : 0.0);
 }
 
 struct MidChoice {
@@ -721,13 +758,13 @@ struct MidChoice {
 
 // the best number of depth ranges for variant v (forced: at least two
 // where the depth has them)
-MidChoice mid_best_split(int64_t m, int64_t e, int64_t depth, int v, bool force_split) {
-  MidChoice best{v, 1, 0, mid_us(m, e, depth, v, 1)};
+MidChoice mid_best_split(int64_t m, int64_t e, int64_t depth, int side, int v, bool force_split) {
+  MidChoice best{v, 1, 0, mid_us(m, e, depth, side, v, 1)};
   MidChoice alt{v, 1, 0, 1e30};
-  for (int S = 2; S <= MID_MAX_SPLIT; ++S) {
+  for (int S = 2; S <= MID_MAXS[v]; ++S) {
     const int R = mid_ranges(depth, v, S);
     if (R < 2 || R != S) continue;  // (S that rounding turns into fewer ranges are covered by those)
-    const double t = mid_us(m, e, depth, v, S);
+    const double t = mid_us(m, e, depth, side, v, S);
     if (t < alt.us) alt = MidChoice{v, S, mid_spl(depth, v, S), t};
   }
   if (alt.S > 1 && (force_split || alt.us < 0.9 * best.us)) return alt;
@@ -735,27 +772,30 @@ MidChoice mid_best_split(int64_t m, int64_t e, int64_t depth, int v, bool force_
 }
 
 // the mid variant and its depth ranges a shape takes (v = MID_NONE: the
-// large tiles)
-MidChoice mid_choice(int64_t m, int64_t e, int64_t depth) {
+// large tiles). Decided on whole 64-token groups, so that a workspace
+// reserved for the largest of a group's token counts serves them all.
+MidChoice mid_choice(int64_t m, int64_t e, int64_t depth, int side) {
   const MidChoice none{MID_NONE, 1, 0, 0.0};
   if (m <= 0 || e <= 0 || g_gemm_path == 1) return none;
-  if (g_gemm_path >= 2) return mid_best_split(m, e, depth, (g_gemm_path - 2) % 2 + 1, g_gemm_path >= 4);
+  m = (m + 63) / 64 * 64;
+  if (g_gemm_path >= 6) return mid_best_split(m, e, depth, side, MID_256, g_gemm_path == 7);
+  if (g_gemm_path >= 2) return mid_best_split(m, e, depth, side, (g_gemm_path - 2) % 2 + 1, g_gemm_path >= 4);
   MidChoice pick = none;
-  pick.us = large_us(m, e, depth);
-  for (int v : {MID_64, MID_128}) {
-    const MidChoice c = mid_best_split(m, e, depth, v, false);
+  pick.us = large_us(m, e, depth, side);
+  for (int v : {MID_64, MID_128, MID_256}) {
+    const MidChoice c = mid_best_split(m, e, depth, side, v, false);
     if (c.us < pick.us) pick = c;
   }
   return pick;
 }
 
 // MID_NONE (the large tiles) or the mid variant a shape takes
-int mid_plan(int64_t m, int64_t e, int64_t depth) { return mid_choice(m, e, depth).v; }
+int mid_plan(int64_t m, int64_t e, int64_t depth, int side) { return mid_choice(m, e, depth, side).v; }
 
 template <bool BWD>
 hipError_t dispatch(hipStream_t st, int fmt, const GemmArgs& a) {
   if (a.m == 0 || a.e == 0) return hipSuccess;
-  const MidChoice mc = mid_choice(a.m, a.e, a.l);
+  const MidChoice mc = mid_choice(a.m, a.e, a.l, a.fold ? (BWD ? SIDE_BWD : SIDE_FWD) : SIDE_NONE);
   if (mc.v != MID_NONE) {
     if (mc.S <= 1) return launch_mid(st, fmt, BWD, a, mc.v);
     if (!a.part || !a.mcnt) return hipErrorInvalidValue;
@@ -787,19 +827,22 @@ void set_num_cus(int n) { g_num_cus_ = n > 0 ? n : 256; }
 int get_num_cus() { return g_num_cus_; }
 
 hipError_t launch_fwd(hipStream_t st, int fmt, const GemmArgs& a) { return dispatch<false>(st, fmt, a); }
-MidSplit mid_split_plan(int64_t m, int64_t e, int64_t depth) {
-  const MidChoice mc = mid_choice(m, e, depth);
+MidSplit mid_split_plan(int64_t m, int64_t e, int64_t depth, int side) {
+  const MidChoice mc = mid_choice(m, e, depth, side);
   if (mc.v == MID_NONE || mc.S <= 1) return MidSplit{1, 0, 0, 0};
-  const int64_t T = MID_T[mc.v], tiles = (m + T - 1) / T * ((e + 63) / 64);
-  return MidSplit{mc.S, mc.spl, tiles, (int64_t)mc.S * tiles * T * 64};
+  const int64_t T = MID_T[mc.v], R = MID_R[mc.v], tiles = (m + T - 1) / T * ((e + R - 1) / R);
+  return MidSplit{mc.S, mc.spl, tiles, (int64_t)mc.S * tiles * T * R};
 }
 
 int64_t gemm_split_floats(int64_t m, int64_t e, int64_t depth) {
   if (m <= 0 || e <= 0) return 0;
-  if (mid_plan(m, e, depth)) return mid_split_plan(m, e, depth).floats;  // the mid tiles' depth ranges
+  if (mid_plan(m, e, depth, SIDE_NONE)) return mid_split_plan(m, e, depth, SIDE_NONE).floats;  // the mid tiles' depth ranges
   const SplitPlan p = plan_split(m, e, depth);
   return p.S > 1 ? (int64_t)p.S * m * e : 0;
 }
 hipError_t launch_bwd(hipStream_t st, int fmt, const GemmArgs& a) { return dispatch<true>(st, fmt, a); }
-int gemm_mid_tokens(int64_t m, int64_t e, int64_t depth) { return MID_T[mid_plan(m, e, depth)]; }
+int mid_tn_lds(int64_t m, int64_t e, int64_t depth) {
+  return mid_plan(m, e, depth, SIDE_BWD) == MID_64 ? MID_TN_LDS : W8_TN_LDS;
+}
+int gemm_mid_tokens(int64_t m, int64_t e, int64_t depth, int side) { return MID_T[mid_plan(m, e, depth, side)]; }
 void set_gemm_path(int path) { g_gemm_path = path; }

@@ -10,8 +10,10 @@
 // kernels, as for the large tiles.)
 //
 // "Rows" are the output columns (n forward, k backward), "depth" the
-// reduction index. A tile is 64 rows x T tokens (T = 16 TT: 64 or 128) over
-// the whole depth, one workgroup of four wavefronts, two workgroups per CU:
+// reduction index. A tile is 64 rows x 64 tokens (T = 16 TT) over the whole
+// depth, one workgroup of four wavefronts, two workgroups per CU (its
+// 128-token tiles gave way to lrq_gemm_w8.hip's: 1024 tokens, 3072 -> 3072,
+// rank 16, forward 39 -> 29 us):
 //   - wavefront w owns rows 16w .. 16w+15 of the tile for all T tokens, so
 //     each weight element is dequantized once per tile and each dequantized
 //     fragment feeds TT matrix-core steps (v_mfma_f32_16x16x32_bf16, weight
@@ -58,24 +60,10 @@
 // outputs past M or E are not stored.
 
 #include "lrq_common.h"
+#include "lrq_fold.h"
 #include "lrq_kernels.h"
-#include "lrq_tn.h"
 
 namespace {
-
-// device-scope accesses of the fold's cross-workgroup data (written through
-// and read past the per-XCD L2s), as in lrq_skinny.hip
-constexpr int MXSCOPE = __HIP_MEMORY_SCOPE_AGENT;
-LRQ_DEV uint32_t madd_dev(uint32_t* c) { return __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, MXSCOPE); }
-LRQ_DEV void mzero_dev(uint32_t* c) { __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, MXSCOPE); }
-LRQ_DEV uint32_t mload_dev(const uint32_t* c) { return __hip_atomic_load(c, __ATOMIC_RELAXED, MXSCOPE); }
-LRQ_DEV u32x4 mbload16_dev(rsrc_t r, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 16); }
-LRQ_DEV void mstore16_dev(rsrc_t r, uint32_t off, const u32x4& v) { __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 16); }
-LRQ_DEV void mstore8_dev(rsrc_t r, uint32_t off, const u32x2& v) { __builtin_amdgcn_raw_buffer_store_b64(v, r, off, 0, 16); }
-LRQ_DEV uint32_t mstamp(uint32_t ep) { return ep + 1 == 0 ? 1u : ep + 1; }
-constexpr uint32_t MID_MAX_POLLS = 1u << 22;  // about 0.2 s of s_sleep 2
-// the fold's counters: per 64-token group the slices' arrivals at [0, G)
-// and the ready flags at [G, 2 G)
 
 constexpr int MD = 64;    // depth per step (one 64 x 64 weight block)
 constexpr int MR = 64;    // rows per tile: four wavefronts of 16
@@ -84,183 +72,6 @@ constexpr int MST = MID_MST;  // pipeline stages
 // LDS chunk swizzle: rows r and r + 1 share a chunk order, so the 16 rows a
 // quarter-wavefront reads at one logical chunk cover all 64 banks
 LRQ_DEV int mswz(int r) { return (r >> 1) & 7; }
-
-// FOLD: workgroup fw of the factor workgroups: 64-token group fw / fold_slices,
-// depth slice fw % fold_slices, RT rank tiles of 16 (rp = 16 RT). Wavefront
-// w takes tokens 16 w .. + 16 of the group; each of its lanes loads the
-// group's token row 16 w + (l & 15) at depths 32 ss + 8 (l >> 4) .. + 8 of
-// the slice (every load of the slice at once) and the factor fragments of
-// the same depths for ranks 16 rt + (l & 15): forward A's rows staged
-// transposed in LDS (rank tile rt's aT [16][FKT + 8] in lds[rt]), backward
-// B's rows read directly. `want` is the launch's stamp.
-template <bool BWD, int RT>
-LRQ_DEV void mid_fold_slice(const GemmArgs& a, int fw, uint16_t* lds0, uint16_t* lds1, uint32_t want) {
-  constexpr int FKT = MID_FOLD_KT, NSS = FKT / 32, AST = FKT + 8, RP = 16 * RT;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c16 = lane & 15, kq = lane >> 4;
-  const int fs = a.fold_slices, g = fw / fs, sl = fw % fs;
-  const int64_t M = a.m, D = a.l, Mp = (M + 63) / 64 * 64;
-  const int r = a.r;
-  const int64_t k0 = (int64_t)sl * FKT, k1 = k0 + FKT < D ? k0 + FKT : D;
-  const int64_t tok = (int64_t)g * 64 + 16 * w + c16;
-  const rsrc_t rx = make_rsrc(a.act, clamp_bytes(M * D * 2));
-  const rsrc_t rf = make_rsrc(a.lact, clamp_bytes(D * r * 2));
-  uint16_t* const lds[2] = {lds0, lds1};
-  u32x4 xf[NSS], bf[RT][NSS];
-#pragma unroll
-  for (int ss = 0; ss < NSS; ++ss) {
-    const int64_t k = k0 + 32 * ss + 8 * kq;
-    xf[ss] = bload16(rx, opaque_u32(tok < M && k < k1 ? (uint32_t)((tok * D + k) * 2) : LRQ_OOB));
-    if (BWD) {
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        const int j = 16 * rt + c16;
-        bf[rt][ss] = bload16(rf, opaque_u32(j < r && k < k1 ? (uint32_t)(((int64_t)j * D + k) * 2) : LRQ_OOB));
-      }
-    }
-  }
-  if (!BWD) {
-    // A [D][r] rows of the slice, 8 ranks per 16-byte run: pair i = tid +
-    // 256 q is depth i / JB, ranks 8 (i % JB) ..; zeros past the rank or depth
-    constexpr int JB = RP / 8, AQ = JB * FKT / 256;
-    u32x4 av[AQ];
-#pragma unroll
-    for (int qq = 0; qq < AQ; ++qq) {
-      const int i = tid + 256 * qq, dd = i / JB, j0 = 8 * (i % JB);
-      av[qq] = bload16(rf, opaque_u32(k0 + dd < k1 && j0 < r ? (uint32_t)(((k0 + dd) * r + j0) * 2) : LRQ_OOB));
-    }
-#pragma unroll
-    for (int qq = 0; qq < AQ; ++qq) {
-      const int i = tid + 256 * qq, dd = i / JB, j0 = 8 * (i % JB);
-      uint16_t* t = lds[j0 >> 4];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) t[((j0 & 15) + e) * AST + dd] = (uint16_t)(av[qq][e >> 1] >> (16 * (e & 1)));
-    }
-    __syncthreads();
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int ss = 0; ss < NSS; ++ss)
-        bf[rt][ss] = *reinterpret_cast<const u32x4*>(lds[rt] + c16 * AST + 32 * ss + 8 * kq);
-  }
-  // C element v of lane (c16, kq) in rank tile rt: rank 16 rt + 4 kq + v,
-  // token 16 w + c16
-  f32x4 acc[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    acc[rt] = acc_zero4();
-#pragma unroll
-    for (int ss = 0; ss < NSS; ++ss) acc[rt] = mfma16(as_bf16x8(bf[rt][ss]), as_bf16x8(xf[ss]), acc[rt]);
-  }
-  const rsrc_t rp = make_rsrc(a.fpart, clamp_bytes((int64_t)fs * Mp * RP * 4));
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-    mstore16_dev(rp, opaque_u32((uint32_t)((((int64_t)sl * Mp + tok) * RP + 16 * rt + 4 * kq) * 4)),
-                 __builtin_bit_cast(u32x4, acc[rt]));
-  // counted once the partial is acknowledged; the last slice of the group
-  // sums the slices in order, stores the factor and publishes the flag
-  __builtin_amdgcn_s_waitcnt(0);
-  __shared__ int last;
-  __syncthreads();
-  const int64_t G = (M + 63) / 64;
-  if (tid == 0) {
-    last = madd_dev(a.fcnt + g) + 1 == (uint32_t)fs;
-    if (last) mzero_dev(a.fcnt + g);
-  }
-  __syncthreads();
-  if (!last) return;
-  // thread: token g 64 + tid / 4, ranks 16 rt + 4 (tid % 4) ..
-  const int64_t tk = (int64_t)g * 64 + (tid >> 2);
-  const rsrc_t ro = make_rsrc(a.fout, clamp_bytes(M * a.fout_ld * 2));
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int rq = 16 * rt + 4 * (tid & 3);
-    f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s0 = 0; s0 < fs; s0 += 8) {
-      u32x4 pv[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        pv[u] = mbload16_dev(rp, opaque_u32(s0 + u < fs ? (uint32_t)((((int64_t)(s0 + u) * Mp + tk) * RP + rq) * 4) : LRQ_OOB));
-#pragma unroll
-      for (int u = 0; u < 8; ++u) sum += __builtin_bit_cast(f32x4, pv[u]);
-    }
-    if (a.fout && tk < M && rq < a.fout_ld) {
-      const u32x2 o = {pack_bf16x2(a.fscale * sum[0], a.fscale * sum[1]), pack_bf16x2(a.fscale * sum[2], a.fscale * sum[3])};
-      mstore8_dev(ro, opaque_u32((uint32_t)((tk * a.fout_ld + rq) * 2)), o);
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (tid == 0) __hip_atomic_store(a.fcnt + G + g, want, __ATOMIC_RELAXED, MXSCOPE);
-}
-
-// FOLD: a reader of the ready flags is done with them (a tile after its
-// LoRA step, a dA block after its wait). The last of the launch's `readers`
-// clears the flags and advances the epoch. Every thread of the workgroup
-// calls it.
-LRQ_DEV void mid_flags_done(const GemmArgs& a, int readers) {
-  __shared__ int fin;
-  __syncthreads();
-  if (threadIdx.x == 0) fin = madd_dev(a.fcnt + SK_DCNT) + 1 == (uint32_t)readers;
-  __syncthreads();
-  if (fin) {
-    const int64_t G = (a.m + 63) / 64;
-    for (int64_t i = threadIdx.x; i < G; i += 256) mzero_dev(a.fcnt + G + i);
-    if (threadIdx.x == 0) {
-      mzero_dev(a.fcnt + SK_DCNT);
-      madd_dev(a.fcnt + SK_EPOCH);
-    }
-  }
-}
-
-// FOLD backward: weight-gradient block tb of the launch's tn jobs (after the
-// tiles). A dA block first waits (bounded, as the tiles do) for the ready
-// flags of the 64-token groups of its token slice, then reads u at device
-// scope; a wait that runs out flags the failure and makes its sums NaN.
-// The factor slice goes to sq, the combine buffer to sr (16 KiB each).
-LRQ_DEV void mid_tn(const GemmArgs& a, int tb, uint32_t want, int readers, uint16_t* sq, uint16_t* sr) {
-  const bool second = tb >= a.tj[0].blocks;
-  const int ji = second ? 1 : 0;
-  const TnArgs& j = a.tj[ji];
-  const int bid = tb - (second ? a.tj[0].blocks : 0);
-  float* const red = reinterpret_cast<float*>(sr);
-  if (ji != a.tn_da) {
-    if (a.rp == 32)
-      tn_block<2, MID_TN_LDS, MID_TN_LDS, false>(j, bid, sq, red, false);
-    else
-      tn_block<1, MID_TN_LDS, MID_TN_LDS, false>(j, bid, sq, red, false);
-    return;
-  }
-  __shared__ int bad;
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    const int64_t G = (a.m + 63) / 64;
-    const int64_t m_lo = (int64_t)(bid / j.tiles) * j.m_per;
-    const int64_t m_hi = min(j.M, m_lo + j.m_per);
-    const int64_t gi = m_lo / 64 + lane;
-    const bool mine = gi < (m_hi + 63) / 64 && gi < G;
-    uint32_t polls = 0;
-    const uint32_t cap = a.fold < 0 ? 16u : MID_MAX_POLLS;  // the test hook: 16 polls
-    bool ok = !mine || mload_dev(a.fcnt + G + gi) == want;
-    while (!__all(ok) && polls < cap) {
-      __builtin_amdgcn_s_sleep(2);
-      ++polls;
-      ok = !mine || mload_dev(a.fcnt + G + gi) == want;
-    }
-    if (lane == 0) {
-      bad = __all(ok) ? 0 : 1;
-      if (!__all(ok)) __hip_atomic_store(a.fcnt + SK_FAIL, 1u, __ATOMIC_RELAXED, MXSCOPE);
-    }
-  }
-  __syncthreads();
-  const bool poison = bad != 0;
-  mid_flags_done(a, readers);
-  if (a.rp == 32)
-    tn_block<2, MID_TN_LDS, MID_TN_LDS, true>(j, bid, sq, red, poison);
-  else
-    tn_block<1, MID_TN_LDS, MID_TN_LDS, true>(j, bid, sq, red, poison);
-}
 
 template <bool BWD, int FMT, int TT, int SD, bool FOLD>
 __global__ void __launch_bounds__(256, 2) k_mid(GemmArgs a, int tiles_m, int tiles_e, int group_m) {
@@ -305,7 +116,7 @@ __global__ void __launch_bounds__(256, 2) k_mid(GemmArgs a, int tiles_m, int til
       if ((int)blockIdx.x >= a.fold_wgs + nunits) {
         static_assert(MID_TN_LDS <= XB * 2, "a weight-gradient block's LDS fits one stage buffer");
         const int nda = a.tn_da >= 0 ? a.tj[a.tn_da].blocks : 0;
-        mid_tn(a, (int)blockIdx.x - a.fold_wgs - nunits, want, ntiles + nda, sx0, sx1);
+        mid_tn<MID_TN_LDS>(a, (int)blockIdx.x - a.fold_wgs - nunits, want, ntiles + nda, sx0, sx1);
         return;
       }
     }
@@ -671,12 +482,12 @@ __global__ void __launch_bounds__(256, 2) k_mid(GemmArgs a, int tiles_m, int til
     const uint32_t off = nok ? (uint32_t)(((16 * j + l16) * E + n) * 2) : LRQ_OOB;
     __builtin_amdgcn_raw_buffer_store_b64(o, ry, opaque_u32(off), 0, 2);  // non-temporal, as the large tiles' output
   }
-  if (FOLD) mid_flags_done(a, ntiles + ((BWD && a.tn_da >= 0) ? a.tj[a.tn_da].blocks : 0));
+  if (FOLD) mid_flags_done<256>(a, ntiles + ((BWD && a.tn_da >= 0) ? a.tj[a.tn_da].blocks : 0));
 }
 
 template <bool BWD, int FMT>
-hipError_t run_mid(hipStream_t st, const GemmArgs& a, int variant) {
-  const int T = variant == MID_64 ? 64 : 128;
+hipError_t run_mid(hipStream_t st, const GemmArgs& a) {
+  constexpr int T = 64;
   const int tiles_m = (int)((a.m + T - 1) / T);
   const int tiles_e = (int)((a.e + MR - 1) / MR);
   const int group_m = tiles_m < 8 ? tiles_m : 8;
@@ -687,12 +498,7 @@ hipError_t run_mid(hipStream_t st, const GemmArgs& a, int variant) {
   // with depth ranges; with the fold, its workgroups first
   if (a.fold) {
     const unsigned grid = (unsigned)(ntiles * S + a.fold_wgs + (BWD ? a.tn_blocks : 0));
-    if (variant == MID_128)
-      hipLaunchKernelGGL((k_mid<BWD, FMT, 8, 1, true>), dim3(grid), dim3(256), 0, st, a, tiles_m, tiles_e, group_m);
-    else
-      hipLaunchKernelGGL((k_mid<BWD, FMT, 4, 2, true>), dim3(grid), dim3(256), 0, st, a, tiles_m, tiles_e, group_m);
-  } else if (variant == MID_128) {
-    hipLaunchKernelGGL((k_mid<BWD, FMT, 8, 1, false>), dim3(ntiles * S), dim3(256), 0, st, a, tiles_m, tiles_e, group_m);
+    hipLaunchKernelGGL((k_mid<BWD, FMT, 4, 2, true>), dim3(grid), dim3(256), 0, st, a, tiles_m, tiles_e, group_m);
   } else {
     hipLaunchKernelGGL((k_mid<BWD, FMT, 4, 2, false>), dim3(ntiles * S), dim3(256), 0, st, a, tiles_m, tiles_e, group_m);
   }
@@ -703,18 +509,21 @@ hipError_t run_mid(hipStream_t st, const GemmArgs& a, int variant) {
 
 hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int variant) {
   if (a.m <= 0 || a.e <= 0) return hipSuccess;
-  if (variant != MID_64 && variant != MID_128) return hipErrorInvalidValue;
+  if (variant != MID_64 && variant != MID_128 && variant != MID_256) return hipErrorInvalidValue;
   if (a.rp > 64 || a.rp % 16 != 0) return hipErrorInvalidValue;
-  // depth ranges: at most MID_MAX_SPLIT, each whole rounds of stages, the
-  // last one non-empty; partials for every unit and a counter per tile
-  const int T = variant == MID_64 ? 64 : 128, SDv = variant == MID_64 ? 2 : 1;
-  const int64_t ntiles = (a.m + T - 1) / T * ((a.e + MR - 1) / MR);
+  // depth ranges: at most MID_MAX_SPLIT (W8_MAX_SPLIT), each whole rounds of
+  // stages (whole stages), the last one non-empty; partials for every unit
+  // and a counter per tile
+  const bool w8 = variant != MID_64;
+  const int T = w8 ? W8_TOKENS : 64, TR = variant == MID_64 ? MR : (variant == MID_128 ? 128 : 256);
+  const int64_t ntiles = (a.m + T - 1) / T * ((a.e + TR - 1) / TR);
   const int S = a.msplit > 1 ? a.msplit : 1;
   if (S > 1) {
-    const int64_t nst = ((a.l + 63) / 64 + SDv - 1) / SDv;
-    if (S > MID_MAX_SPLIT || a.mspl <= 0 || a.mspl % MST != 0 || (int64_t)(S - 1) * a.mspl >= nst ||
+    const int64_t stage = variant == MID_128 ? 256 : 128;
+    const int64_t nst = (a.l + stage - 1) / stage;
+    if (S > (w8 ? W8_MAX_SPLIT : MID_MAX_SPLIT) || a.mspl <= 0 || a.mspl % (w8 ? 1 : MST) != 0 || (int64_t)(S - 1) * a.mspl >= nst ||
         (int64_t)S * a.mspl < nst || !a.part || !a.mcnt ||
-        (int64_t)S * ntiles * T * 64 * 4 >= ((int64_t)1 << 32))
+        (int64_t)S * ntiles * T * TR * 4 >= ((int64_t)1 << 32))
       return hipErrorInvalidValue;
   }
   // the fold: ranks 8 to 32 (multiples of 8, padded to 16 or 32), both raw factors, its output, partials and
@@ -730,7 +539,7 @@ hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int 
         (int64_t)a.fold_slices * G * 64 * a.rp * 4 >= ((int64_t)1 << 32))
       return hipErrorInvalidValue;
     // the weight gradients' jobs after the tiles (backward): each a whole
-    // plan of token slices that fit MID_TN_LDS, over all the launch's
+    // plan of token slices that fit the variant's LDS, over all the launch's
     // tokens, with its counters past the fold's and apart from the other's
     if (a.tn_blocks != 0) {
       if (!bwd || a.tn_blocks < 0 || a.tj[0].blocks + a.tj[1].blocks != a.tn_blocks || a.tn_da < -1 ||
@@ -742,7 +551,7 @@ hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int 
         const TnArgs& j = a.tj[i];
         if (j.blocks == 0) continue;
         if (j.C <= 0 || j.tiles != (j.C + 127) / 128 || j.splits < 1 || j.blocks != j.tiles * j.splits ||
-            j.m_per <= 0 || j.m_per % 128 != 0 || a.rp * (j.m_per + 8) * 2 > MID_TN_LDS || j.M != a.m ||
+            j.m_per <= 0 || j.m_per % 128 != 0 || a.rp * (j.m_per + 8) * 2 > (w8 ? W8_TN_LDS : MID_TN_LDS) || j.M != a.m ||
             (int64_t)j.splits * j.m_per < j.M || (int64_t)(j.splits - 1) * j.m_per >= j.M || !j.p || !j.q ||
             !j.out || j.R < 1 || j.R > a.rp || j.ldq < j.R || (j.splits > 1 && !j.partial) || !j.cnt ||
             j.cnt < lo || j.cnt + TN_WAVES * j.tiles > a.fcnt + SK_MAX_NB ||
@@ -762,9 +571,10 @@ hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int 
   // run of the weight's block row
   if ((int64_t)128 * a.l * 2 >= ((int64_t)1 << 31) || (int64_t)128 * a.e * 2 >= ((int64_t)1 << 31))
     return hipErrorInvalidValue;
+  if (w8) return launch_w8(st, fmt, bwd, a, TR);
   if (fmt == LRQ_FMT_INT4)
-    return bwd ? run_mid<true, LRQ_FMT_INT4>(st, a, variant) : run_mid<false, LRQ_FMT_INT4>(st, a, variant);
+    return bwd ? run_mid<true, LRQ_FMT_INT4>(st, a) : run_mid<false, LRQ_FMT_INT4>(st, a);
   if (fmt == LRQ_FMT_INT8)
-    return bwd ? run_mid<true, LRQ_FMT_INT8>(st, a, variant) : run_mid<false, LRQ_FMT_INT8>(st, a, variant);
-  return bwd ? run_mid<true, LRQ_FMT_FP8>(st, a, variant) : run_mid<false, LRQ_FMT_FP8>(st, a, variant);
+    return bwd ? run_mid<true, LRQ_FMT_INT8>(st, a) : run_mid<false, LRQ_FMT_INT8>(st, a);
+  return bwd ? run_mid<true, LRQ_FMT_FP8>(st, a) : run_mid<false, LRQ_FMT_FP8>(st, a);
 }

@@ -108,15 +108,25 @@ hipError_t launch_fwd(hipStream_t st, int fmt, const GemmArgs& a);
 hipError_t launch_bwd(hipStream_t st, int fmt, const GemmArgs& a);
 int64_t gemm_split_floats(int64_t m, int64_t e, int64_t depth);
 int get_num_cus();
-// lrq_gemm_mid.hip: the same products on 64-row tiles of 64 or 128 tokens
-// over the whole depth or a few depth ranges finished in the launch, 16
-// rows per wavefront (MID_64, MID_128); lrq_gemm.hip's launchers take one
-// when it is modelled faster (gemm_mid_tokens: its tile's tokens, or 0).
-// With depth ranges the caller provides a.part (gemm_split_floats) and
-// a.mcnt (mid_split_plan(...).tiles counters).
-enum { MID_NONE = 0, MID_64 = 1, MID_128 = 2 };
-constexpr int MID_MAX_SPLIT = 4;
-constexpr int MID_MST = 4;  // the mid kernel's pipeline stages (a range is whole rounds of them)
+// lrq_gemm_mid.hip (64-row x 64-token tiles, MID_64) and lrq_gemm_w8.hip
+// (128-token tiles of 128 or 256 rows, MID_128 and MID_256): the same
+// products over the whole depth or a few depth ranges finished in the
+// launch; lrq_gemm.hip's launchers take one when it is modelled faster
+// (gemm_mid_tokens: its tile's tokens, or 0). `side` says which LoRA factors
+// the launch would form too (SIDE_*: t; u, dA and dB; none, or they have
+// launches of their own): a call plans, reserves and launches with the same.
+// With depth ranges the caller provides a.part (gemm_split_floats without,
+// mid_split_plan(...).floats with such factors) and a.mcnt
+// (mid_split_plan(...).tiles counters).
+enum { SIDE_NONE = 0, SIDE_FWD = 1, SIDE_BWD = 2 };
+enum { MID_NONE = 0, MID_64 = 1, MID_128 = 2, MID_256 = 3 };
+constexpr int MID_MAX_SPLIT = 4;  // depth ranges of a MID_64 tile
+constexpr int MID_MST = 4;  // MID_64: the kernel's pipeline stages (a range is whole rounds of them)
+// lrq_gemm_w8.hip: tiles of 128 tokens x 128 (MID_128) or 256 rows (MID_256),
+// one workgroup of eight wavefronts per CU, stages of 256 or 128 depth
+constexpr int W8_TOKENS = 128;
+constexpr int W8_MAX_SPLIT = 8;  // depth ranges of a tile
+hipError_t launch_w8(hipStream_t st, int fmt, bool bwd, const struct GemmArgs& a, int rows);
 // The mid-size tiles' depth ranges for a product (m tokens, e outputs,
 // `depth`): S = 1 (whole depth) when the large tiles or one range per tile
 // are modelled faster; tiles and the partial floats the ranges need.
@@ -124,14 +134,16 @@ struct MidSplit {
   int S, spl;
   int64_t tiles, floats;
 };
-MidSplit mid_split_plan(int64_t m, int64_t e, int64_t depth);
+MidSplit mid_split_plan(int64_t m, int64_t e, int64_t depth, int side);
 hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int variant);
-int gemm_mid_tokens(int64_t m, int64_t e, int64_t depth);
+int gemm_mid_tokens(int64_t m, int64_t e, int64_t depth, int side);
 // depth per slice of the folded factor's workgroups (GemmArgs.fold)
 constexpr int MID_FOLD_KT = 384;
 // the token slices of a weight-gradient job run inside the mid-size
 // backward: the factor slice takes at most 16 KiB of LDS (ranks padded to 16 or 32)
 constexpr int MID_TN_LDS = 16384;
+constexpr int W8_TN_LDS = 36864;  // in lrq_gemm_w8.hip
+int mid_tn_lds(int64_t m, int64_t e, int64_t depth);  // of the variant an input gradient takes
 // tuning and test hook (lrq_debug_gemm_path): 0 planned, 1 large tiles,
 // 2 MID_64, 3 MID_128
 void set_gemm_path(int path);
@@ -198,9 +210,10 @@ struct LoraPlan {
 };
 LoraPlan lora_plan_nt(int64_t M, int64_t C, int rp);
 LoraPlan lora_plan_tn(int64_t M, int64_t C, int rp, int64_t other_c = 0);
-// tn slices that fit the mid-size backward's LDS (MID_TN_LDS for the factor
-// slice): as few token slices as that allows
-LoraPlan mid_tn_plan(int64_t M, int64_t C, int rp);
+// tn slices that fit the mid-size backward's LDS (`lds` bytes for the factor
+// slice, mid_tn_lds): as few token slices as that allows, but in lrq_gemm_w8.hip
+// as many as keep this job's and the other's (other_c columns) within TN_BLOCKS
+LoraPlan mid_tn_plan(int64_t M, int64_t C, int64_t other_c, int rp, int lds);
 // out = bf16(s * sum over slices of p[m, c] * q(j, c)) as [M, rp] (columns
 // >= r zero) and/or [M, r], with q(j, c) = q[j * ldq + c] when qrow (B [r, n]),
 // else q[c * ldq + j] (A [k, r]); entries j >= R read as zero. One launch:

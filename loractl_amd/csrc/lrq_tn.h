@@ -64,7 +64,7 @@ LRQ_DEV void tn_block(const TnArgs& a, int bid, uint16_t* sQ, float* red, bool p
   constexpr int NH = 128 / RCOLS;
   constexpr int CPW = RCOLS / TW;  // columns a wavefront sums per round
   static_assert(QBYTES >= RP * (128 + 8) * 2, "the factor slice holds at least 128 tokens");
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x % TNT, lane = tid & 63;  // one of the halves of a 512-thread workgroup
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t c0 = (int64_t)(bid % a.tiles) * 128;
   const int split = bid / a.tiles;

@@ -371,16 +371,17 @@ def debug_force_wait_timeout(on: bool):
     L.load().lrq_debug_force_wait_timeout(int(on))
 
 
-GEMM_PATHS = {"planned": 0, "large": 1, "mid64": 2, "mid128": 3, "mid64s": 4, "mid128s": 5}
+GEMM_PATHS = {"planned": 0, "large": 1, "mid64": 2, "mid128": 3, "mid64s": 4, "mid128s": 5, "mid256": 6, "mid256s": 7}
 
 
 def debug_gemm_path(path: str):
     """Tuning and test hook: force the kernel the fused products of m > 16
     tokens take in this process ("planned", "large": the 256-token tiles,
-    split in depth when too few, "mid64" / "mid128": 64-row tiles of 64 or
-    128 tokens, with depth ranges as planned, "mid64s" / "mid128s": the same
-    with at least two depth ranges where the depth allows). Every path
-    computes the same products."""
+    split in depth when too few, "mid64" / "mid128" / "mid256": tiles of 64
+    rows and tokens, 128 rows and tokens, or 256 rows and 128 tokens, with
+    depth ranges as planned, "mid64s" / "mid128s" / "mid256s": the same with
+    at least two depth ranges where the depth allows). Every path computes the
+    same products."""
     L.load().lrq_debug_gemm_path(GEMM_PATHS[path])
 
 
