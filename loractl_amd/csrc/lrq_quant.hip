@@ -3,8 +3,8 @@
 // dequantize kernels that expose the f32 values (src/quant.rs:232,
 // src/fp8.rs:306-318) and the bf16 matrix-core operands.
 //
-// All of these are HBM-bound byte/integer work: one thread per 8-value run,
-// 16-byte stores where the layout allows it, no LDS.
+// All of these are HBM-bound byte/integer work: 16-byte loads and stores, one
+// thread per run of values; the blocked layout's transpose goes through LDS.
 #include "lrq_common.h"
 #include "lrq_kernels.h"
 
@@ -129,39 +129,115 @@ __device__ __forceinline__ uint32_t fp8_encode_rne(float x) {
   return sign | code;
 }
 
-// Per-row (or whole-tensor) amax -> scale. One block per row for per-channel;
-// for a scalar scale a first pass writes per-row amax and a second block folds.
-__global__ void __launch_bounds__(256) k_rowabsmax(const float* __restrict__ w, int64_t k,
-                                                   float* __restrict__ out) {
-  const int64_t row = blockIdx.x;
-  const float* src = w + row * k;
-  float m = 0.0f;
-  for (int64_t i = threadIdx.x; i < k; i += blockDim.x) m = fmaxf(m, fabsf(src[i]));
+// The largest |v| over a 256-thread workgroup, in every thread (NaN is passed
+// over, as fmaxf does).
+LRQ_DEV float wg_max(float m) {
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
   __shared__ float red[4];
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
-  if (threadIdx.x == 0) out[row] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+LRQ_DEV float fp8_scale(float amax) {
+  const float s = amax / 448.0f;
+  return s < 1e-12f ? 1e-12f : s;
+}
+
+// Four f32 over their scale -> four e4m3fn bytes. The quotient is RN(v / s)
+// without a division (as in k_quantize: y = RN(1/s), q0 = RN(v y), exact
+// remainder, one fma; s >= 1e-12 and |v/s| <= 448, so no remainder that
+// matters underflows; an infinite scale divides), and |v/s| < 464 always, so
+// the hardware's round-to-nearest-even conversion never overflows. A NaN
+// quotient keeps its sign bit and encodes as 0x7f, like fp8_encode_rne.
+LRQ_DEV uint32_t fp8x4_encode(const f32x4& v, float s, float y, bool fast) {
+  float q[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (fast) {
+      const float q0 = v[j] * y;
+      // (the sign of a zero or a NaN would be lost on the way)
+      q[j] = __builtin_copysignf(__builtin_fmaf(__builtin_fmaf(-q0, s, v[j]), y, q0), v[j]);
+    } else {
+      q[j] = v[j] / s;
+    }
+  }
+  uint32_t w = 0;
+  if (fast) {
+    int r = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
+    r = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], r, true);
+    w = (uint32_t)r;
+    if (q[0] + q[1] + q[2] + q[3] == q[0] + q[1] + q[2] + q[3]) return w;  // no NaN (finite: |q| <= 448)
+    w = 0;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) w |= fp8_encode_rne(q[j]) << (8 * j);
+  return w;
+}
+
+// Per-row amax (the first pass of a scalar scale, and of rows longer than
+// k_fp8_rows holds). One workgroup per row, 16-byte loads.
+__global__ void __launch_bounds__(256) k_rowabsmax(const float* __restrict__ w, int64_t k,
+                                                   float* __restrict__ out) {
+  const f32x4* src = reinterpret_cast<const f32x4*>(w + (int64_t)blockIdx.x * k);
+  float m = 0.0f;
+  for (int64_t i = threadIdx.x; i < k / 4; i += 1024) {
+    f32x4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = i + 256 * u < k / 4 ? src[i + 256 * u] : (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(v[u][e]));
+  }
+  m = wg_max(m);
+  if (threadIdx.x == 0) out[blockIdx.x] = m;
+}
+
+// Per-row scale and bytes in one pass: a workgroup holds its row (k <= 1024
+// NV values) in registers between the absmax and the encoding, so the weight
+// is read once. HBM-bound: 5 bytes per value; 9216 x 3072 in 33 us against 75
+// us for absmax, scale and encode launches (0.23 GB moved instead of 0.14).
+template <int NV>
+__global__ void __launch_bounds__(256) k_fp8_rows(const float* __restrict__ w, int64_t k, float* __restrict__ scales,
+                                                  uint8_t* __restrict__ out) {
+  const int64_t row = blockIdx.x;
+  const f32x4* src = reinterpret_cast<const f32x4*>(w + row * k);
+  const int n4 = (int)(k / 4);
+  f32x4 v[NV];
+  float m = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (int)threadIdx.x + 256 * i;
+    v[i] = c < n4 ? src[c] : (f32x4){0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(v[i][e]));
+  const float s = fp8_scale(wg_max(m));
+  if (threadIdx.x == 0) scales[row] = s;
+  const bool fast = s < 3.0e38f;
+  const float y = 1.0f / s;
+  uint32_t* dst = reinterpret_cast<uint32_t*>(out + row * k);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (int)threadIdx.x + 256 * i;
+    if (c < n4) dst[c] = fp8x4_encode(v[i], s, y, fast);
+  }
 }
 
 __global__ void __launch_bounds__(256) k_fp8_scales(float* __restrict__ amax, int64_t n,
                                                     int per_channel, float* __restrict__ scales) {
   if (per_channel) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-      float s = amax[i] / 448.0f;
-      scales[i] = s < 1e-12f ? 1e-12f : s;
+      scales[i] = fp8_scale(amax[i]);
     }
   } else if (blockIdx.x == 0) {
     float m = 0.0f;
     for (int64_t i = threadIdx.x; i < n; i += blockDim.x) m = fmaxf(m, amax[i]);
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    __shared__ float red[4];
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      float s = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) / 448.0f;
-      scales[0] = s < 1e-12f ? 1e-12f : s;
-    }
+    m = wg_max(m);
+    if (threadIdx.x == 0) scales[0] = fp8_scale(m);
   }
 }
 
@@ -174,11 +250,8 @@ __global__ void __launch_bounds__(256) k_fp8_encode(const float* __restrict__ w,
   if (tid >= total) return;
   const int64_t row = (tid * 4) / k;
   const float s = per_channel ? scales[row] : scales[0];
-  f32x4 v = *reinterpret_cast<const f32x4*>(w + tid * 4);
-  uint32_t word = 0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) word |= fp8_encode_rne(v[j] / s) << (8 * j);
-  reinterpret_cast<uint32_t*>(out)[tid] = word;
+  reinterpret_cast<uint32_t*>(out)[tid] =
+      fp8x4_encode(*reinterpret_cast<const f32x4*>(w + tid * 4), s, 1.0f / s, s < 3.0e38f);
 }
 
 // ------------------------------------------------------------------ blocked layout
@@ -195,85 +268,134 @@ LRQ_DEV int64_t blk_data_off(int fmt, int64_t n, int64_t k, int64_t KB) {
   return (((n >> 6) * KB + kb) * 64 + (n & 63)) * rb + ((fmt == LRQ_FMT_INT4) ? (kin >> 1) : kin);
 }
 
-// one thread per 16 output bytes of the blocked data
-__global__ void __launch_bounds__(256) k_block_data(const uint8_t* __restrict__ src, int64_t n, int64_t k,
-                                                    int fmt, int64_t NB, int64_t KB, uint8_t* __restrict__ dst) {
-  const int64_t rb = (fmt == LRQ_FMT_INT4) ? 32 : 64;
-  const int64_t chunks = NB * KB * 64 * (rb / 16);
-  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid >= chunks) return;
-  const int64_t per_row = rb / 16, per_blk = 64 * per_row;
-  const int64_t blk = tid / per_blk, inb = tid % per_blk;
-  const int64_t nb = blk / KB, kb = blk % KB;
-  const int64_t row = nb * 64 + inb / per_row;
-  const int64_t kcol = kb * 64 + (inb % per_row) * ((fmt == LRQ_FMT_INT4) ? 32 : 16);
-  u32x4 v;
-  const uint32_t fill = (fmt == LRQ_FMT_INT4) ? 0x88888888u : 0u;
-  v[0] = v[1] = v[2] = v[3] = fill;
-  if (row < n && kcol < k) {
-    const int64_t rowb = (fmt == LRQ_FMT_INT4) ? k / 2 : k;
-    v = ld16(src + row * rowb + ((fmt == LRQ_FMT_INT4) ? kcol / 2 : kcol));
+// Both sections and both scale tables in one pass. The second, transposed
+// section is read by the input-gradient GEMM (its reduction runs along n):
+// the blocked layout of W^T [k, n], i.e. 64 (k) x 64 (n) blocks, block (kb,
+// nb) at (kb * NB + nb) * block bytes, block row r = k. int4: 32 bytes per
+// row, byte c holding n = 2c in its low nibble and 2c+1 in its high nibble,
+// each nibble q in two's complement (the kernel sign-extends it); fp8 and
+// int8: 64 bytes per row, bytes as in the row layout. Padding is q = 0
+// (int4) or byte 0 (fp8, int8). Scales: [NB][Gp][64] and ST [Gp][NB*64],
+// ST[kg][n] = scale of row n, group kg (zero for padding rows and groups).
+//
+// A workgroup takes 64 rows x 128 bytes of the row layout (int4: 256 columns,
+// four blocks; 8-bit: 128 columns, two) through LDS: 16-byte coalesced loads,
+// 16-byte stores of whole blocks in both sections. The transpose works in
+// registers on 8 x 8 nibbles (8 dwords, three rounds of exchanges, 4
+// instructions a value) or 4 x 4 bytes. HBM-bound: the packed bytes read once
+// and written twice. 12288 x 3072 int4 13 us; one thread per 16 output bytes
+// gathering 32 single bytes from as many rows, and three more launches, took
+// 58 us.
+constexpr int BLK_ST = 33;  // LDS row stride in dwords (an odd number: no bank conflicts down a column)
+
+LRQ_DEV void transpose8_nibbles(uint32_t (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // 16-bit halves
+    const uint32_t a = v[i], b = v[i + 4];
+    v[i] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+    v[i + 4] = __builtin_amdgcn_perm(b, a, 0x07060302u);
   }
-  st16(dst + tid * 16, v);
+#pragma unroll
+  for (int h = 0; h < 8; h += 4)
+#pragma unroll
+    for (int i = h; i < h + 2; ++i) {  // bytes
+      const uint32_t a = v[i], b = v[i + 2];
+      v[i] = __builtin_amdgcn_perm(b, a, 0x06020400u);
+      v[i + 2] = __builtin_amdgcn_perm(b, a, 0x07030501u);
+    }
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {  // nibbles
+    const uint32_t a = v[i], b = v[i + 1];
+    v[i] = (a & 0x0f0f0f0fu) | ((b << 4) & 0xf0f0f0f0u);
+    v[i + 1] = ((a >> 4) & 0x0f0f0f0fu) | (b & 0xf0f0f0f0u);
+  }
 }
 
-__global__ void __launch_bounds__(256) k_block_scales(const float* __restrict__ src, int64_t n, int64_t G,
-                                                      int64_t NB, int64_t Gp, float* __restrict__ dst) {
-  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid >= NB * Gp * 64) return;
-  const int64_t r = tid & 63, j = (tid >> 6) % Gp, nb = (tid >> 6) / Gp;
-  const int64_t row = nb * 64 + r;
-  dst[tid] = (row < n && j < G) ? src[row * G + j] : 0.0f;
+LRQ_DEV void transpose4_bytes(uint32_t (&v)[4]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t a = v[i], b = v[i + 2];
+    v[i] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+    v[i + 2] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i += 2) {
+    const uint32_t a = v[i], b = v[i + 1];
+    v[i] = __builtin_amdgcn_perm(b, a, 0x06020400u);
+    v[i + 1] = __builtin_amdgcn_perm(b, a, 0x07030501u);
+  }
 }
 
-// Transposed section, read by the input-gradient GEMM (its reduction runs
-// along n): the blocked layout of W^T [k, n], i.e. 64 (k) x 64 (n) blocks,
-// block (kb, nb) at (kb * NB + nb) * block bytes, block row r = k. int4: 32
-// bytes per row, byte c holding n = 2c in its low nibble and 2c+1 in its high
-// nibble, each nibble q in two's complement (the kernel sign-extends it);
-// fp8 and int8: 64 bytes per row, bytes as in the row layout. Padding is
-// q = 0 (int4) or byte 0 (fp8, int8). One thread
-// per 16 output bytes (32 or 16 values of one k row, gathered from as many
-// rows of the row layout).
-__global__ void __launch_bounds__(256) k_block_data_t(const uint8_t* __restrict__ src, int64_t n, int64_t k,
-                                                      int fmt, int64_t NB, int64_t KB, uint8_t* __restrict__ dst) {
-  const bool i4 = fmt == LRQ_FMT_INT4;
-  const int64_t per_row = i4 ? 2 : 4;  // 16-byte chunks per block row
-  const int64_t chunks = KB * NB * 64 * per_row;
-  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid >= chunks) return;
-  const int64_t per_blk = 64 * per_row;
-  const int64_t blk = tid / per_blk, inb = tid % per_blk;
-  const int64_t kb = blk / NB, nb = blk % NB;
-  const int64_t kk = kb * 64 + inb / per_row;
-  const int64_t n0 = nb * 64 + (inb % per_row) * (i4 ? 32 : 16);
-  u32x4 v = zero4();
-  if (kk < k) {
-    if (i4) {
-      for (int e = 0; e < 32; ++e) {
-        if (n0 + e >= n) break;
-        const uint32_t byte = src[(n0 + e) * (k / 2) + kk / 2];
-        const uint32_t u = (kk & 1) ? (byte >> 4) : (byte & 15u);  // q + 8
-        v[e >> 3] |= ((u - 8u) & 15u) << (4 * (e & 7));
-      }
-    } else {
-      for (int e = 0; e < 16; ++e) {
-        if (n0 + e >= n) break;
-        v[e >> 2] |= (uint32_t)src[(n0 + e) * k + kk] << (8 * (e & 3));
-      }
+template <bool I4>
+__global__ void __launch_bounds__(256) k_block(const uint8_t* __restrict__ src, const float* __restrict__ ssrc, int64_t n,
+                                               int64_t k, int g, int64_t NB, int64_t KB, int64_t KBX, uint8_t* __restrict__ dst,
+                                               uint8_t* __restrict__ dstt, float* __restrict__ sdst,
+                                               float* __restrict__ sdstt) {
+  constexpr int NBK = I4 ? 4 : 2;          // blocks per workgroup
+  constexpr int RB = I4 ? 32 : 64;         // bytes per block row
+  constexpr uint32_t fill = I4 ? 0x88888888u : 0u;
+  __shared__ uint32_t sr[64 * BLK_ST];                                      // rows [64][128 bytes]
+  __shared__ __attribute__((aligned(16))) uint32_t st_[64 * NBK * RB / 4];  // transposed [64 NBK][RB bytes]
+  const int tid = threadIdx.x;
+  const int64_t nb = blockIdx.x / KBX, kb0 = blockIdx.x % KBX * NBK;
+  const int64_t rowb = I4 ? k / 2 : k, b0 = kb0 * RB;  // the row layout's row bytes; this workgroup's first
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int id = tid + 256 * q, r = id >> 3, c = (id & 7) * 16;
+    u32x4 v = {fill, fill, fill, fill};
+    // (k is a multiple of 32, so 16 bytes are in or out together)
+    if (nb * 64 + r < n && b0 + c < rowb) v = ld16(src + (nb * 64 + r) * rowb + b0 + c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sr[r * BLK_ST + (c >> 2) + e] = v[e];
+  }
+  __syncthreads();
+  // row section: 16-byte chunk id of the workgroup's blocks
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int id = tid + 256 * q, blk = id / (4 * RB), in = id % (4 * RB), r = in / (RB / 16), c = in % (RB / 16);
+    u32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = sr[r * BLK_ST + blk * (RB / 4) + c * 4 + e];
+    if (kb0 + blk < KB) st16(dst + ((nb * KB + kb0 + blk) * 64 + r) * RB + c * 16, v);
+  }
+  if (I4) {
+    // columns 8 i .. +8 of rows 8 j .. +8
+    const int i = tid >> 3, j = tid & 7;
+    uint32_t v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = sr[(8 * j + e) * BLK_ST + i];
+    transpose8_nibbles(v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) st_[(8 * i + e) * (RB / 4) + j] = v[e] ^ 0x88888888u;  // q + 8 -> two's complement
+  } else {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int id = tid + 256 * q, i = id >> 4, j = id & 15;
+      uint32_t v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = sr[(4 * j + e) * BLK_ST + i];
+      transpose4_bytes(v);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st_[(4 * i + e) * (RB / 4) + j] = v[e];
     }
   }
-  st16(dst + tid * 16, v);
-}
-
-// int4 and int8 scales of the transposed section: ST [KGt][NB*64], ST[kg][n] = scale
-// of row n, group kg (zero for padding rows and groups).
-__global__ void __launch_bounds__(256) k_block_scales_t(const float* __restrict__ src, int64_t n, int64_t G,
-                                                        int64_t KGt, int64_t NP, float* __restrict__ dst) {
-  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid >= KGt * NP) return;
-  const int64_t kg = tid / NP, row = tid % NP;
-  dst[tid] = (row < n && kg < G) ? src[row * G + kg] : 0.0f;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int id = tid + 256 * q, blk = id / (4 * RB), in = id % (4 * RB);
+    if (kb0 + blk < KB) st16(dstt + ((kb0 + blk) * NB + nb) * 64 * RB + in * 16, *reinterpret_cast<const u32x4*>(st_ + id * 4));
+  }
+  if (!sdst) return;
+  // group scales of the workgroup's columns (a group wider than them: its
+  // first workgroup), one row per thread
+  const int64_t G = k / g, Gp = KB * 64 / g;
+  const int64_t j0 = (kb0 * 64 + g - 1) / g, j1 = min(Gp, ((kb0 + NBK) * 64 + g - 1) / g);
+  const int64_t row = nb * 64 + (tid & 63);
+  for (int64_t j = j0 + (tid >> 6); j < j1; j += 4) {
+    const float v = (row < n && j < G) ? ssrc[row * G + j] : 0.0f;
+    sdst[(nb * Gp + j) * 64 + (tid & 63)] = v;
+    sdstt[j * NB * 64 + row] = v;
+  }
 }
 
 // ------------------------------------------------------------------ dequantize
@@ -391,6 +513,18 @@ hipError_t launch_requantize_fp8_int4(hipStream_t st, const uint8_t* bytes, cons
 hipError_t launch_quantize_fp8(hipStream_t st, const float* w, int64_t n, int64_t k,
                                int per_channel, uint8_t* bytes, float* scales, float* amax_ws) {
   if (n == 0 || k == 0) return hipSuccess;
+  if (per_channel && k <= 16 * 1024) {
+    const dim3 grid((unsigned)n);
+    if (k <= 2 * 1024)
+      hipLaunchKernelGGL(k_fp8_rows<2>, grid, dim3(256), 0, st, w, k, scales, bytes);
+    else if (k <= 4 * 1024)
+      hipLaunchKernelGGL(k_fp8_rows<4>, grid, dim3(256), 0, st, w, k, scales, bytes);
+    else if (k <= 8 * 1024)
+      hipLaunchKernelGGL(k_fp8_rows<8>, grid, dim3(256), 0, st, w, k, scales, bytes);
+    else
+      hipLaunchKernelGGL(k_fp8_rows<16>, grid, dim3(256), 0, st, w, k, scales, bytes);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_rowabsmax, dim3((unsigned)n), dim3(256), 0, st, w, k, amax_ws);
   hipLaunchKernelGGL(k_fp8_scales, dim3(per_channel ? blocks_for(n, 256) : 1), dim3(256), 0, st,
                      amax_ws, n, per_channel, scales);
@@ -458,16 +592,17 @@ hipError_t launch_block(hipStream_t st, const lrq_weight* w, uint8_t* data, floa
   blocked_sections(w->format, n, k, w->group, &db, &sc);
   if (db == 0) return hipSuccess;
   const uint8_t* src = reinterpret_cast<const uint8_t*>(w->data);
-  hipLaunchKernelGGL(k_block_data, dim3(blocks_for(db / 16, 256)), dim3(256), 0, st, src, n, k, w->format, NB, KB,
-                     data);
-  hipLaunchKernelGGL(k_block_data_t, dim3(blocks_for(db / 16, 256)), dim3(256), 0, st, src, n, k, w->format, NB,
-                     KB, data + db);
-  if (w->format != LRQ_FMT_FP8 && sc > 0) {
-    hipLaunchKernelGGL(k_block_scales, dim3(blocks_for(sc, 256)), dim3(256), 0, st, w->scales, n,
-                       k / w->group, NB, KB * 64 / w->group, scales);
-    const int64_t st_count = blocked_t_scale_count(w->format, n, k, w->group);
-    hipLaunchKernelGGL(k_block_scales_t, dim3(blocks_for(st_count, 256)), dim3(256), 0, st, w->scales, n,
-                       k / w->group, st_count / (NB * 64), NB * 64, scales + sc);
-  }
+  const bool gs = w->format != LRQ_FMT_FP8 && sc > 0;
+  const int nbk = w->format == LRQ_FMT_INT4 ? 4 : 2;
+  const int64_t kbx = (KB + nbk - 1) / nbk;
+  const dim3 grid((unsigned)(kbx * NB));
+  float* const s0 = gs ? scales : nullptr;
+  float* const s1 = gs ? scales + sc : nullptr;
+  if (w->format == LRQ_FMT_INT4)
+    hipLaunchKernelGGL(k_block<true>, grid, dim3(256), 0, st, src, w->scales, n, k, w->group, NB, KB, kbx, data,
+                       data + db, s0, s1);
+  else
+    hipLaunchKernelGGL(k_block<false>, grid, dim3(256), 0, st, src, w->scales, n, k, w->group, NB, KB, kbx, data,
+                       data + db, s0, s1);
   return hipGetLastError();
 }
