@@ -40,6 +40,11 @@ extern "C" {
 /* Message of the last failed call on this host thread ("" if none). */
 const char* lmd_last_error(void);
 
+/* The rotation tables cos, sin f32 [l, ceil(head_dim / 2)]: pair j of position
+ * p turns by p * theta^(-2j / head_dim), the angle and its cosine and sine
+ * formed in f64 and rounded once (mmdit.rs:385-399's angles). */
+int lmd_rope_tables(int64_t l, int head_dim, double theta, float* cos, float* sin, void* stream);
+
 /* q = rope(x_q * rstd_q), k = rope(x_k * rstd_k), v = x_v, per head, in f32,
  * rounded once to bf16 (mmdit.rs:599-619 for one token sequence). */
 int lmd_attn_prep_fwd(const uint16_t* qkv_txt, int64_t l_txt, const uint16_t* qkv_img, int64_t l_img,

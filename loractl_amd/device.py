@@ -57,7 +57,9 @@ class Context:
     def call(self, name: str, *args):
         """Call ``name(ctx, *args)`` under the context's lock; raise on error."""
         with self.lock:
-            self.check(getattr(self.lib, name)(self.h, *args), name)
+            rc = getattr(self.lib, name)(self.h, *args)
+            if rc != 0:
+                self.check(rc, name)
 
 
 _ctx_lock = threading.Lock()
@@ -69,17 +71,18 @@ def context(device: Optional[int] = None) -> Context:
     current stream on it."""
     if device is None:
         device = torch.cuda.current_device()
-    stream = torch.cuda.current_stream(device).cuda_stream
-    key = (device, stream)
-    with _ctx_lock:
-        c = _ctxs.get(key)
-        if c is None:
-            c = _ctxs[key] = Context(device, stream)
+    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    c = _ctxs.get(key)  # (contexts are never removed)
+    if c is None:
+        with _ctx_lock:
+            c = _ctxs.get(key)
+            if c is None:
+                c = _ctxs[key] = Context(*key)
     return c
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _need(t: torch.Tensor, dtype: torch.dtype, name: str, shape=None):

@@ -52,8 +52,8 @@ class _QuantLoraFn(torch.autograd.Function):
                 factors=None):
         xb = x2.to(torch.bfloat16).contiguous()
         if factors is None:
-            ab = a.detach().to(torch.bfloat16).contiguous()
-            bb = b.detach().to(torch.bfloat16).contiguous()
+            ab = a.to(torch.bfloat16).contiguous()
+            bb = b.to(torch.bfloat16).contiguous()
         else:
             ab, bb = factors
         y, t = D.lora_fwd(xb, wq, ab, bb, scaling)

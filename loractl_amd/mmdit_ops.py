@@ -23,10 +23,11 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libloractl_mmdit.so")
 
-_vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
+_vp, _i64, _i32, _f32, _f64 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float, ctypes.c_double
 SIGNATURES = {
     "lmd_last_error": ([], ctypes.c_char_p),
     "lmd_colsum_groups": ([_i64], _i64),
+    "lmd_rope_tables": ([_i64, _i32, _f64, _vp, _vp, _vp], _i32),
     "lmd_modnorm_fwd": ([_vp, _i64, _i32, _vp, _vp, _f32, _vp, _vp, _vp], _i32),
     "lmd_modnorm_bwd": ([_vp, _vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp], _i32),
     "lmd_gated_residual_bwd": ([_vp, _vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp], _i32),
@@ -60,7 +61,16 @@ def _check(rc: int, what: str) -> None:
 
 def rope_tables(L: int, head_dim: int, device, theta: float = 10000.0) -> Tuple[torch.Tensor, torch.Tensor]:
     """(cos, sin) f32 ``[L, head_dim / 2]``: pair (2j, 2j+1) of position p
-    turns by ``p * theta^(-2j / head_dim)``; the angles are formed in f64."""
+    turns by ``p * theta^(-2j / head_dim)``; the angles are formed in f64
+    (on a GPU by one kernel on the current stream)."""
+    dev = torch.device(device)
+    if dev.type == "cuda":
+        cos = torch.empty((L, (head_dim + 1) // 2), device=dev, dtype=torch.float32)
+        sin = torch.empty_like(cos)
+        with torch.cuda.device(cos.device):
+            _check(load().lmd_rope_tables(L, head_dim, theta, _ptr(cos), _ptr(sin), _stream(cos.device)),
+                   "lmd_rope_tables")
+        return cos, sin
     inv = theta ** (-torch.arange(0, head_dim, 2, dtype=torch.float64) / head_dim)
     ang = torch.arange(L, dtype=torch.float64)[:, None] * inv[None]
     return (torch.cos(ang).float().contiguous().to(device), torch.sin(ang).float().contiguous().to(device))
