@@ -234,6 +234,26 @@ LRQ_DEV void mul_row_bcast8(float (&f)[8], float v, int h) {
         : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]), "+v"(f[7])
         : "v"(v));
 }
+// The same for four values: f[e] *= lane L + e, L = 0, 4, 8 or 12 (e = 0..3).
+LRQ_DEV void mul_row_bcast4(float& f0, float& f1, float& f2, float& f3, float v, int L) {
+#define LRQ_MUL4(A, B, C, D)                                                                  \
+  asm volatile("s_nop 1\n"                                                                    \
+               "v_mul_f32_dpp %0, %4, %0 row_newbcast:" #A " row_mask:0xf bank_mask:0xf bound_ctrl:1\n" \
+               "v_mul_f32_dpp %1, %4, %1 row_newbcast:" #B " row_mask:0xf bank_mask:0xf bound_ctrl:1\n" \
+               "v_mul_f32_dpp %2, %4, %2 row_newbcast:" #C " row_mask:0xf bank_mask:0xf bound_ctrl:1\n" \
+               "v_mul_f32_dpp %3, %4, %3 row_newbcast:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:1\n" \
+               : "+v"(f0), "+v"(f1), "+v"(f2), "+v"(f3)                                       \
+               : "v"(v))
+  if (L == 0)
+    LRQ_MUL4(0, 1, 2, 3);
+  else if (L == 4)
+    LRQ_MUL4(4, 5, 6, 7);
+  else if (L == 8)
+    LRQ_MUL4(8, 9, 10, 11);
+  else
+    LRQ_MUL4(12, 13, 14, 15);
+#undef LRQ_MUL4
+}
 #undef LRQ_MUL_BCAST
 
 // ---------------------------------------------------------------- buffer loads

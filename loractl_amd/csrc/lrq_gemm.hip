@@ -48,8 +48,24 @@
 //     of a tile prefetch the first steps of the workgroup's next tile, so
 //     that tile's loads are in flight while this tile's epilogue (LoRA step,
 //     bias, stores) runs, and the stores drain under the next tile's
-//     matrix-core work. The one barrier of a step sits between its third and
-//     fourth sub-steps, after the last fragment reads of the current buffer;
+//     matrix-core work. The one barrier of a step sits four matrix-core steps
+//     into its fourth sub-step, after the last fragment reads of the current
+//     buffer;
+//   - the order inside a sub-step: with one wavefront per SIMD nothing else
+//     issues while a run of conversions goes by, so what the next sub-step
+//     needs (8 activation reads, two weight fragments in 4 or 6 pieces each,
+//     and in the fourth sub-step the copies of the refill) is dealt out over
+//     the 12 or 16 matrix-core steps. The two passes of the base product at
+//     4096 tokens, us (before: reads, conversions and copies in front of the
+//     sub-step's matrix-core steps, placed by the compiler):
+//                            forward            backward
+//       int4  3072->12288    254 -> 252         273 -> 262
+//       int4 12288->3072     280 -> 270         268 -> 248
+//       int4  4096->4096     116 -> 115         118 -> 112
+//       int8  3072->12288    276 -> 257         287 -> 267
+//       fp8   3072-> 9216    211 -> 199         223 -> 219
+//     which is 1.06 to 1.25 PFLOP/s; a plain bf16 product of these sizes
+//     reaches 1.36 to 1.43 here, power-limited;
 //   - edges: buffer loads past a resource's size return zeros (partial token
 //     and weight tiles, the depth tail and the zero step that rounds a tile's
 //     steps up to an even count); padding weight rows and depth columns hold
@@ -71,6 +87,8 @@
 //     partials in range order, applies the forward fp8 scales and bias and
 //     rounds once to bf16.
 
+#include <type_traits>
+
 #include "lrq_common.h"
 #include "lrq_kernels.h"
 
@@ -87,6 +105,15 @@ constexpr int NBUF = 2;        // pipeline depth (LDS buffers, register sets)
 // row r at chunk c ^ swz(r), so the 16 lanes of a read pass (16 rows at one
 // logical chunk) cover all 64 banks
 LRQ_DEV int swz(int r) { return (r >> 1) & 7; }
+
+// f(0), f(1), .. f(N - 1) with constant arguments
+template <int N, int I = 0, class F>
+LRQ_DEV void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
 
 // Per-unit load sources: the activation rows of wavefront w's DMA share, the
 // weight block row(s) (data; forward int4 scales), backward int4 the byte
@@ -189,7 +216,7 @@ k_gemm(GemmArgs a, int tiles_m, int ntiles) {
   const int drow = lane >> 3;
   const int dq0 = (lane & 7) ^ ((lane >> 4) & 7), dq1 = (lane & 7) ^ (((lane >> 4) + 4) & 7);
   const uint32_t doff0 = (uint32_t)((drow * K + dq0 * 8) * 2), doff1 = (uint32_t)((drow * K + dq1 * 8) * 2);
-  auto dma = [&](uint16_t* buf, const rsrc_t& ract, int kt) {
+  auto dma = [&](uint16_t* buf, const rsrc_t& ract, int kt, int only) {  // copy `only`, or all (-1)
     const int64_t k0 = (int64_t)kt * BK;
     const bool kok0 = k0 + dq0 * 8 < K, kok1 = k0 + dq1 * 8 < K;  // K % 8 == 0
     const uint32_t koff = (uint32_t)(k0 * 2);
@@ -200,6 +227,7 @@ k_gemm(GemmArgs a, int tiles_m, int ntiles) {
     const uint32_t o0 = opaque_u32(doff0) + koff, o1 = opaque_u32(doff1) + koff;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
+      if (only >= 0 && c != only) continue;
       const bool kok = (c & 1) ? kok1 : kok0;
       const uint32_t off = opaque_u32(kok ? ((c & 1) ? o1 : o0) + (uint32_t)(c * 8 * K * 2) : LRQ_OOB);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ract, (lds_void*)(base + c * 8 * BK * 2), 16, off, 0, 0, 0);
@@ -316,38 +344,117 @@ k_gemm(GemmArgs a, int tiles_m, int ntiles) {
   uint16_t* const bufs[2] = {sX0, sX1};
   bf16x8 fa[2][2], fb[2][MJ];
 
+  // The A-role fragment of row tile i, sub-step kk in pieces: piece p
+  // (0 .. NPC - 1) forms part of `o` (wfrag's value once all have run). The
+  // pieces sit one by one between matrix-core steps: left to itself, the
+  // compiler runs 15 to 30 of these instructions in a row with the matrix
+  // cores idle (one wavefront per SIMD has nothing else to issue), then eight
+  // matrix-core steps with none.
+  constexpr int NPC = BWD ? 6 : 4;  // forward: two values each; backward: 2, 2, scale and pack four, again
+  auto wpiece = [&](int set, int i, int kk, int p, float (&f)[8], u32x4& o) {
+    const u32x4 v = wp[set][i * WV + (I4 ? 0 : (kk >> 1))];
+    const uint32_t d4 = v[kk];                                     // int4: eight nibbles
+    const uint32_t d8[2] = {v[2 * (kk & 1)], v[2 * (kk & 1) + 1]};  // 8-bit: two dwords of four
+    if (!BWD) {
+      const int e = 2 * p;  // values e, e + 1
+      if (I4) {
+        const float sc = wsc[set][i], nb = -8.0f * sc;
+        const uint32_t lo = d4 & a.nib, hi = (d4 >> 4) & a.nib;
+        o[p] = pack_bf16x2(__builtin_fmaf((float)((lo >> (8 * p)) & 0xffu), sc, nb),
+                           __builtin_fmaf((float)((hi >> (8 * p)) & 0xffu), sc, nb));
+      } else if (I8) {
+        const float sc = wsc[set][i], nb = -128.0f * sc;
+        const uint32_t u = d8[e >> 2] ^ 0x80808080u;
+        o[p] = pack_bf16x2(__builtin_fmaf((float)((u >> (8 * (e & 3))) & 0xffu), sc, nb),
+                           __builtin_fmaf((float)((u >> (8 * (e & 3) + 8)) & 0xffu), sc, nb));
+      } else {
+        const f32x2 q = (e & 2) ? __builtin_amdgcn_cvt_pk_f32_fp8((int)d8[e >> 2], true)
+                                : __builtin_amdgcn_cvt_pk_f32_fp8((int)d8[e >> 2], false);
+        o[p] = pack_bf16x2(q[0], q[1]);
+      }
+      asm volatile("" : "+v"(o[p]));  // formed here, not where it is first used
+      return;
+    }
+    const int h = p / 3, r = p % 3;  // four values 4 h .. 4 h + 3
+    if (r < 2) {
+      const int e = 4 * h + 2 * r;
+      if (I4) {
+        f[e] = (float)((int)(d4 << (28 - 4 * e)) >> 28);
+        f[e + 1] = (float)((int)(d4 << (24 - 4 * e)) >> 28);
+      } else if (I8) {
+        f[e] = (float)((int)(d8[h] << (24 - 16 * r)) >> 24);
+        f[e + 1] = (float)((int)(d8[h] << (16 - 16 * r)) >> 24);
+      } else {
+        const f32x2 q = r ? __builtin_amdgcn_cvt_pk_f32_fp8((int)d8[h], true)
+                          : __builtin_amdgcn_cvt_pk_f32_fp8((int)d8[h], false);
+        f[e] = q[0];
+        f[e + 1] = q[1];
+      }
+      asm volatile("" : "+v"(f[e]), "+v"(f[e + 1]));
+      return;
+    }
+    mul_row_bcast4(f[4 * h], f[4 * h + 1], f[4 * h + 2], f[4 * h + 3], bsc[set][GS ? i : 0][kk >> 1], 8 * (kk & 1) + 4 * h);
+    o[2 * h] = pack_bf16x2(f[4 * h], f[4 * h + 1]);
+    o[2 * h + 1] = pack_bf16x2(f[4 * h + 2], f[4 * h + 3]);
+    asm volatile("" : "+v"(o[2 * h]), "+v"(o[2 * h + 1]));
+  };
+
   // One step on LDS buffer `b` and register set `b` (b = step % 2; the
   // unrolled loop makes both static). On entry fa[0] and fb[0] hold sub-step
   // 0's fragments; on exit they hold the next step's. After the barrier the
-  // step refills buffer and set b with step `lkt` of tile `ls`.
-  auto step = [&](const int b, const TileSrc& ls, const int lkt) {
-    const uint16_t* buf = bufs[b];
-    const int nb_ = (b + 1) % NBUF;
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const int cur = kk & 1;
-      if (kk < 3) {
-#pragma unroll
-        for (int j = 0; j < MJ; ++j) fb[cur ^ 1][j] = xfrag(buf, j, kk + 1);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) fa[cur ^ 1][i] = wfrag(b, i, kk + 1);
-      } else {
-        // every read of buffer b is issued: one barrier, then refill buffer
-        // and register set b, and read the next step's first fragments from
-        // buffer nb_ while sub-step 3 runs
-        __syncthreads();
-        dma(bufs[b], ls.act, lkt);
-        load_w(b, ls, lkt);
-#pragma unroll
-        for (int j = 0; j < MJ; ++j) fb[cur ^ 1][j] = xfrag(bufs[nb_], j, 0);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) fa[cur ^ 1][i] = wfrag(nb_, i, 0);
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < (i == 0 ? MJ : MJ1); ++j) acc[i][j] = mfma32(fa[cur][i], fb[cur][j], acc[i][j]);
-    }
+  // step refills buffer and set b with step `lkt` of tile `ls`. Each
+  // matrix-core step is followed by its share of the next sub-step's
+  // fragment reads and dequantization pieces (sub-step 3: and of the refill).
+  auto step = [&](auto bc, const TileSrc& ls, const int lkt) {
+    constexpr int b = decltype(bc)::value, nb_ = (b + 1) % NBUF;
+    uint16_t* const buf = b ? sX1 : sX0;
+    uint16_t* const nbuf = b ? sX0 : sX1;
+    constexpr int SLOTS = MJ + MJ1;
+    constexpr int BAR = 4;  // sub-step 3: slots before the barrier
+    // Whether a sched_barrier ends every slot, or the compiler places the
+    // pieces. Without / with, us at the sizes above: int4 backward 272 / 262,
+    // 256 / 248, 115 / 112, int8 261 / 257 and 279 / 267, fp8 forward 204 /
+    // 199; but int4 forward (the fewest conversions) 252 / 259, 270 / 274,
+    // 115 / 119 and fp8 backward (the most) 219 / 226.
+    constexpr bool SB = !(I4 && !BWD) && !(FMT == LRQ_FMT_FP8 && BWD);
+    static_for<4>([&](auto kc) {
+      constexpr int kk = decltype(kc)::value, cur = kk & 1;
+      float f[2][8];
+      u32x4 o[2];
+      static_for<SLOTS>([&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        // both row tiles of a token tile in turn (row tile 0's others last), but
+        // one row tile after the other where the compiler places the pieces
+        constexpr int i = SB ? (s < 2 * MJ1 ? s & 1 : 0) : (s < MJ ? 0 : 1);
+        constexpr int j = SB ? (s < 2 * MJ1 ? s / 2 : s - MJ1) : (s < MJ ? s : s - MJ);
+        acc[i][j] = mfma32(fa[cur][i], fb[cur][j], acc[i][j]);
+        if (kk < 3 && s < MJ) fb[cur ^ 1][s < MJ ? s : 0] = xfrag(buf, s, kk + 1);
+        if (kk == 3) {
+          // every read of buffer b is issued: one barrier, then refill buffer
+          // and register set b (its last pieces ran in sub-step 2), and read
+          // the next step's first fragments from the other buffer
+          if (s == BAR) {
+            // the copies into the other buffer have landed: said here, since
+            // the compiler does not carry them over the loop's back edge
+            __builtin_amdgcn_s_waitcnt(0xf70);  // vmcnt(0)
+            __syncthreads();
+            load_w(b, ls, lkt);
+          }
+          if (s >= BAR && s < BAR + MJ) {
+            dma(buf, ls.act, lkt, s - BAR);
+            fb[cur ^ 1][(s - BAR) & (MJ - 1)] = xfrag(nbuf, s - BAR, 0);
+          }
+        }
+        constexpr int p0 = s * 2 * NPC / SLOTS, p1 = (s + 1) * 2 * NPC / SLOTS;
+        static_for<p1 - p0>([&](auto pc) {
+          constexpr int p = p0 + decltype(pc)::value;
+          wpiece(kk < 3 ? b : nb_, p / NPC, (kk + 1) & 3, p % NPC, f[p / NPC], o[p / NPC]);
+        });
+        if constexpr (SB) __builtin_amdgcn_sched_barrier(0);
+      });
+      fa[cur ^ 1][0] = as_bf16x8(o[0]);
+      fa[cur ^ 1][1] = as_bf16x8(o[1]);
+    });
   };
 
   const int rp = a.rp;
@@ -531,11 +638,12 @@ k_gemm(GemmArgs a, int tiles_m, int ntiles) {
   TileSrc cur = tile_src(vb);
 #pragma unroll
   for (int b = 0; b < NBUF; ++b) {
-    dma(bufs[b], cur.act, cur.k0 + b);
+    dma(bufs[b], cur.act, cur.k0 + b, -1);
     load_w(b, cur, cur.k0 + b);
   }
   dma_aux(cur.m0, cur.e0);
   zero_acc();
+  __builtin_amdgcn_s_waitcnt(0xf70);  // vmcnt(0)
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < MJ; ++j) fb[0][j] = xfrag(bufs[0], j, 0);
@@ -545,13 +653,13 @@ k_gemm(GemmArgs a, int tiles_m, int ntiles) {
   for (;;) {
     int kt = 0;
     for (; kt + NBUF < nkp; kt += NBUF) {
-#pragma unroll
-      for (int b = 0; b < NBUF; ++b) step(b, cur, cur.k0 + kt + NBUF + b);
+      step(std::integral_constant<int, 0>{}, cur, cur.k0 + kt + NBUF);
+      step(std::integral_constant<int, 1>{}, cur, cur.k0 + kt + NBUF + 1);
     }
     // last two steps: prefetch the next unit's first steps
     const TileSrc nxt = tile_src(vb + G);
-#pragma unroll
-    for (int b = 0; b < NBUF; ++b) step(b, nxt, nxt.k0 + b);
+    step(std::integral_constant<int, 0>{}, nxt, nxt.k0);
+    step(std::integral_constant<int, 1>{}, nxt, nxt.k0 + 1);
     if (SPLIT)
       epilogue_partial(cur);
     else
