@@ -145,7 +145,14 @@ def test_c4_width_checkpointed_step_with_atomic_attention(cuda):
     (loss_m, gm), (loss_m2, gm2), (loss_c, gc) = _steps(cfg, cuda, ["monolithic", "monolithic", "checkpointed"])
     assert loss_c == loss_m == loss_m2
     noise = [0.0 if r is None else O.rel_deviation(g.cpu().numpy(), r.cpu().numpy()) for r, g in zip(gm, gm2)]
-    worst = _compare(cfg, gm, gc, lambda i: max(1e-3, 4.0 * noise[i]))
+    # A modulation site has one token: its dA is x^T u and its dB t^T dy with u
+    # and dy rounded to bf16, so a value that the noise carries over a rounding
+    # boundary moves a whole column of the gradient by one bf16 ulp. At the
+    # peak that is up to 2^-7 of it, whatever the other pair of steps shows
+    # (seen: 1/231 of the peak, the ulp of 231, in 2 of 13 steps). Sites with
+    # more tokens average such steps out.
+    ulp = [2.0**-7 if p.endswith(".mod") else 0.0 for p in cfg.site_paths()]
+    worst = _compare(cfg, gm, gc, lambda i: max(1e-3, 4.0 * noise[i], ulp[i // 2]))
     print(f"worst gradient deviation {worst:.3e}; monolithic-to-monolithic up to {max(noise):.3e}")
 
 
