@@ -64,11 +64,11 @@ def rope_tables(L: int, head_dim: int, device, theta: float = 10000.0) -> Tuple[
     turns by ``p * theta^(-2j / head_dim)``; the angles are formed in f64
     (on a GPU by one kernel on the current stream)."""
     dev = torch.device(device)
-    if dev.type == "cuda":
+    if dev.type == "cuda" and head_dim > 0:
         cos = torch.empty((L, (head_dim + 1) // 2), device=dev, dtype=torch.float32)
         sin = torch.empty_like(cos)
         with torch.cuda.device(cos.device):
-            _check(load().lmd_rope_tables(L, head_dim, theta, _ptr(cos), _ptr(sin), _stream(cos.device)),
+            _check(load().lmd_rope_tables(L, head_dim, float(theta), _ptr(cos), _ptr(sin), _stream(cos.device)),
                    "lmd_rope_tables")
         return cos, sin
     inv = theta ** (-torch.arange(0, head_dim, 2, dtype=torch.float64) / head_dim)
