@@ -5,6 +5,7 @@ rotation tables at odd sizes."""
 
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -52,3 +53,11 @@ def test_rope_tables_kernel_matches_host(cuda, L, hd, theta):
     assert c.shape == ch.shape == (L, hd // 2) and c.dtype == torch.float32
     if L:
         assert float((c.cpu() - ch).abs().max()) <= 2.0**-24 and float((s.cpu() - sh).abs().max()) <= 2.0**-24
+
+
+def test_rope_tables_kernel_takes_what_the_host_takes(cuda):
+    """A theta that is no Python float, and an empty head."""
+    theta = np.float32(500.0)
+    for got, ref in zip(rope_tables(70, 64, cuda, theta), rope_tables(70, 64, "cpu", theta)):
+        assert float((got.cpu() - ref).abs().max()) <= 2.0**-24
+    assert rope_tables(3, 0, cuda)[0].shape == rope_tables(3, 0, "cpu")[0].shape

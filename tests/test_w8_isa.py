@@ -1,5 +1,6 @@
 """The matrix-core and DPP distances of lrq_gemm_w8.hip's gfx950 build (CPU:
-compiles to assembly), checked as the other kernel files' are."""
+compiles to assembly), checked as the other kernel files' are, and
+the wait for the copies before each barrier of its pipelined loop."""
 
 import os
 import tempfile
@@ -15,6 +16,9 @@ def test_w8_meets_wait_states():
                              os.path.join(ROOT, "include"), d)
     total, bad = 0, []
     for k in H.parse_asm(text):
+        # a stage's barrier publishes the next stage's LDS copies: they have landed
+        waits = H.stage_waits(k)
+        assert "k_w8" not in k.name or (waits and all(w == 0 for w, _ in waits)), (k.name, waits)
         v, n = H.check_kernel(k)
         total += n
         bad += v + H.check_dpp(k)[0]
