@@ -10,7 +10,7 @@ use std::env;
 use std::path::{Path, PathBuf};
 use std::process::Command;
 
-const SOURCES: [&str; 7] = [
+const SOURCES: [&str; 8] = [
     "lrq_quant.hip",
     "lrq_gemm.hip",
     "lrq_gemm_mid.hip",
@@ -36,7 +36,7 @@ fn main() {
     println!("cargo:rerun-if-env-changed=HIPCC");
     println!("cargo:rerun-if-env-changed=ROCM_PATH");
     println!("cargo:rerun-if-changed={}", include.join("loractl_rocm.h").display());
-    for f in ["lrq_common.h", "lrq_kernels.h"] {
+    for f in ["lrq_common.h", "lrq_fold.h", "lrq_kernels.h", "lrq_tn.h"] {
         println!("cargo:rerun-if-changed={}", csrc.join(f).display());
     }
 

@@ -121,6 +121,14 @@ def test_build_script_compiles_every_library_source():
     listed = set(re.findall(r'"(lrq_\w+\.hip)"', src))
     from loractl_amd import _build
     assert listed == set(_build.SOURCES)
+    # the array's declared length is its number of entries (rustc refuses any other)
+    length = int(re.search(r"const SOURCES: \[&str; (\d+)\]", src).group(1))
+    assert length == len(re.findall(r'"(lrq_\w+\.hip)"', src)) == len(_build.SOURCES)
+    # and a change to any header the sources include rebuilds the crate
+    csrc = os.path.join(ROOT, "loractl_amd", "csrc")
+    included = {h for f in _build.SOURCES for h in re.findall(r'#include "(lrq_\w+\.h)"', open(os.path.join(csrc, f)).read())}
+    included |= {h for f in list(included) for h in re.findall(r'#include "(lrq_\w+\.h)"', open(os.path.join(csrc, f)).read())}
+    assert set(re.findall(r'"(lrq_\w+\.h)"', src)) == included
     assert "--offload-arch=gfx950" in src and "-packed-fp32-ops" in src
     assert 'links = "loractl_rocm"' in open(os.path.join(CRATE, "Cargo.toml")).read()
 
