@@ -275,6 +275,16 @@ int lrq_debug_force_wait_timeout(int on);
  * if another needs more. */
 int lrq_debug_gemm_path(int path);
 
+/* Test hook, no counterpart in the reference; host only, no context: how a
+ * call of m tokens at rank r (0: no adapter) would run. pass 0 the forward, 1
+ * the backward with an input gradient; out[0] = its workspace bytes, and past
+ * 16 tokens out[1] = the kernel (0 the 256-token tiles; the mid-size tiles of
+ * 1: 64 x 64, 2: 128 x 128, 3: 256 rows x 128 tokens), out[2] = its depth
+ * ranges, out[3] = 1 if it forms the adapter's products in its own launch.
+ * pass 2: out[0] = what lrq_reserve takes. out[4] = cost-model evaluations of
+ * this process before the call. */
+int lrq_debug_plan(int pass, int64_t m, int64_t n, int64_t k, int64_t r, int64_t* out);
+
 #ifdef __cplusplus
 }
 #endif

@@ -219,40 +219,138 @@ int ensure_ws(lrq_ctx* c, size_t bytes) {
   return LRQ_OK;
 }
 
-// Workspace layout of the fused calls (sizes only when base == nullptr): t
-// and u padded to rp columns (the GEMM epilogue operands) and the f32
-// partials of the LoRA reductions (t or u; dA and dB side by side).
-// f32 partials of the fused GEMMs when they split the depth (few output
-// tiles): the larger of the forward's and the backward's
-int64_t gemm_part_floats(int64_t m, int64_t n, int64_t k) {
-  return std::max(gemm_split_floats(m, n, k), gemm_split_floats(m, k, n));
-}
-
-// LoRA workspace: t and u padded to rp columns, the weight-side factor rows
-// of the fused GEMM's LoRA step (B^T [n, rp] forward, A [k, rp] backward),
-// the side kernels' f32 partials and the fused GEMMs' split partials.
+// LoRA workspace (sizes only when base == nullptr) of a pass with its side
+// launches: t (u) padded to rp columns, the weight-side factor rows of the
+// fused GEMM's LoRA step (B^T [n, rp] forward, A [k, rp] backward), the side
+// kernels' f32 partials (backward also dA's and dB's). The GEMM's own partials
+// follow it.
 struct LoraWs {
-  uint16_t *tp, *up, *fr;
-  float *pn, *pa, *pb, *gp;
+  uint16_t *tp, *fr;  // t forward, u backward
+  float *pn, *pa, *pb;
   size_t bytes;
 };
 
-// fwd_only: the forward's slices alone (t, the B^T rows, t's partials and
-// the forward GEMM's split partials); u and the dA/dB partials take no bytes
-LoraWs lora_layout(char* base, int64_t m, int64_t n, int64_t k, int rp, bool fwd_only = false) {
+LoraWs lora_layout(char* base, int64_t m, int64_t n, int64_t k, int rp, bool bwd) {
   Slab s{base};
   LoraWs w{};
   w.tp = s.take<uint16_t>(m * rp);
-  w.up = s.take<uint16_t>(fwd_only ? 0 : m * rp);
-  w.fr = s.take<uint16_t>((fwd_only ? n : std::max(n, k)) * rp);
-  const int64_t nt = fwd_only ? lora_plan_nt(m, k, rp).splits
-                              : std::max((int64_t)lora_plan_nt(m, k, rp).splits, (int64_t)lora_plan_nt(m, n, rp).splits);
+  w.fr = s.take<uint16_t>((bwd ? k : n) * rp);
+  const int64_t nt = lora_plan_nt(m, bwd ? n : k, rp).splits;
   w.pn = s.take<float>(std::max(nt * round_up(m, 128) * rp, (int64_t)1));
-  w.pa = s.take<float>(fwd_only ? 0 : (int64_t)lora_plan_tn(m, k, rp).splits * k * rp);
-  w.pb = s.take<float>(fwd_only ? 0 : (int64_t)lora_plan_tn(m, n, rp).splits * n * rp);
-  w.gp = s.take<float>(std::max(fwd_only ? gemm_split_floats(m, n, k) : gemm_part_floats(m, n, k), (int64_t)1));
+  w.pa = s.take<float>(bwd ? (int64_t)lora_plan_tn(m, k, rp).splits * k * rp : 0);
+  w.pb = s.take<float>(bwd ? (int64_t)lora_plan_tn(m, n, rp).splits * n * rp : 0);
   w.bytes = s.off;
   return w;
+}
+
+// How a LoRA pass of m > 16 tokens runs, and the workspace it takes. fold:
+// ranks 8 to 32 (multiples of 8) may form t (u, dA and dB) in the launch of
+// mid-size tiles, by workgroups ahead of (and after) the tiles: the factor's
+// slice partials, then the tiles' depth-range partials, then (backward, after
+// the LoRA workspace) dB's and dA's token-slice partials.
+struct LoraPass {
+  bool fold = false;
+  GemmPlan g;
+  int64_t G = 0, fs = 0;           // 64-token groups, depth slices of the factor
+  int64_t fp = 0, ms = 0;          // floats: the factor's partials, the ranges'
+  size_t bytes = 0;
+  // backward: the weight gradients in the fold's launch (fold_tn)
+  bool fold_tn = false;
+  LoraPlan tpb{}, tpa{};
+  int64_t tb = 0, ta = 0;          // floats of their partials
+};
+
+bool fold_rank(int64_t r) { return r > 0 && r % 8 == 0 && r <= 32; }
+
+LoraPass plan_fwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold) {
+  LoraPass p;
+  const int rp = (int)round_up(r, 16);
+  p.G = (m + 63) / 64;
+  p.fs = (k + MID_FOLD_KT - 1) / MID_FOLD_KT;
+  p.fp = round_up(p.fs * p.G * 64 * rp, 64);
+  p.fold = may_fold && fold_rank(r) && fold_plan(m, n, k, false, PLAN_ANY, false, &p.g);
+  if (p.fold) {
+    p.ms = p.g.floats;
+    p.bytes = (size_t)(p.fp + p.ms) * 4;
+    return p;
+  }
+  gemm_plan(m, n, k, PLAN_ANY, &p.g);
+  p.bytes = lora_layout(nullptr, m, n, k, rp, false).bytes + (size_t)p.g.floats * 4;
+  return p;
+}
+
+// gemm: the pass has an input gradient
+LoraPass plan_bwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, bool gemm) {
+  LoraPass p;
+  const int rp = (int)round_up(r, 16);
+  const size_t lb = lora_layout(nullptr, m, n, k, rp, true).bytes;
+  p.G = (m + 63) / 64;
+  p.fs = (n + MID_FOLD_KT - 1) / MID_FOLD_KT;
+  p.fold = gemm && may_fold && fold_rank(r) && fold_plan(m, k, n, true, PLAN_ANY, false, &p.g);
+  if (!p.fold) {
+    if (gemm) gemm_plan(m, k, n, PLAN_ANY, &p.g);
+    p.bytes = lb + (size_t)p.g.floats * 4;
+    return p;
+  }
+  p.fp = round_up(p.fs * p.G * 64 * rp, 64);
+  p.ms = round_up(p.g.floats, 64);
+  // the weight gradients in token slices that fit the tiles' LDS, their
+  // counters after the fold's and the ranges'
+  const int lds = mid_tn_lds(p.g.v);
+  p.tpb = mid_tn_plan(m, n, k, rp, lds);
+  p.tpa = mid_tn_plan(m, k, n, rp, lds);
+  p.fold_tn = p.tpb.splits > 0 && p.tpa.splits > 0 &&
+              2 * p.G + p.g.tiles + TN_WAVES * (p.tpb.tiles + p.tpa.tiles) <= SK_MAX_NB;
+  p.tb = p.tpb.splits > 1 ? (int64_t)p.tpb.splits * n * rp : 0;
+  p.ta = p.tpa.splits > 1 ? (int64_t)p.tpa.splits * k * rp : 0;
+  p.bytes = lb + (size_t)(p.fp + p.ms + p.tb + p.ta) * 4;
+  return p;
+}
+
+// workspace bytes of the few-token kernels (m <= 16): the forward's; the
+// backward's, after u [m, rp]
+size_t few_fwd_bytes(int64_t m, int64_t n, int64_t k, int rp) {
+  return skinny_ws_bytes(skinny_plan(n, k, rp, get_num_cus()), m, n, rp);
+}
+size_t few_u_bytes(int64_t m, int rp) { return (size_t)round_up(m * rp * 2, 256); }
+size_t few_bwd_bytes(int64_t m, int64_t n, int64_t k, int rp) {
+  return few_u_bytes(m, rp) + skinny_ws_bytes(skinny_plan(k, n, rp, get_num_cus()), m, k, rp);
+}
+
+// Workspace of every call of up to m tokens at this rank.
+size_t reserve_bytes(int64_t m, int64_t n, int64_t k, int64_t r) {
+  const int64_t lr = r > 0 ? r : 16;
+  const int rp = (int)round_up(lr, 16);
+  size_t need = std::max(plan_fwd(m, n, k, lr, false).bytes, plan_bwd(m, n, k, lr, false, true).bytes);
+  // the fused GEMMs' split partials are not monotonic in the token count
+  // (fewer tiles, more depth ranges): their largest size over m' <= m, which
+  // peaks at a whole number of 64-token tiles
+  GemmPlan f, b;
+  gemm_plan(m, n, k, PLAN_ANY, &f);
+  gemm_plan(m, k, n, PLAN_ANY, &b);
+  const int64_t gp_m = std::max(f.floats, b.floats);
+  int64_t gp_max = gp_m;
+  for (int64_t mm = 64; mm < m; mm += 64) {
+    gemm_plan(mm, n, k, PLAN_ANY, &f);
+    gemm_plan(mm, k, n, PLAN_ANY, &b);
+    gp_max = std::max(gp_max, std::max(f.floats, b.floats));
+  }
+  need += (size_t)(gp_max - gp_m) * 4;
+  if (m >= 1) {
+    const int64_t mm = m < 16 ? m : 16;
+    need = std::max(need, std::max(few_fwd_bytes(mm, n, k, rp), few_bwd_bytes(mm, n, k, rp)));
+  }
+  if (fold_rank(r) && m > 16) {
+    // the one-launch mid-size passes, at every token count up to m
+    const size_t lb = lora_layout(nullptr, m, n, k, rp, true).bytes;
+    for (int64_t mm = 64;; mm += 64) {
+      const int64_t mt = mm < m ? mm : m;
+      const LoraPass p = plan_bwd(mt, n, k, r, true, true);
+      need = std::max(need, std::max(plan_fwd(mt, n, k, r, true).bytes, lb + (size_t)(p.fp + p.ms + p.tb + p.ta) * 4));
+      if (mt == m) break;
+    }
+  }
+  return std::max(need, (size_t)round_up(n * 4, 256));  // and the fp8 quantizer's row maxima
 }
 
 // Shape limit of the LoRA kernels: 32-bit buffer offsets over one slice.
@@ -442,6 +540,34 @@ int lrq_debug_gemm_path(int path) {
   return LRQ_OK;
 }
 
+int lrq_debug_plan(int pass, int64_t m, int64_t n, int64_t k, int64_t r, int64_t* out) {
+  if (pass < 0 || pass > 2 || m < 1 || n < 1 || k < 1 || r < 0 || r > 64 || !out) return LRQ_EINVAL;
+  for (int i = 0; i < 4; ++i) out[i] = 0;
+  out[4] = plans_formed();
+  if (pass == 2) {
+    out[0] = (int64_t)reserve_bytes(m, n, k, r);
+    return LRQ_OK;
+  }
+  const bool bwd = pass == 1;
+  const int rp = (int)round_up(r, 16);
+  if (m <= 16) {
+    out[0] = (int64_t)(bwd ? few_bwd_bytes(m, n, k, rp) : few_fwd_bytes(m, n, k, rp));
+    return LRQ_OK;
+  }
+  LoraPass p;
+  if (r > 0) {
+    p = bwd ? plan_bwd(m, n, k, r, true, true) : plan_fwd(m, n, k, r, true);
+  } else {
+    gemm_plan(m, bwd ? k : n, bwd ? n : k, PLAN_ANY, &p.g);
+    p.bytes = (size_t)p.g.floats * 4;
+  }
+  out[0] = (int64_t)p.bytes;
+  out[1] = p.g.v;
+  out[2] = p.g.S;
+  out[3] = p.fold;
+  return LRQ_OK;
+}
+
 int lrq_debug_force_wait_timeout(int on) {
   set_force_wait_timeout(on != 0);
   return LRQ_OK;
@@ -449,57 +575,10 @@ int lrq_debug_force_wait_timeout(int on) {
 
 const char* lrq_last_error(const lrq_ctx* c) { return c ? c->err : "null context"; }
 
-// Workspace floats of the mid-size passes at ranks 8 to 32 (multiples of 8)
-// that form the
-// LoRA factors in their own launch: the factor's slice partials, then the
-// tiles' depth-range partials, then (backward) dB's and dA's token-slice
-// partials (both jobs counted).
-static int64_t fold_fwd_floats(int64_t m, int64_t n, int64_t k, int rp) {
-  const int64_t G = (m + 63) / 64, fs = (k + MID_FOLD_KT - 1) / MID_FOLD_KT;
-  return round_up(fs * G * 64 * rp, 64) + mid_split_plan(m, n, k, SIDE_FWD).floats;
-}
-static int64_t fold_bwd_floats(int64_t m, int64_t n, int64_t k, int rp) {
-  const int64_t G = (m + 63) / 64, fs = (n + MID_FOLD_KT - 1) / MID_FOLD_KT;
-  const int lds = mid_tn_lds(m, k, n);
-  const LoraPlan tpb = mid_tn_plan(m, n, k, rp, lds), tpa = mid_tn_plan(m, k, n, rp, lds);
-  return round_up(fs * G * 64 * rp, 64) + round_up(mid_split_plan(m, k, n, SIDE_BWD).floats, 64) +
-         (tpb.splits > 1 ? (int64_t)tpb.splits * n * rp : 0) + (tpa.splits > 1 ? (int64_t)tpa.splits * k * rp : 0);
-}
-
 int lrq_reserve(lrq_ctx* c, int64_t m, int64_t n, int64_t k, int64_t r) {
   LRQ_TRY(begin(c));
   if (m < 0 || n < 0 || k < 0 || r < 0 || r > 64) return fail(c, LRQ_EINVAL, "bad reserve shape");
-  const int rp = (int)round_up(r > 0 ? r : 16, 16);
-  size_t need = lora_layout(nullptr, m, n, k, rp).bytes;
-  // the fused GEMMs' split partials are not monotonic in the token count
-  // (fewer tiles, more depth ranges): their largest size over m' <= m, which
-  // peaks at a whole number of 64-token tiles
-  const int64_t gp_m = gemm_part_floats(m, n, k);
-  int64_t gp_max = gp_m;
-  for (int64_t mm = 64; mm < m; mm += 64) gp_max = std::max(gp_max, gemm_part_floats(mm, n, k));
-  need += (size_t)(gp_max - gp_m) * 4;
-  if (m >= 1) {  // the few-token forward, at up to 16 tokens
-    const size_t sk = skinny_ws_bytes(skinny_plan(n, k, rp, get_num_cus()), m < 16 ? m : 16, n, rp);
-    if (sk > need) need = sk;
-    // the few-token input gradient: its partials (and u's) follow the LoRA workspace
-    const int64_t mm = m < 16 ? m : 16;
-    const size_t skd = lora_layout(nullptr, mm, n, k, rp).bytes +
-                       skinny_ws_bytes(skinny_plan(k, n, rp, get_num_cus()), mm, k, rp);
-    if (skd > need) need = skd;
-  }
-  if (r % 8 == 0 && r > 0 && r <= 32 && m > 16) {
-    // the one-launch mid-size passes, at every token count up to m
-    const size_t lb = lora_layout(nullptr, m, n, k, rp).bytes;
-    for (int64_t mm = 64;; mm += 64) {
-      const int64_t mt = mm < m ? mm : m;
-      need = std::max(need, (size_t)fold_fwd_floats(mt, n, k, rp) * 4);
-      need = std::max(need, lb + (size_t)fold_bwd_floats(mt, n, k, rp) * 4);
-      if (mt == m) break;
-    }
-  }
-  const size_t fp8_need = (size_t)round_up(n * 4, 256);
-  if (fp8_need > need) need = fp8_need;
-  return ensure_ws(c, need);
+  return ensure_ws(c, reserve_bytes(m, n, k, r));
 }
 
 int lrq_quantize_int4(lrq_ctx* c, const float* w, int64_t n, int64_t k, int64_t group,
@@ -681,6 +760,7 @@ static int fwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t 
   }
   char* ws = nullptr;
   uint32_t* cnt = nullptr;
+  GemmPlan plan;
   if (m >= 1 && m <= 16) {
     // few tokens: one launch streams the packed weight once (split-k
     // partials, t's partials alongside); the last arrival at each block row
@@ -704,23 +784,19 @@ static int fwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t 
   if (lora) {
     const int rp = (int)round_up(r, 16);
     LRQ_TRY(check_lora_shapes(c, m, w->n, w->k, rp));
-    // mid-size tiles at ranks 8 to 32 (multiples of 8): t is formed in the same launch by
-    // workgroups ahead of the tiles (no side launch)
-    const int64_t G = (m + 63) / 64, fs = (w->k + MID_FOLD_KT - 1) / MID_FOLD_KT;
-    // (and the tiles' depth ranges, if any: partials after t's, counters
-    // after the fold's)
-    const MidSplit ms = mid_split_plan(m, w->n, w->k, SIDE_FWD);
-    if (r % 8 == 0 && r <= 32 && gemm_mid_tokens(m, w->n, w->k, SIDE_FWD) > 0 && aligned16(a) && t_out && aligned16(t_out) &&
-        2 * G + ms.tiles <= SK_MAX_NB) {
-      const int64_t fp = round_up(fs * G * 64 * rp, 64);
-      LRQ_TRY(acquire_ws(c, src, (size_t)(fp + ms.floats) * 4, &ws, &cnt));
+    const LoraPass p = plan_fwd(m, w->n, w->k, r, aligned16(a) && t_out && aligned16(t_out));
+    plan = p.g;
+    LRQ_TRY(acquire_ws(c, src, p.bytes, &ws, &cnt));
+    if (p.fold) {
+      // t formed in the GEMM's launch (the tiles' range counters after the
+      // fold's)
       ga.fold = force_wait_timeout() ? -1 : 1;
-      ga.fold_slices = (int)fs;
-      ga.fold_wgs = (int)round_up(fs * G, 8);
+      ga.fold_slices = (int)p.fs;
+      ga.fold_wgs = (int)round_up(p.fs * p.G, 8);
       ga.fpart = reinterpret_cast<float*>(ws);
       ga.fcnt = cnt;
-      ga.part = ms.floats > 0 ? ga.fpart + fp : nullptr;
-      ga.mcnt = cnt + 2 * G;
+      ga.part = p.ms > 0 ? ga.fpart + p.fp : nullptr;
+      ga.mcnt = cnt + 2 * p.G;
       ga.lact = a;
       ga.lw = b;
       ga.fscale = scaling;
@@ -728,10 +804,9 @@ static int fwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t 
       ga.fout_ld = (int)r;
       ga.r = (int)r;
       ga.rp = rp;
-      return run_hot(c, KID_FWD_MAIN, "fwd_main", [=] { return launch_fwd(c->stream, fmt, ga); });
+      return run_hot(c, KID_FWD_MAIN, "fwd_main", [=] { return launch_fwd(c->stream, fmt, plan, ga); });
     }
-    LRQ_TRY(acquire_ws(c, src, lora_layout(nullptr, m, w->n, w->k, rp, true).bytes, &ws, &cnt));
-    LoraWs lw = lora_layout(ws, m, w->n, w->k, rp, true);
+    const LoraWs lw = lora_layout(ws, m, w->n, w->k, rp, false);
     // t = s . x . A   (bf16 [m, rp] for the fused step, [m, r] for the caller)
     const LoraPlan pt = lora_plan_nt(m, w->k, rp);
     // fp8: B^T divided by the weight scale (the GEMM scales base + LoRA)
@@ -746,17 +821,17 @@ static int fwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t 
     ga.lw = lw.fr;
     ga.r = (int)r;
     ga.rp = rp;
-    ga.part = lw.gp;
+    ga.part = reinterpret_cast<float*>(ws + lw.bytes);
     ga.mcnt = cnt;
   } else {
-    const int64_t pf = gemm_split_floats(m, w->n, w->k);
-    if (pf > 0) {
-      LRQ_TRY(acquire_ws(c, src, (size_t)pf * 4, &ws, &cnt));
+    gemm_plan(m, w->n, w->k, PLAN_ANY, &plan);
+    if (plan.floats > 0) {
+      LRQ_TRY(acquire_ws(c, src, (size_t)plan.floats * 4, &ws, &cnt));
       ga.part = reinterpret_cast<float*>(ws);
       ga.mcnt = cnt;
     }
   }
-  return run_hot(c, KID_FWD_MAIN, "fwd_main", [=] { return launch_fwd(c->stream, fmt, ga); });
+  return run_hot(c, KID_FWD_MAIN, "fwd_main", [=] { return launch_fwd(c->stream, fmt, plan, ga); });
 }
 
 int lrq_quant_matmul_t(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t m, uint16_t* y) {
@@ -795,23 +870,6 @@ int lrq_lora_fwd_noalloc(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int
   return rc;
 }
 
-// The input gradient: the few-token path for m <= 16 (partials at `skpart`),
-// else the fused GEMM.
-static hipError_t launch_dx(lrq_ctx* c, int fmt, int64_t wn, int64_t wk, const GemmArgs& ga, int64_t m,
-                            float* skpart) {
-  if (m >= 1 && m <= 16) {
-    const SkinnyPlan p = skinny_plan(wk, wn, 0, get_num_cus());
-    return launch_skinny(c->stream, fmt, true, ga, nullptr, p, skpart, nullptr, c->cnt, 1.0f, nullptr);
-  }
-  return launch_bwd(c->stream, fmt, ga);
-}
-
-// workspace bytes of the few-token input gradient's partials (0 for m > 16)
-static size_t skinny_dx_bytes(const lrq_weight* w, int64_t m) {
-  if (m < 1 || m > 16) return 0;
-  return skinny_ws_bytes(skinny_plan(w->k, w->n, 0, get_num_cus()), m, w->k, 0);
-}
-
 static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const uint16_t* dy, int64_t m,
                     const uint16_t* a, const uint16_t* b, int64_t r, float scaling, const uint16_t* t,
                     uint16_t* dx, float* da, float* db) {
@@ -825,6 +883,7 @@ static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const ui
   if (dx && !aligned16(dx)) return fail(c, LRQ_EINVAL, "dx must be 16-byte aligned");
   const bool lora = a != nullptr && b != nullptr && r > 0;
   GemmArgs ga = gemm_args(w, true, dy, m, dx);
+  GemmPlan plan;
   if (lora) {
     if (r > 64) return fail(c, LRQ_EINVAL, "rank %lld outside [1, 64]", (long long)r);
     if ((da && (!x || !aligned16(x))) || (db && !t))
@@ -832,41 +891,17 @@ static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const ui
     if (!aligned16(b)) return fail(c, LRQ_EINVAL, "B must be 16-byte aligned");
     const int rp = (int)round_up(r, 16);
     LRQ_TRY(check_lora_shapes(c, m, w->n, w->k, rp));
-    const bool few = dx && m >= 1 && m <= 16;
-    const SkinnyPlan sp = skinny_plan(w->k, w->n, rp, get_num_cus());
-    const size_t lbytes = lora_layout(nullptr, m, w->n, w->k, rp).bytes;
-    // mid-size tiles at ranks 8 to 32 (multiples of 8): u is formed in the input gradient's
-    // launch by workgroups ahead of the tiles (partials after the LoRA
-    // workspace)
-    const int64_t G = (m + 63) / 64, fs = (w->n + MID_FOLD_KT - 1) / MID_FOLD_KT;
-    const bool fold = !few && dx && r % 8 == 0 && r <= 32 && gemm_mid_tokens(m, w->k, w->n, SIDE_BWD) > 0 && aligned16(a) &&
-                      2 * G + mid_split_plan(m, w->k, w->n, SIDE_BWD).tiles <= SK_MAX_NB;
-    // and the weight gradients by workgroups after its tiles, in token
-    // slices that fit its LDS (their counters after the fold's, partials
-    // after u's)
-    const int tlds = mid_tn_lds(m, w->k, w->n);
-    const LoraPlan tpb = fold ? mid_tn_plan(m, w->n, w->k, rp, tlds) : LoraPlan{};
-    const LoraPlan tpa = fold ? mid_tn_plan(m, w->k, w->n, rp, tlds) : LoraPlan{};
-    const int64_t tb_floats = (db && tpb.splits > 1) ? (int64_t)tpb.splits * w->n * rp : 0;
-    const int64_t ta_floats = (da && tpa.splits > 1) ? (int64_t)tpa.splits * w->k * rp : 0;
-    // the tiles' depth ranges, if any (their partials and counters first)
-    const MidSplit ms = fold ? mid_split_plan(m, w->k, w->n, SIDE_BWD) : MidSplit{1, 0, 0, 0};
-    const bool fold_tn = fold && (da || db) && tpb.splits > 0 && tpa.splits > 0 &&
-                         2 * G + ms.tiles + TN_WAVES * ((db ? tpb.tiles : 0) + (da ? tpa.tiles : 0)) <= SK_MAX_NB;
-    const int64_t fp_floats = round_up(fs * G * 64 * rp, 64);
-    const int64_t ms_floats = round_up(ms.floats, 64);
-    const size_t fbytes = fold ? (size_t)(fp_floats + ms_floats + (fold_tn ? tb_floats + ta_floats : 0)) * 4 : 0;
-    LRQ_TRY(ensure_ws(c, lbytes + (few ? skinny_ws_bytes(sp, m, w->k, rp) : fbytes)));
-    LoraWs ws = lora_layout(c->ws, m, w->n, w->k, rp);
     ga.r = (int)r;
     ga.rp = rp;
-    if (few) {
+    if (dx && m >= 1 && m <= 16) {
       // few tokens: u = s . dy . B^T (bf16 [m, rp], dA's factor) comes out
       // of the input gradient's own launch, as t does in the forward
-      float* part = reinterpret_cast<float*>(c->ws + lbytes);
+      const SkinnyPlan sp = skinny_plan(w->k, w->n, rp, get_num_cus());
+      LRQ_TRY(ensure_ws(c, few_bwd_bytes(m, w->n, w->k, rp)));
+      uint16_t* up = reinterpret_cast<uint16_t*>(c->ws);
+      float* part = reinterpret_cast<float*>(c->ws + few_u_bytes(m, rp));
       float* tpart = part + round_up((int64_t)sp.S * m * w->k, 64);
       ga.lw = a;
-      uint16_t* up = ws.up;
       // and dA = x^T . u, dB = t^T . dy in the same launch: dB by the split
       // workgroups (nothing to wait for), dA by each block row's epilogue
       // once u is in
@@ -875,52 +910,58 @@ static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const ui
         return launch_skinny(c->stream, fmt, true, ga, b, sp, part, tpart, c->cnt, scaling, up, gr);
       }));
       return LRQ_OK;
-    } else if (fold) {
-      // u (stored to the workspace for dA) from the fold's workgroups
+    }
+    const LoraPass p = plan_bwd(m, w->n, w->k, r, aligned16(a), dx != nullptr);
+    plan = p.g;
+    LRQ_TRY(ensure_ws(c, p.bytes));
+    const LoraWs ws = lora_layout(c->ws, m, w->n, w->k, rp, true);
+    float* const tail = reinterpret_cast<float*>(c->ws + ws.bytes);
+    if (p.fold) {
+      // u (stored to the workspace for dA) formed in the input gradient's
+      // launch
       ga.fold = force_wait_timeout() ? -1 : 1;
-      ga.fold_slices = (int)fs;
-      ga.fold_wgs = (int)round_up(fs * G, 8);
-      ga.fpart = reinterpret_cast<float*>(c->ws + lbytes);
+      ga.fold_slices = (int)p.fs;
+      ga.fold_wgs = (int)round_up(p.fs * p.G, 8);
+      ga.fpart = tail;
       ga.fcnt = c->cnt;
       ga.lact = b;
       ga.lw = a;
       ga.fscale = scaling;
-      ga.fout = ws.up;
+      ga.fout = ws.tp;
       ga.fout_ld = rp;
-      ga.part = ms.floats > 0 ? ga.fpart + fp_floats : nullptr;
-      ga.mcnt = c->cnt + 2 * G;
-      if (fold_tn) {
+      ga.part = p.ms > 0 ? tail + p.fp : nullptr;
+      ga.mcnt = c->cnt + 2 * p.G;
+      if (p.fold_tn && (da || db)) {
         // dB = t^T . dy first (nothing to wait for), then dA = x^T . u
-        float* tpart = ga.fpart + fp_floats + ms_floats;
-        uint32_t* tcnt = c->cnt + 2 * G + ms.tiles;
+        float* const tpart = tail + p.fp + p.ms;
+        uint32_t* tcnt = c->cnt + 2 * p.G + p.g.tiles;
         int nj = 0;
         if (db) {
-          ga.tj[nj++] = tn_args(TnSpec{dy, t, r, m, w->n, (int)r, tpb, tpart, db, 1, w->n}, tcnt);
-          tpart += tb_floats;
-          tcnt += TN_WAVES * tpb.tiles;
+          ga.tj[nj++] = tn_args(TnSpec{dy, t, r, m, w->n, (int)r, p.tpb, tpart, db, 1, w->n}, tcnt);
+          tcnt += TN_WAVES * p.tpb.tiles;
         }
         if (da) {
           ga.tn_da = nj;
-          ga.tj[nj++] = tn_args(TnSpec{x, ws.up, rp, m, w->k, (int)r, tpa, tpart, da, r, 1}, tcnt);
+          ga.tj[nj++] = tn_args(TnSpec{x, ws.tp, rp, m, w->k, (int)r, p.tpa, tpart + p.tb, da, r, 1}, tcnt);
         }
         ga.tn_blocks = ga.tj[0].blocks + ga.tj[1].blocks;
       }
-      LRQ_TRY(run_hot(c, KID_BWD_DX, "bwd_dx", [=] { return launch_bwd(c->stream, fmt, ga); }));
-      if (fold_tn) return LRQ_OK;
+      LRQ_TRY(run_hot(c, KID_BWD_DX, "bwd_dx", [=] { return launch_bwd(c->stream, fmt, plan, ga); }));
+      if (p.fold_tn) return LRQ_OK;
     } else {
       // u = s . dy . B^T   (bf16 [m, rp]: the dx epilogue operand and dA's factor)
       const LoraPlan pu = lora_plan_nt(m, w->n, rp);
       const LoraWs wsv = ws;
       LRQ_TRY(run_hot(c, KID_LORA_U, "lora_u", [=] {
         // and A [k, r] padded to [k, rp]: the dx GEMM's weight-side LoRA rows
-        const NtFinish fin{c->cnt, scaling, (int)r, wsv.up, nullptr, a, wk, 1, wsv.fr, nullptr, 0};
+        const NtFinish fin{c->cnt, scaling, (int)r, wsv.tp, nullptr, a, wk, 1, wsv.fr, nullptr, 0};
         return launch_lora_nt(c->stream, dy, b, true, wn, (int)r, m, wn, rp, pu, wsv.pn, fin);
       }));
-      ga.lact = ws.up;
+      ga.lact = ws.tp;
       ga.lw = ws.fr;
-      ga.part = ws.gp;
+      ga.part = tail;
       ga.mcnt = c->cnt;
-      if (dx) LRQ_TRY(run_hot(c, KID_BWD_DX, "bwd_dx", [=] { return launch_bwd(c->stream, fmt, ga); }));
+      if (dx) LRQ_TRY(run_hot(c, KID_BWD_DX, "bwd_dx", [=] { return launch_bwd(c->stream, fmt, plan, ga); }));
     }
     // dA = x^T . u -> f32 [k, r] and dB = t^T . dy -> f32 [r, n]: token-slice
     // partials of both in one launch (dB's longer workgroups dispatched
@@ -931,7 +972,7 @@ static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const ui
     // alone, so the partials reserved for the single-job plans suffice)
     const int64_t ob = da ? w->k : 0, oa = db ? w->n : 0;
     if (db) specs[nj++] = TnSpec{dy, t, r, m, w->n, (int)r, lora_plan_tn(m, w->n, rp, ob), ws.pb, db, 1, w->n};
-    if (da) specs[nj++] = TnSpec{x, ws.up, rp, m, w->k, (int)r, lora_plan_tn(m, w->k, rp, oa), ws.pa, da, r, 1};
+    if (da) specs[nj++] = TnSpec{x, ws.tp, rp, m, w->k, (int)r, lora_plan_tn(m, w->k, rp, oa), ws.pa, da, r, 1};
     if (nj) {
       const int kid = nj == 2 ? KID_LORA_DADB : (db ? KID_LORA_DB : KID_LORA_DA);
       const TnSpec s0 = specs[0], s1 = specs[1];
@@ -943,14 +984,21 @@ static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const ui
     return LRQ_OK;
   }
   if (!dx) return LRQ_OK;
-  const int64_t pf = (m >= 1 && m <= 16) ? 0 : gemm_split_floats(m, w->k, w->n);
-  LRQ_TRY(ensure_ws(c, std::max((size_t)pf * 4, skinny_dx_bytes(w, m))));
-  if (pf > 0) {
+  if (m >= 1 && m <= 16) {
+    const SkinnyPlan sp = skinny_plan(wk, wn, 0, get_num_cus());
+    LRQ_TRY(ensure_ws(c, skinny_ws_bytes(sp, m, wk, 0)));
+    float* part = reinterpret_cast<float*>(c->ws);
+    return run_hot(c, KID_BWD_DX, "bwd_dx", [=] {
+      return launch_skinny(c->stream, fmt, true, ga, nullptr, sp, part, nullptr, c->cnt, 1.0f, nullptr);
+    });
+  }
+  gemm_plan(m, wk, wn, PLAN_ANY, &plan);
+  LRQ_TRY(ensure_ws(c, (size_t)plan.floats * 4));
+  if (plan.floats > 0) {
     ga.part = reinterpret_cast<float*>(c->ws);
     ga.mcnt = c->cnt;
   }
-  float* skpart = reinterpret_cast<float*>(c->ws);
-  return run_hot(c, KID_BWD_DX, "bwd_dx", [=] { return launch_dx(c, fmt, wn, wk, ga, m, skpart); });
+  return run_hot(c, KID_BWD_DX, "bwd_dx", [=] { return launch_bwd(c->stream, fmt, plan, ga); });
 }
 
 int lrq_quant_matmul_t_bwd(lrq_ctx* c, const lrq_weight* w, const uint16_t* dy, int64_t m, uint16_t* dx) {

@@ -87,6 +87,7 @@
 //     partials in range order, applies the forward fp8 scales and bias and
 //     rounds once to bf16.
 
+#include <atomic>
 #include <type_traits>
 
 #include "lrq_common.h"
@@ -780,12 +781,18 @@ hipError_t run_fmt(hipStream_t st, int fmt, bool r192, const GemmArgs& a) {
 //   - a tile may split its depth into ranges (one workgroup each, whole
 //     rounds of stages) when the tiles leave CUs idle; the ranges'
 //     accumulators meet in the launch, and S > 1 must model a tenth faster;
-//   - `side`: what forming the LoRA factors beside the product adds. The
+//   - what forming the LoRA factors adds (large_side_us, w8_side_us). The
 //     large tiles need a launch for t, or for u and for dA and dB (8 and 20
 //     us plus their streams at 6 TB/s); the others form them in their own
 //     launch: the factor slices' workgroups hold up tiles, and weight-gradient
 //     blocks beyond half a round of workgroups follow the tiles (4096 tokens,
 //     3072 -> 12288, rank 32: 100 us, where 1999 tokens, 2560 -> 4096 add 4).
+//     A call that gives up the folded plan for those launches takes the
+//     kernel that is fastest without the factors, the large tiles or not.
+// Decided on whole 64-token groups, so that a workspace reserved for the
+// largest of a group's token counts serves them all. A plan keeps the limits
+// of the call (its workspace, the counter area) and of the launch (32-bit
+// buffer offsets).
 constexpr double LARGE_STEP_US = 1.75;
 // per variant MID_64, MID_128, MID_256: tile tokens and rows, a fixed cost
 // per round of tiles, 64-deep blocks per pipeline stage, stages a depth range
@@ -808,20 +815,30 @@ int g_gemm_path = 0;
 // microseconds that a product's bytes take beside a launch's fixed cost
 double stream_us(double bytes) { return bytes / 6.0e6; }
 
-double large_us(int64_t m, int64_t e, int64_t depth, int side) {
-  const SplitPlan p = plan_split(m, e, depth);
+double large_us(int64_t m, int64_t e, int64_t depth, const SplitPlan& p) {
   const int64_t cus = get_num_cus();
   const int64_t RA = p.r192 ? 192 : 256;
   const int64_t tiles = (m + RB - 1) / RB * ((e + RA - 1) / RA);
   const double f = p.r192 ? 0.8 : 1.0;
-  const double act = 2.0 * (double)m * (double)depth;
-  const double extra = side == SIDE_FWD ? 8.0 + stream_us(act)
-                       : side == SIDE_BWD ? 20.0 + stream_us(2.0 * act + 2.0 * (double)m * (double)e)
-                                          : 0.0;
-  if (p.S <= 1)
-    return (double)((tiles + cus - 1) / cus) * (double)((depth + 63) / 64) * LARGE_STEP_US * f + 3.0 + extra;
+  if (p.S <= 1) return (double)((tiles + cus - 1) / cus) * (double)((depth + 63) / 64) * LARGE_STEP_US * f + 3.0;
   const double part = 4.0 * (double)p.S * (double)m * (double)e;
-  return (double)p.spl * LARGE_STEP_US * f + 2.0 * part / 4.0e6 + 8.0 + extra;
+  return (double)p.spl * LARGE_STEP_US * f + 2.0 * part / 4.0e6 + 8.0;
+}
+
+double large_side_us(int64_t m, int64_t e, int64_t depth, bool bwd) {
+  const double act = 2.0 * (double)m * (double)depth;
+  return bwd ? 20.0 + stream_us(2.0 * act + 2.0 * (double)m * (double)e) : 8.0 + stream_us(act);
+}
+
+double w8_side_us(int64_t m, int64_t e, int64_t depth, bool bwd) {
+  const double slots = 2.0 * (double)get_num_cus();
+  // factor slices, two a workgroup, about 10 us a round with what they hold up
+  double us = 10.0 * (double)((m + 63) / 64 * ((depth + MID_FOLD_KT - 1) / MID_FOLD_KT)) / slots;
+  if (bwd) {
+    const LoraPlan pa = mid_tn_plan(m, e, depth, 32, W8_TN_LDS), pb = mid_tn_plan(m, depth, e, 32, W8_TN_LDS);
+    us += 45.0 * std::max(0.0, (double)(pa.tiles * pa.splits + pb.tiles * pb.splits) / slots - 0.5);
+  }
+  return us;
 }
 
 // stages per range (whole rounds) for S ranges of a depth, and the ranges
@@ -836,22 +853,18 @@ int mid_ranges(int64_t depth, int v, int S) {
   return (int)((nst + spl - 1) / spl);
 }
 
-double mid_us(int64_t m, int64_t e, int64_t depth, int side, int v, int S = 1) {
-  const int64_t T = MID_T[v], cus = get_num_cus();
-  const int64_t tiles = (m + T - 1) / T * ((e + MID_R[v] - 1) / MID_R[v]) * S;
-  const int64_t n = (tiles + cus - 1) / cus;
+int64_t mid_tiles(int64_t m, int64_t e, int v) { return (m + MID_T[v] - 1) / MID_T[v] * ((e + MID_R[v] - 1) / MID_R[v]); }
+
+// the product alone in S ranges
+double mid_us(int64_t m, int64_t e, int64_t depth, int v, int S) {
+  const int64_t cus = get_num_cus(), units = mid_tiles(m, e, v) * S;
+  const int64_t n = (units + cus - 1) / cus;
   if (v != MID_64) {
     const int64_t nst = ((depth + 63) / 64 + MID_SD[v] - 1) / MID_SD[v];
-    const double part = S > 1 ? W8_FINISH_US + 0.5 * S + 0.75 * stream_us(2.0 * 4.0 * (double)(tiles * T * MID_R[v])) : 0.0;
-    const double stage = W8_STAGE_US + W8_STAGE_FULL_US * std::min(1.0, (double)tiles / (double)cus);
-    double extra = 0.0;
-    if (side != SIDE_NONE)  // factor slices, two a workgroup, about 10 us a round with what they hold up
-      extra = 10.0 * (double)((m + 63) / 64 * ((depth + MID_FOLD_KT - 1) / MID_FOLD_KT)) / (2.0 * (double)cus);
-    if (side == SIDE_BWD) {
-      const LoraPlan pa = mid_tn_plan(m, e, depth, 32, W8_TN_LDS), pb = mid_tn_plan(m, depth, e, 32, W8_TN_LDS);
-      extra += 45.0 * std::max(0.0, (double)(pa.tiles * pa.splits + pb.tiles * pb.splits) / (2.0 * (double)cus) - 0.5);
-    }
-    return (double)n * ((double)(S > 1 ? mid_spl(depth, v, S) : nst) * stage + MID_FIX[v]) + part + extra;
+    const double part =
+        S > 1 ? W8_FINISH_US + 0.5 * S + 0.75 * stream_us(2.0 * 4.0 * (double)(units * MID_T[v] * MID_R[v])) : 0.0;
+    const double stage = W8_STAGE_US + W8_STAGE_FULL_US * std::min(1.0, (double)units / (double)cus);
+    return (double)n * ((double)(S > 1 ? mid_spl(depth, v, S) : nst) * stage + MID_FIX[v]) + part;
   }
   const int64_t nb = S > 1 ? std::min<int64_t>((int64_t)mid_spl(depth, v, S) * MID_SD[v], (depth + 63) / 64)
                            : (depth + 63) / 64;
@@ -859,60 +872,59 @@ double mid_us(int64_t m, int64_t e, int64_t depth, int side, int v, int S = 1) {
          MID_FIX[v] + MID_ROUND_US * (double)((n + 1) / 2 - 1) + (S > 1 ? MID_FINISH_US : 0.0);
 }
 
-struct MidChoice {
-  int v, S, spl;
+struct Pick {
+  GemmPlan p;
   double us;
 };
 
-// the best number of depth ranges for variant v (forced: at least two
-// where the depth has them)
-MidChoice mid_best_split(int64_t m, int64_t e, int64_t depth, int side, int v, bool force_split) {
-  MidChoice best{v, 1, 0, mid_us(m, e, depth, side, v, 1)};
-  MidChoice alt{v, 1, 0, 1e30};
-  for (int S = 2; S <= MID_MAXS[v]; ++S) {
-    const int R = mid_ranges(depth, v, S);
-    if (R < 2 || R != S) continue;  // (S that rounding turns into fewer ranges are covered by those)
-    const double t = mid_us(m, e, depth, side, v, S);
-    if (t < alt.us) alt = MidChoice{v, S, mid_spl(depth, v, S), t};
+// the best number of depth ranges for variant v, its partials and counters
+// within the limits (forced: at least two where the depth has them). False
+// if the launch cannot take the shape.
+bool mid_best(int64_t m, int64_t e, int64_t depth, int v, double side_us, bool force_split, int64_t max_floats,
+              int64_t max_tiles, Pick* out) {
+  // 32-bit buffer offsets of a tile's activation rows, outputs and weight rows
+  if ((int64_t)128 * depth * 2 >= ((int64_t)1 << 31) || (int64_t)128 * e * 2 >= ((int64_t)1 << 31)) return false;
+  if (max_floats < 0) return false;
+  const int64_t tiles = mid_tiles(m, e, v);
+  GemmPlan p;
+  p.v = v;
+  Pick best{p, mid_us(m, e, depth, v, 1) + side_us}, alt{p, 1e30};
+  for (int S = 2; S <= MID_MAXS[v] && tiles <= max_tiles; ++S) {
+    const int64_t floats = S * tiles * MID_T[v] * MID_R[v];
+    if (floats > max_floats || floats * 4 >= ((int64_t)1 << 32)) break;
+    if (mid_ranges(depth, v, S) != S) continue;  // (rounding turns it into fewer ranges, covered by those)
+    const double us = mid_us(m, e, depth, v, S) + side_us;
+    if (us >= alt.us) continue;
+    p.S = S;
+    p.spl = mid_spl(depth, v, S);
+    p.tiles = tiles;
+    p.floats = floats;
+    alt = Pick{p, us};
   }
-  if (alt.S > 1 && (force_split || alt.us < 0.9 * best.us)) return alt;
-  return best;
+  *out = alt.p.S > 1 && (force_split || alt.us < 0.9 * best.us) ? alt : best;
+  return true;
 }
 
-// the mid variant and its depth ranges a shape takes (v = MID_NONE: the
-// large tiles). Decided on whole 64-token groups, so that a workspace
-// reserved for the largest of a group's token counts serves them all.
-MidChoice mid_choice(int64_t m, int64_t e, int64_t depth, int side) {
-  const MidChoice none{MID_NONE, 1, 0, 0.0};
-  if (m <= 0 || e <= 0 || g_gemm_path == 1) return none;
-  m = (m + 63) / 64 * 64;
-  if (g_gemm_path >= 6) return mid_best_split(m, e, depth, side, MID_256, g_gemm_path == 7);
-  if (g_gemm_path >= 2) return mid_best_split(m, e, depth, side, (g_gemm_path - 2) % 2 + 1, g_gemm_path >= 4);
-  MidChoice pick = none;
-  pick.us = large_us(m, e, depth, side);
-  for (int v : {MID_64, MID_128, MID_256}) {
-    const MidChoice c = mid_best_split(m, e, depth, side, v, false);
-    if (c.us < pick.us) pick = c;
-  }
-  return pick;
+// the variant that lrq_debug_gemm_path forces (MID_NONE: none), and whether
+// with at least two depth ranges
+int forced_variant(bool* split) {
+  *split = g_gemm_path == 4 || g_gemm_path == 5 || g_gemm_path == 7;
+  return g_gemm_path >= 6 ? MID_256 : g_gemm_path >= 2 ? (g_gemm_path - 2) % 2 + 1 : MID_NONE;
 }
 
-// MID_NONE (the large tiles) or the mid variant a shape takes
-int mid_plan(int64_t m, int64_t e, int64_t depth, int side) { return mid_choice(m, e, depth, side).v; }
+std::atomic<int64_t> g_plans{0};
 
 template <bool BWD>
-hipError_t dispatch(hipStream_t st, int fmt, const GemmArgs& a) {
+hipError_t dispatch(hipStream_t st, int fmt, const GemmPlan& p, const GemmArgs& a) {
   if (a.m == 0 || a.e == 0) return hipSuccess;
-  const MidChoice mc = mid_choice(a.m, a.e, a.l, a.fold ? (BWD ? SIDE_BWD : SIDE_FWD) : SIDE_NONE);
-  if (mc.v != MID_NONE) {
-    if (mc.S <= 1) return launch_mid(st, fmt, BWD, a, mc.v);
+  if (p.v != MID_NONE) {
+    if (p.S <= 1) return launch_mid(st, fmt, BWD, a, p.v);
     if (!a.part || !a.mcnt) return hipErrorInvalidValue;
     GemmArgs b = a;
-    b.msplit = mc.S;
-    b.mspl = mc.spl;
-    return launch_mid(st, fmt, BWD, b, mc.v);
+    b.msplit = p.S;
+    b.mspl = p.spl;
+    return launch_mid(st, fmt, BWD, b, p.v);
   }
-  const SplitPlan p = plan_split(a.m, a.e, a.l);
   if (p.S <= 1) return run_fmt<BWD, false>(st, fmt, p.r192, a);
   if (!a.part) return hipErrorInvalidValue;
   GemmArgs b = a;
@@ -934,23 +946,63 @@ int g_num_cus_ = 256;  // compute units of the context's device (the persistent 
 void set_num_cus(int n) { g_num_cus_ = n > 0 ? n : 256; }
 int get_num_cus() { return g_num_cus_; }
 
-hipError_t launch_fwd(hipStream_t st, int fmt, const GemmArgs& a) { return dispatch<false>(st, fmt, a); }
-MidSplit mid_split_plan(int64_t m, int64_t e, int64_t depth, int side) {
-  const MidChoice mc = mid_choice(m, e, depth, side);
-  if (mc.v == MID_NONE || mc.S <= 1) return MidSplit{1, 0, 0, 0};
-  const int64_t T = MID_T[mc.v], R = MID_R[mc.v], tiles = (m + T - 1) / T * ((e + R - 1) / R);
-  return MidSplit{mc.S, mc.spl, tiles, (int64_t)mc.S * tiles * T * R};
+bool gemm_plan(int64_t m, int64_t e, int64_t depth, int64_t max_floats, GemmPlan* p) {
+  *p = GemmPlan{};
+  if (m <= 0 || e <= 0) return true;
+  g_plans.fetch_add(1, std::memory_order_relaxed);
+  const int64_t mg = (m + 63) / 64 * 64;
+  bool split = false;
+  const int fv = forced_variant(&split);
+  Pick pick{GemmPlan{}, 1e30}, c;
+  if (fv != MID_NONE && mid_best(mg, e, depth, fv, 0.0, split, max_floats, SK_MAX_NB, &c)) {
+    *p = c.p;
+    return true;
+  }
+  const SplitPlan sp = plan_split(m, e, depth);
+  const int64_t floats = sp.S > 1 ? (int64_t)sp.S * m * e : 0;
+  const bool large = floats <= max_floats;
+  if (large) {
+    pick.p.r192 = sp.r192;
+    pick.p.S = sp.S;
+    pick.p.spl = sp.spl;
+    pick.p.floats = floats;
+    pick.us = large_us(mg, e, depth, plan_split(mg, e, depth));
+  }
+  bool found = large;
+  if (g_gemm_path == 0)
+    for (int v : {MID_64, MID_128, MID_256})
+      if (mid_best(mg, e, depth, v, 0.0, false, max_floats, SK_MAX_NB, &c) && c.us < pick.us) {
+        pick = c;
+        found = true;
+      }
+  *p = pick.p;
+  return found;
 }
 
-int64_t gemm_split_floats(int64_t m, int64_t e, int64_t depth) {
-  if (m <= 0 || e <= 0) return 0;
-  if (mid_plan(m, e, depth, SIDE_NONE)) return mid_split_plan(m, e, depth, SIDE_NONE).floats;  // the mid tiles' depth ranges
-  const SplitPlan p = plan_split(m, e, depth);
-  return p.S > 1 ? (int64_t)p.S * m * e : 0;
+bool fold_plan(int64_t m, int64_t e, int64_t depth, bool bwd, int64_t max_floats, bool always, GemmPlan* p) {
+  *p = GemmPlan{};
+  const int64_t G = (m + 63) / 64, mg = G * 64;
+  if (m <= 0 || e <= 0 || g_gemm_path == 1) return false;
+  // the groups' arrivals and flags have counters
+  if (2 * G > SK_MAX_NB) return false;
+  g_plans.fetch_add(1, std::memory_order_relaxed);
+  bool split = false;
+  const int fv = forced_variant(&split);
+  const double w8 = w8_side_us(mg, e, depth, bwd);
+  Pick pick{GemmPlan{}, 1e30}, c;
+  if (fv == MID_NONE && !always)
+    pick.us = large_us(mg, e, depth, plan_split(mg, e, depth)) + large_side_us(mg, e, depth, bwd);
+  for (int v : {MID_64, MID_128, MID_256}) {
+    if (fv != MID_NONE && v != fv) continue;
+    if (mid_best(mg, e, depth, v, v == MID_64 ? 0.0 : w8, split, max_floats, SK_MAX_NB - 2 * G, &c) && c.us < pick.us)
+      pick = c;
+  }
+  *p = pick.p;
+  return pick.p.v != MID_NONE;
 }
-hipError_t launch_bwd(hipStream_t st, int fmt, const GemmArgs& a) { return dispatch<true>(st, fmt, a); }
-int mid_tn_lds(int64_t m, int64_t e, int64_t depth) {
-  return mid_plan(m, e, depth, SIDE_BWD) == MID_64 ? MID_TN_LDS : W8_TN_LDS;
-}
-int gemm_mid_tokens(int64_t m, int64_t e, int64_t depth, int side) { return MID_T[mid_plan(m, e, depth, side)]; }
+
+int64_t plans_formed() { return g_plans.load(std::memory_order_relaxed); }
+
+hipError_t launch_fwd(hipStream_t st, int fmt, const GemmPlan& p, const GemmArgs& a) { return dispatch<false>(st, fmt, p, a); }
+hipError_t launch_bwd(hipStream_t st, int fmt, const GemmPlan& p, const GemmArgs& a) { return dispatch<true>(st, fmt, p, a); }
 void set_gemm_path(int path) { g_gemm_path = path; }

@@ -62,7 +62,7 @@ struct GemmArgs {
   const uint16_t* lw;    // the weight-side LoRA factor (user layout)
   int r, rp;             // rank and rank padded to 16 (rp == 0: no LoRA)
   uint16_t* out;         // [m, e]
-  float* part;           // lrq_gemm.hip split-depth partials [S][m][e] (gemm_split_floats), or null
+  float* part;           // depth ranges' partials: lrq_gemm.hip [S][m][e]; the mid-size tiles' own layout; or null
   int splits, spl;       // set by lrq_gemm.hip: depth ranges and steps per range
   // lrq_gemm_mid.hip with the token-side LoRA factor formed in the same
   // launch (fold != 0, rank 8 to 32, a multiple of 8): the first fold_wgs workgroups (a
@@ -97,29 +97,40 @@ struct GemmArgs {
   uint32_t* mcnt;
 };
 
-// lrq_gemm.hip: the forward for m > 16 and the input gradient, weight
-// dequantized into registers. a.lw is the weight-side LoRA rows [e, rp]
-// (B^T forward, A backward; zero-padded columns), a.lact is t or u [m, rp].
-// The backward's a.wdata / a.wscale point at the transposed section.
-// With fewer output tiles than CUs the depth is split into S ranges whose
-// f32 partials a.part must hold: gemm_split_floats(m, e, depth) floats (0
-// when the shape is not split).
-hipError_t launch_fwd(hipStream_t st, int fmt, const GemmArgs& a);
-hipError_t launch_bwd(hipStream_t st, int fmt, const GemmArgs& a);
-int64_t gemm_split_floats(int64_t m, int64_t e, int64_t depth);
-int get_num_cus();
-// lrq_gemm_mid.hip (64-row x 64-token tiles, MID_64) and lrq_gemm_w8.hip
-// (128-token tiles of 128 or 256 rows, MID_128 and MID_256): the same
-// products over the whole depth or a few depth ranges finished in the
-// launch; lrq_gemm.hip's launchers take one when it is modelled faster
-// (gemm_mid_tokens: its tile's tokens, or 0). `side` says which LoRA factors
-// the launch would form too (SIDE_*: t; u, dA and dB; none, or they have
-// launches of their own): a call plans, reserves and launches with the same.
-// With depth ranges the caller provides a.part (gemm_split_floats without,
-// mid_split_plan(...).floats with such factors) and a.mcnt
-// (mid_split_plan(...).tiles counters).
-enum { SIDE_NONE = 0, SIDE_FWD = 1, SIDE_BWD = 2 };
+// How a fused product (m tokens, e outputs, `depth`) runs. A call forms its
+// plan once and sizes its workspace and launches from it; lrq_reserve forms
+// the same plans.
 enum { MID_NONE = 0, MID_64 = 1, MID_128 = 2, MID_256 = 3 };
+struct GemmPlan {
+  int v = MID_NONE;    // lrq_gemm_mid.hip (64-row x 64-token tiles, MID_64), lrq_gemm_w8.hip (128-token
+                       // tiles of 128 or 256 rows, MID_128 and MID_256), or the 256-token tiles
+  bool r192 = false;   // 256-token tiles: of 192 rows instead of 256
+  int S = 1, spl = 0;  // depth ranges (1: the whole depth), and steps or stages in each
+  int64_t tiles = 0;   // arrival counters that the ranges of a MID_* plan need
+  int64_t floats = 0;  // f32 partials that the ranges need
+};
+constexpr int64_t PLAN_ANY = INT64_MAX;
+// The product by itself, or with its LoRA factors from launches of their own:
+// the kernel modelled fastest of those whose partials fit max_floats. False
+// if none does.
+bool gemm_plan(int64_t m, int64_t e, int64_t depth, int64_t max_floats, GemmPlan* p);
+// The product and its LoRA factors (t; backward u, dA and dB) in one
+// launch: the fastest such kernel within max_floats. False if none is
+// modelled faster than the 256-token tiles and their side launches (`always`:
+// if there is none).
+bool fold_plan(int64_t m, int64_t e, int64_t depth, bool bwd, int64_t max_floats, bool always, GemmPlan* p);
+// cost-model evaluations of this process (lrq_debug_plan)
+int64_t plans_formed();
+
+// lrq_gemm.hip: the forward for m > 16 and the input gradient, weight
+// dequantized into registers, on the kernel of plan `p`. a.lw is the
+// weight-side LoRA rows [e, rp] (B^T forward, A backward; zero-padded
+// columns), a.lact is t or u [m, rp] (a folded plan: see GemmArgs.fold). The
+// backward's a.wdata / a.wscale point at the transposed section. With depth
+// ranges a.part holds p.floats floats and a.mcnt p.tiles counters.
+hipError_t launch_fwd(hipStream_t st, int fmt, const GemmPlan& p, const GemmArgs& a);
+hipError_t launch_bwd(hipStream_t st, int fmt, const GemmPlan& p, const GemmArgs& a);
+int get_num_cus();
 constexpr int MID_MAX_SPLIT = 4;  // depth ranges of a MID_64 tile
 constexpr int MID_MST = 4;  // MID_64: the kernel's pipeline stages (a range is whole rounds of them)
 // lrq_gemm_w8.hip: tiles of 128 tokens x 128 (MID_128) or 256 rows (MID_256),
@@ -127,25 +138,15 @@ constexpr int MID_MST = 4;  // MID_64: the kernel's pipeline stages (a range is 
 constexpr int W8_TOKENS = 128;
 constexpr int W8_MAX_SPLIT = 8;  // depth ranges of a tile
 hipError_t launch_w8(hipStream_t st, int fmt, bool bwd, const struct GemmArgs& a, int rows);
-// The mid-size tiles' depth ranges for a product (m tokens, e outputs,
-// `depth`): S = 1 (whole depth) when the large tiles or one range per tile
-// are modelled faster; tiles and the partial floats the ranges need.
-struct MidSplit {
-  int S, spl;
-  int64_t tiles, floats;
-};
-MidSplit mid_split_plan(int64_t m, int64_t e, int64_t depth, int side);
 hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int variant);
-int gemm_mid_tokens(int64_t m, int64_t e, int64_t depth, int side);
 // depth per slice of the folded factor's workgroups (GemmArgs.fold)
 constexpr int MID_FOLD_KT = 384;
 // the token slices of a weight-gradient job run inside the mid-size
 // backward: the factor slice takes at most 16 KiB of LDS (ranks padded to 16 or 32)
 constexpr int MID_TN_LDS = 16384;
 constexpr int W8_TN_LDS = 36864;  // in lrq_gemm_w8.hip
-int mid_tn_lds(int64_t m, int64_t e, int64_t depth);  // of the variant an input gradient takes
-// tuning and test hook (lrq_debug_gemm_path): 0 planned, 1 large tiles,
-// 2 MID_64, 3 MID_128
+inline int mid_tn_lds(int v) { return v == MID_64 ? MID_TN_LDS : W8_TN_LDS; }
+// tuning and test hook: the values of lrq_debug_gemm_path
 void set_gemm_path(int path);
 
 // lrq_skinny.hip: the forward for m <= 16 in one launch. Split workgroups

@@ -374,6 +374,16 @@ def debug_force_wait_timeout(on: bool):
     L.load().lrq_debug_force_wait_timeout(int(on))
 
 
+def debug_plan(what: str, m: int, n: int, k: int, r: int) -> dict:
+    """Test hook, host only: how a "fwd" or "bwd" call would run, or what
+    "reserve" takes (lrq_debug_plan)."""
+    out = (ctypes.c_int64 * 5)()
+    rc = L.load().lrq_debug_plan(("fwd", "bwd", "reserve").index(what), m, n, k, r, out)
+    if rc != 0:
+        raise L.LrqError(rc, f"lrq_debug_plan({what}, {m}, {n}, {k}, {r})")
+    return dict(zip(("bytes", "kernel", "ranges", "folded", "plans"), out))
+
+
 GEMM_PATHS = {"planned": 0, "large": 1, "mid64": 2, "mid128": 3, "mid64s": 4, "mid128s": 5, "mid256": 6, "mid256s": 7}
 
 
