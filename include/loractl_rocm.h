@@ -201,12 +201,14 @@ int lrq_lora_fwd(lrq_ctx* ctx, const lrq_weight* w, const uint16_t* x, int64_t m
 /* lrq_lora_fwd without any allocation. No counterpart in the reference: it
  * is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). Same
- * arguments, kernels and results as lrq_lora_fwd; its workspace is a
+ * arguments as lrq_lora_fwd, and the same kernel and results wherever that
+ * one's workspace fits; else the fastest kernel whose workspace does (the same
+ * products, summed in another order). The workspace is a
  * file-scope device array of LRQ_NOALLOC_SCRATCH_BYTES held by every GPU
  * the library runs on until the process ends, so it calls no hipMalloc,
  * hipFree or event creation. Its first 64 KiB hold the few-token kernels'
- * arrival counters; a shape whose forward needs more scratch than the rest
- * returns LRQ_EINVAL. Every call on one GPU shares that GPU's array:
+ * arrival counters; a shape that no kernel fits into the rest returns
+ * LRQ_EINVAL. Every call on one GPU shares that GPU's array:
  * calls that overlap on one GPU (two streams, two contexts, two threads)
  * race and must be ordered by the caller. */
 int lrq_lora_fwd_noalloc(lrq_ctx* ctx, const lrq_weight* w, const uint16_t* x, int64_t m,
@@ -281,7 +283,8 @@ int lrq_debug_gemm_path(int path);
  * 16 tokens out[1] = the kernel (0 the 256-token tiles; the mid-size tiles of
  * 1: 64 x 64, 2: 128 x 128, 3: 256 rows x 128 tokens), out[2] = its depth
  * ranges, out[3] = 1 if it forms the adapter's products in its own launch.
- * pass 2: out[0] = what lrq_reserve takes. out[4] = cost-model evaluations of
+ * pass 2: out[0] = what lrq_reserve takes. pass 3: the forward in the fixed
+ * scratch of lrq_lora_fwd_noalloc. out[4] = cost-model evaluations of
  * this process before the call. */
 int lrq_debug_plan(int pass, int64_t m, int64_t n, int64_t k, int64_t r, int64_t* out);
 

@@ -50,6 +50,7 @@ struct lrq_ctx {
 // (hipGetSymbolAddress, with that device current) and every later use goes
 // through that pointer.
 static __device__ __align__(256) char scratch[LRQ_NOALLOC_SCRATCH_BYTES];
+constexpr size_t SCRATCH_WS_BYTES = (size_t)LRQ_NOALLOC_SCRATCH_BYTES - LRQ_CNT_BYTES;
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
 static char* g_scratch[kMaxDevices] = {};
@@ -262,20 +263,27 @@ struct LoraPass {
 
 bool fold_rank(int64_t r) { return r > 0 && r % 8 == 0 && r <= 32; }
 
-LoraPass plan_fwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold) {
+// cap: the workspace's size where it cannot grow (the no-allocation
+// forward's scratch); the plan is the fastest that fits it, or, if none does,
+// the fastest.
+constexpr size_t WS_GROWS = SIZE_MAX;
+LoraPass plan_fwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, size_t cap = WS_GROWS) {
   LoraPass p;
   const int rp = (int)round_up(r, 16);
+  const bool fold_ok = may_fold && fold_rank(r);
+  // floats left for the ranges' partials beside `used` bytes
+  auto left = [&](int64_t used) { return cap == WS_GROWS ? PLAN_ANY : ((int64_t)cap - used) / 4 - ((int64_t)cap < used); };
   p.G = (m + 63) / 64;
   p.fs = (k + MID_FOLD_KT - 1) / MID_FOLD_KT;
   p.fp = round_up(p.fs * p.G * 64 * rp, 64);
-  p.fold = may_fold && fold_rank(r) && fold_plan(m, n, k, false, PLAN_ANY, false, &p.g);
-  if (p.fold) {
-    p.ms = p.g.floats;
-    p.bytes = (size_t)(p.fp + p.ms) * 4;
-    return p;
+  p.fold = fold_ok && fold_plan(m, n, k, false, left(p.fp * 4), false, &p.g);
+  const size_t lb = p.fold ? 0 : lora_layout(nullptr, m, n, k, rp, false).bytes;
+  if (!p.fold && !gemm_plan(m, n, k, left((int64_t)lb), &p.g)) {
+    p.fold = fold_ok && fold_plan(m, n, k, false, left(p.fp * 4), true, &p.g);
+    if (!p.fold) gemm_plan(m, n, k, PLAN_ANY, &p.g);
   }
-  gemm_plan(m, n, k, PLAN_ANY, &p.g);
-  p.bytes = lora_layout(nullptr, m, n, k, rp, false).bytes + (size_t)p.g.floats * 4;
+  p.ms = p.fold ? p.g.floats : 0;
+  p.bytes = p.fold ? (size_t)(p.fp + p.ms) * 4 : lb + (size_t)p.g.floats * 4;
   return p;
 }
 
@@ -541,7 +549,7 @@ int lrq_debug_gemm_path(int path) {
 }
 
 int lrq_debug_plan(int pass, int64_t m, int64_t n, int64_t k, int64_t r, int64_t* out) {
-  if (pass < 0 || pass > 2 || m < 1 || n < 1 || k < 1 || r < 0 || r > 64 || !out) return LRQ_EINVAL;
+  if (pass < 0 || pass > 3 || m < 1 || n < 1 || k < 1 || r < 0 || r > 64 || !out) return LRQ_EINVAL;
   for (int i = 0; i < 4; ++i) out[i] = 0;
   out[4] = plans_formed();
   if (pass == 2) {
@@ -556,7 +564,7 @@ int lrq_debug_plan(int pass, int64_t m, int64_t n, int64_t k, int64_t r, int64_t
   }
   LoraPass p;
   if (r > 0) {
-    p = bwd ? plan_bwd(m, n, k, r, true, true) : plan_fwd(m, n, k, r, true);
+    p = bwd ? plan_bwd(m, n, k, r, true, true) : plan_fwd(m, n, k, r, true, pass == 3 ? SCRATCH_WS_BYTES : WS_GROWS);
   } else {
     gemm_plan(m, bwd ? k : n, bwd ? n : k, PLAN_ANY, &p.g);
     p.bytes = (size_t)p.g.floats * 4;
@@ -732,7 +740,7 @@ static int acquire_ws(lrq_ctx* c, WsSource* src, size_t bytes, char** out, uint3
     *cnt = c->cnt;
     return LRQ_OK;
   }
-  const size_t cap = (size_t)LRQ_NOALLOC_SCRATCH_BYTES - LRQ_CNT_BYTES;
+  constexpr size_t cap = SCRATCH_WS_BYTES;
   if (bytes > cap)
     return fail(c, LRQ_EINVAL,
                 "lrq_lora_fwd_noalloc: this shape needs %zu bytes of scratch, more than its fixed %zu; use "
@@ -784,7 +792,8 @@ static int fwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t 
   if (lora) {
     const int rp = (int)round_up(r, 16);
     LRQ_TRY(check_lora_shapes(c, m, w->n, w->k, rp));
-    const LoraPass p = plan_fwd(m, w->n, w->k, r, aligned16(a) && t_out && aligned16(t_out));
+    const LoraPass p = plan_fwd(m, w->n, w->k, r, aligned16(a) && t_out && aligned16(t_out),
+                                src->scratch ? SCRATCH_WS_BYTES : WS_GROWS);
     plan = p.g;
     LRQ_TRY(acquire_ws(c, src, p.bytes, &ws, &cnt));
     if (p.fold) {

@@ -375,10 +375,10 @@ def debug_force_wait_timeout(on: bool):
 
 
 def debug_plan(what: str, m: int, n: int, k: int, r: int) -> dict:
-    """Test hook, host only: how a "fwd" or "bwd" call would run, or what
-    "reserve" takes (lrq_debug_plan)."""
+    """Test hook, host only: how a "fwd", "bwd" or "noalloc" forward call
+    would run, or what "reserve" takes (lrq_debug_plan)."""
     out = (ctypes.c_int64 * 5)()
-    rc = L.load().lrq_debug_plan(("fwd", "bwd", "reserve").index(what), m, n, k, r, out)
+    rc = L.load().lrq_debug_plan(("fwd", "bwd", "reserve", "noalloc").index(what), m, n, k, r, out)
     if rc != 0:
         raise L.LrqError(rc, f"lrq_debug_plan({what}, {m}, {n}, {k}, {r})")
     return dict(zip(("bytes", "kernel", "ranges", "folded", "plans"), out))

@@ -4,6 +4,7 @@ the launch."""
 import pytest
 import torch
 
+from gpu_helpers import check
 from loractl_amd import device as D
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +43,20 @@ def test_a_call_evaluates_the_cost_model_once(cuda, M, r, most):
         before = formed()
         call()
         assert formed() - before <= most
+
+
+@pytest.mark.parametrize("M,K,N,r", [(96, 15360, 12288, 64), (512, 15360, 3072, 32), (640, 16384, 9728, 16),
+                                     (1024, 16384, 9216, 16), (2112, 14336, 4096, 16), (8192, 12288, 9216, 32)])
+def test_noalloc_takes_a_kernel_that_fits_its_scratch(cuda, M, K, N, r):
+    """Shapes whose fastest plan needs more than the 32 MiB scratch array
+    (depth-range partials, t's slice partials) run on another that fits."""
+    wq, x, _, a, b = _case(cuda, M, K, N, r, M + K)
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
+    t = torch.empty((M, r), dtype=torch.bfloat16, device=cuda)
+    D.lora_fwd_noalloc(x, wq, a, b, 1.0, y, t)
+    D.sync()
+    rows = torch.linspace(0, M - 1, min(M, 64), device=cuda).long()
+    xf = x[rows].float()
+    t_ref = xf @ a.float()
+    check("t", t[rows], t_ref.cpu().numpy())
+    check("y", y[rows], (xf @ D.dequant(wq).t() + t_ref @ b.float()).cpu().numpy())

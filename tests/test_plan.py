@@ -1,0 +1,31 @@
+"""How calls plan their kernel and workspace, through the host-only planner
+hook (no GPU)."""
+
+import itertools
+
+import pytest
+
+from loractl_amd import _lib as L
+from loractl_amd import device as D
+
+SCRATCH = L.LRQ_NOALLOC_SCRATCH_BYTES - (64 << 10)  # past the arrival counters
+TOKENS = [17, 96, 192, 320, 512, 640, 896, 1024, 1792, 2112, 4096, 8192]
+DIMS = [512, 2560, 3072, 4096, 9216, 12288, 14336, 16384, 18432]
+
+
+@pytest.mark.parametrize("m,k,n,r", [(96, 15360, 12288, 64), (128, 18432, 12288, 64), (320, 16384, 16384, 16),
+                                     (512, 15360, 3072, 32), (640, 16384, 9728, 16), (1024, 16384, 9216, 16),
+                                     (2112, 14336, 4096, 16), (8192, 12288, 2560, 32), (8192, 12288, 9216, 32)])
+def test_noalloc_plans_a_kernel_that_fits(m, k, n, r):
+    """The fastest plan of these needs more than the scratch; another fits."""
+    assert D.debug_plan("fwd", m, n, k, r)["bytes"] > SCRATCH
+    assert D.debug_plan("noalloc", m, n, k, r)["bytes"] <= SCRATCH
+
+
+def test_noalloc_takes_the_ordinary_plan_where_it_fits():
+    for m, k, n, r in itertools.product(TOKENS, DIMS, DIMS, (16, 32, 64)):
+        p, q = D.debug_plan("fwd", m, n, k, r), D.debug_plan("noalloc", m, n, k, r)
+        keys = ("bytes", "kernel", "ranges", "folded")
+        if p["bytes"] <= SCRATCH:
+            assert all(p[x] == q[x] for x in keys), (m, k, n, r)
+        assert q["bytes"] <= SCRATCH, (m, k, n, r)
