@@ -276,10 +276,10 @@ LoraPass plan_fwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, siz
   p.G = (m + 63) / 64;
   p.fs = (k + MID_FOLD_KT - 1) / MID_FOLD_KT;
   p.fp = round_up(p.fs * p.G * 64 * rp, 64);
-  p.fold = fold_ok && fold_plan(m, n, k, false, left(p.fp * 4), false, &p.g);
+  p.fold = fold_ok && fold_plan(m, n, k, false, rp, left(p.fp * 4), false, &p.g);
   const size_t lb = p.fold ? 0 : lora_layout(nullptr, m, n, k, rp, false).bytes;
   if (!p.fold && !gemm_plan(m, n, k, left((int64_t)lb), &p.g)) {
-    p.fold = fold_ok && fold_plan(m, n, k, false, left(p.fp * 4), true, &p.g);
+    p.fold = fold_ok && fold_plan(m, n, k, false, rp, left(p.fp * 4), true, &p.g);
     if (!p.fold) gemm_plan(m, n, k, PLAN_ANY, &p.g);
   }
   p.ms = p.fold ? p.g.floats : 0;
@@ -294,7 +294,7 @@ LoraPass plan_bwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, boo
   const size_t lb = lora_layout(nullptr, m, n, k, rp, true).bytes;
   p.G = (m + 63) / 64;
   p.fs = (n + MID_FOLD_KT - 1) / MID_FOLD_KT;
-  p.fold = gemm && may_fold && fold_rank(r) && fold_plan(m, k, n, true, PLAN_ANY, false, &p.g);
+  p.fold = gemm && may_fold && fold_rank(r) && fold_plan(m, k, n, true, rp, PLAN_ANY, false, &p.g);
   if (!p.fold) {
     if (gemm) gemm_plan(m, k, n, PLAN_ANY, &p.g);
     p.bytes = lb + (size_t)p.g.floats * 4;
@@ -307,10 +307,10 @@ LoraPass plan_bwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, boo
   const int lds = mid_tn_lds(p.g.v);
   p.tpb = mid_tn_plan(m, n, k, rp, lds);
   p.tpa = mid_tn_plan(m, k, n, rp, lds);
-  p.fold_tn = p.tpb.splits > 0 && p.tpa.splits > 0 &&
-              2 * p.G + p.g.tiles + TN_WAVES * (p.tpb.tiles + p.tpa.tiles) <= SK_MAX_NB;
   p.tb = p.tpb.splits > 1 ? (int64_t)p.tpb.splits * n * rp : 0;
   p.ta = p.tpa.splits > 1 ? (int64_t)p.tpa.splits * k * rp : 0;
+  p.fold_tn = p.tpb.splits > 0 && p.tpa.splits > 0 && std::max(p.tb, p.ta) * 4 < (int64_t)1 << 31 &&
+              2 * p.G + p.g.tiles + TN_WAVES * (p.tpb.tiles + p.tpa.tiles) <= SK_MAX_NB;
   p.bytes = lb + (size_t)(p.fp + p.ms + p.tb + p.ta) * 4;
   return p;
 }

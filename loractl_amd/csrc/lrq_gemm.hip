@@ -979,12 +979,16 @@ bool gemm_plan(int64_t m, int64_t e, int64_t depth, int64_t max_floats, GemmPlan
   return found;
 }
 
-bool fold_plan(int64_t m, int64_t e, int64_t depth, bool bwd, int64_t max_floats, bool always, GemmPlan* p) {
+bool fold_plan(int64_t m, int64_t e, int64_t depth, bool bwd, int rp, int64_t max_floats, bool always, GemmPlan* p) {
   *p = GemmPlan{};
   const int64_t G = (m + 63) / 64, mg = G * 64;
   if (m <= 0 || e <= 0 || g_gemm_path == 1) return false;
-  // the groups' arrivals and flags have counters
-  if (2 * G > SK_MAX_NB) return false;
+  // the groups' arrivals and flags have counters; the factor slices address
+  // the activations [m][depth], and their partials, as one buffer each, with
+  // 32-bit offsets, and a masked access (offset LRQ_OOB) must lie past its end
+  if (2 * G > SK_MAX_NB || m * depth * 2 > (int64_t)LRQ_OOB ||
+      (depth + MID_FOLD_KT - 1) / MID_FOLD_KT * mg * rp * 4 > (int64_t)LRQ_OOB)
+    return false;
   g_plans.fetch_add(1, std::memory_order_relaxed);
   bool split = false;
   const int fv = forced_variant(&split);

@@ -535,8 +535,8 @@ hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int 
         !a.fout || a.fout_ld % 8 != 0 || a.fout_ld < a.r || a.fout_ld > a.rp || !a.fpart || !a.fcnt ||
         2 * G > SK_MAX_NB || a.fold_wgs % 8 != 0 ||
         a.fold_slices != (int)((a.l + MID_FOLD_KT - 1) / MID_FOLD_KT) || a.fold_wgs < a.fold_slices * G ||
-        a.m * a.l * 2 >= ((int64_t)1 << 32) || a.m * a.fout_ld * 2 >= ((int64_t)1 << 32) ||
-        (int64_t)a.fold_slices * G * 64 * a.rp * 4 >= ((int64_t)1 << 32))
+        a.m * a.l * 2 > (int64_t)LRQ_OOB || a.m * a.fout_ld * 2 > (int64_t)LRQ_OOB ||
+        (int64_t)a.fold_slices * G * 64 * a.rp * 4 > (int64_t)LRQ_OOB)
       return hipErrorInvalidValue;
     // the weight gradients' jobs after the tiles (backward): each a whole
     // plan of token slices that fit the variant's LDS, over all the launch's

@@ -114,11 +114,11 @@ constexpr int64_t PLAN_ANY = INT64_MAX;
 // the kernel modelled fastest of those whose partials fit max_floats. False
 // if none does.
 bool gemm_plan(int64_t m, int64_t e, int64_t depth, int64_t max_floats, GemmPlan* p);
-// The product and its LoRA factors (t; backward u, dA and dB) in one
-// launch: the fastest such kernel within max_floats. False if none is
-// modelled faster than the 256-token tiles and their side launches (`always`:
-// if there is none).
-bool fold_plan(int64_t m, int64_t e, int64_t depth, bool bwd, int64_t max_floats, bool always, GemmPlan* p);
+// The product and its LoRA factors (t; backward u, dA and dB; padded rank rp)
+// in one launch: the fastest such kernel within max_floats. False if the
+// launch cannot take the shape, or none is modelled faster than the 256-token
+// tiles and their side launches (`always`: the first alone).
+bool fold_plan(int64_t m, int64_t e, int64_t depth, bool bwd, int rp, int64_t max_floats, bool always, GemmPlan* p);
 // cost-model evaluations of this process (lrq_debug_plan)
 int64_t plans_formed();
 

@@ -60,3 +60,21 @@ def test_noalloc_takes_a_kernel_that_fits_its_scratch(cuda, M, K, N, r):
     t_ref = xf @ a.float()
     check("t", t[rows], t_ref.cpu().numpy())
     check("y", y[rows], (xf @ D.dequant(wq).t() + t_ref @ b.float()).cpu().numpy())
+
+
+@pytest.mark.parametrize("M,N", [(100000, 21512), (100000, 18440)], ids=["past 4 GiB", "past 2 GiB"])
+def test_input_gradient_of_activations_past_the_fold_offsets(cuda, M, N):
+    """The side products formed beside the tiles address dy [m, n] as one
+    buffer with 32-bit offsets; a larger dy takes separate launches. A NaN in
+    dy (at the byte offset that masked loads use) stays in its own token."""
+    K, r = 512, 16
+    wq, x, dy, a, b = _case(cuda, M, K, N, r, N)
+    bad = 2 ** 30 // N
+    dy.view(-1)[2 ** 30] = float("nan")
+    dx, da, db = D.lora_bwd(x, dy, wq, a, b, 1.0, torch.zeros(M, r, dtype=torch.bfloat16, device=cuda))
+    D.sync()
+    rows = torch.tensor([0, 1, bad - 1, bad + 1, M // 2, M - 1], device=cuda)
+    dyf = dy[rows].float()
+    check("dx", dx[rows], (dyf @ D.dequant(wq) + (dyf @ b.float().t()) @ a.float().t()).cpu().numpy())
+    nan = torch.isnan(dx.float()).any(1).nonzero().flatten()
+    assert nan.tolist() == [bad]

@@ -29,3 +29,13 @@ def test_noalloc_takes_the_ordinary_plan_where_it_fits():
         if p["bytes"] <= SCRATCH:
             assert all(p[x] == q[x] for x in keys), (m, k, n, r)
         assert q["bytes"] <= SCRATCH, (m, k, n, r)
+
+
+@pytest.mark.parametrize("what,m,n,k", [("bwd", 100000, 21512, 512), ("bwd", 100000, 18440, 512), ("bwd", 80000, 18440, 128),
+                                        ("fwd", 100000, 512, 18432)])
+def test_folded_factors_stay_within_32_bit_offsets(what, m, n, k):
+    """Activations of 2 GiB and more (the folded factor's masked loads use
+    that offset) take side launches; smaller ones fold."""
+    for r in (8, 16, 32):
+        assert not D.debug_plan(what, m, n, k, r)["folded"]
+        assert D.debug_plan(what, 2048, 1536, 1536, r)["folded"]
