@@ -325,40 +325,27 @@ size_t few_bwd_bytes(int64_t m, int64_t n, int64_t k, int rp) {
   return few_u_bytes(m, rp) + skinny_ws_bytes(skinny_plan(k, n, rp, get_num_cus()), m, k, rp);
 }
 
-// Workspace of every call of up to m tokens at this rank.
+// Workspace of every call of up to m tokens at rank r, and without an
+// adapter. The plans' partials are not monotonic in the token count (fewer
+// tiles, more depth ranges), but within a 64-token group every part grows
+// with it: the largest over the groups' last counts. A call may not fold for
+// its pointers' alignment.
 size_t reserve_bytes(int64_t m, int64_t n, int64_t k, int64_t r) {
   const int64_t lr = r > 0 ? r : 16;
   const int rp = (int)round_up(lr, 16);
-  size_t need = std::max(plan_fwd(m, n, k, lr, false).bytes, plan_bwd(m, n, k, lr, false, true).bytes);
-  // the fused GEMMs' split partials are not monotonic in the token count
-  // (fewer tiles, more depth ranges): their largest size over m' <= m, which
-  // peaks at a whole number of 64-token tiles
-  GemmPlan f, b;
-  gemm_plan(m, n, k, PLAN_ANY, &f);
-  gemm_plan(m, k, n, PLAN_ANY, &b);
-  const int64_t gp_m = std::max(f.floats, b.floats);
-  int64_t gp_max = gp_m;
-  for (int64_t mm = 64; mm < m; mm += 64) {
-    gemm_plan(mm, n, k, PLAN_ANY, &f);
-    gemm_plan(mm, k, n, PLAN_ANY, &b);
-    gp_max = std::max(gp_max, std::max(f.floats, b.floats));
+  size_t need = (size_t)round_up(n * 4, 256);  // the fp8 quantizer's row maxima
+  for (int64_t mg = 0; mg < m; mg += 64) {
+    const int64_t mm = std::min(mg + 64, m);
+    for (bool fold : {false, true}) {
+      if (fold && !fold_rank(r)) continue;
+      need = std::max(need, std::max(plan_fwd(mm, n, k, lr, fold).bytes, plan_bwd(mm, n, k, lr, fold, true).bytes));
+    }
   }
-  need += (size_t)(gp_max - gp_m) * 4;
   if (m >= 1) {
     const int64_t mm = m < 16 ? m : 16;
     need = std::max(need, std::max(few_fwd_bytes(mm, n, k, rp), few_bwd_bytes(mm, n, k, rp)));
   }
-  if (fold_rank(r) && m > 16) {
-    // the one-launch mid-size passes, at every token count up to m
-    const size_t lb = lora_layout(nullptr, m, n, k, rp, true).bytes;
-    for (int64_t mm = 64;; mm += 64) {
-      const int64_t mt = mm < m ? mm : m;
-      const LoraPass p = plan_bwd(mt, n, k, r, true, true);
-      need = std::max(need, std::max(plan_fwd(mt, n, k, r, true).bytes, lb + (size_t)(p.fp + p.ms + p.tb + p.ta) * 4));
-      if (mt == m) break;
-    }
-  }
-  return std::max(need, (size_t)round_up(n * 4, 256));  // and the fp8 quantizer's row maxima
+  return need;
 }
 
 // Shape limit of the LoRA kernels: 32-bit buffer offsets over one slice.

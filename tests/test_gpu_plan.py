@@ -78,3 +78,38 @@ def test_input_gradient_of_activations_past_the_fold_offsets(cuda, M, N):
     check("dx", dx[rows], (dyf @ D.dequant(wq) + (dyf @ b.float().t()) @ a.float().t()).cpu().numpy())
     nan = torch.isnan(dx.float()).any(1).nonzero().flatten()
     assert nan.tolist() == [bad]
+
+
+@pytest.mark.parametrize("M,m,K,N,r", [(1024, 192, 3072, 3072, 16), (4096, 896, 3072, 12288, 32)])
+def test_reserve_serves_every_smaller_token_count(cuda, M, m, K, N, r):
+    """After lrq_reserve for M tokens a call of m < M tokens is captured
+    without allocating, although it may split its depth into more ranges."""
+    wq, x, dy, a, b = _case(cuda, m, K, N, r, m)
+    y, dx = torch.empty_like(dy), torch.empty_like(x)
+    t = torch.empty((m, r), dtype=torch.bfloat16, device=cuda)
+    da = torch.empty((K, r), device=cuda)
+    db = torch.empty((r, N), device=cuda)
+    stream = torch.cuda.Stream()
+    ctx = D.Context(0, stream.cuda_stream)  # a context of its own: no workspace yet
+    key = (0, stream.cuda_stream)
+    old = D._ctxs.get(key)
+    D._ctxs[key] = ctx
+    try:
+        stream.wait_stream(torch.cuda.current_stream())
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(stream):
+            D.reserve(M, N, K, r)
+            with torch.cuda.graph(graph, stream=stream):
+                D.lora_fwd(x, wq, a, b, 1.0, y=y, t=t)
+                D.lora_bwd(x, dy, wq, a, b, 1.0, t, out=(dx, da, db))
+        graph.replay()
+        torch.cuda.synchronize()
+    finally:
+        del graph
+        if old is None:
+            del D._ctxs[key]
+        else:
+            D._ctxs[key] = old
+    y0, t0 = D.lora_fwd(x, wq, a, b, 1.0)
+    for got, want in zip((y, t, dx, da, db), (y0, t0) + tuple(D.lora_bwd(x, dy, wq, a, b, 1.0, t0))):
+        assert torch.equal(got, want)

@@ -2,6 +2,7 @@
 hook (no GPU)."""
 
 import itertools
+import random
 
 import pytest
 
@@ -39,3 +40,16 @@ def test_folded_factors_stay_within_32_bit_offsets(what, m, n, k):
     for r in (8, 16, 32):
         assert not D.debug_plan(what, m, n, k, r)["folded"]
         assert D.debug_plan(what, 2048, 1536, 1536, r)["folded"]
+
+
+@pytest.mark.parametrize("n,k", [(12288, 3072), (3072, 12288), (3072, 3072), (9728, 2560), (8192, 512), (520, 96)])
+def test_reserve_covers_every_smaller_token_count(n, k):
+    """Also at counts inside a 64-token group, past the kernels' tiles."""
+    rng = random.Random(n + k)
+    for r in (0, 8, 16, 17, 32, 64):
+        for m in (1, 16, 100, 512, 1000, 1024, 2048, 4096):
+            have = D.debug_plan("reserve", m, n, k, r)["bytes"]
+            counts = set(range(64, m, 64)) | {m} | {rng.randint(1, m) for _ in range(200)}
+            for q in counts:
+                need = max(D.debug_plan(w, q, n, k, r)["bytes"] for w in ("fwd", "bwd"))
+                assert need <= have, (m, q, r, need, have)
