@@ -190,6 +190,15 @@ LRQ_DEV f32x4 acc_zero4() {
   return z;
 }
 
+// The same in vector registers, for kernels whose accumulators are there: one
+// accumulator register anywhere makes the compiler halve the vector registers
+// of the whole kernel.
+LRQ_DEV f32x4 acc_zero4_v() {
+  f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+  asm volatile("" : "+v"(z));
+  return z;
+}
+
 LRQ_DEV bf16x8 as_bf16x8(const u32x4& v) { return __builtin_bit_cast(bf16x8, v); }
 
 LRQ_DEV u32x4 ld16(const void* p) { return *reinterpret_cast<const u32x4*>(p); }

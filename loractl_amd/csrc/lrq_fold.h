@@ -171,8 +171,11 @@ LRQ_DEV void mid_flags_done(const GemmArgs& a, int readers) {
 // flags of the 64-token groups of its token slice, then reads u at device
 // scope; a wait that runs out flags the failure and makes its sums NaN.
 // The factor slice goes to sq, the combine buffer to sr (LDSB bytes each; one
-// buffer may serve as both).
-template <int LDSB>
+// buffer may serve as both). VACC: sums in vector registers (the 128-token
+// tiles'): in accumulator registers their kernels had 128 vector registers
+// left and spilled 33 to 36 of them in a rank-32 block (backward at 384
+// tokens, 3072 -> 12288, rank 32: 72 -> 58 us without the spills).
+template <int LDSB, bool VACC>
 LRQ_DEV void mid_tn(const GemmArgs& a, int tb, uint32_t want, int readers, uint16_t* sq, uint16_t* sr) {
   const bool second = tb >= a.tj[0].blocks;
   const int ji = second ? 1 : 0;
@@ -181,9 +184,9 @@ LRQ_DEV void mid_tn(const GemmArgs& a, int tb, uint32_t want, int readers, uint1
   float* const red = reinterpret_cast<float*>(sr);
   if (ji != a.tn_da) {
     if (a.rp == 32)
-      tn_block<2, LDSB, LDSB, false>(j, bid, sq, red, false);
+      tn_block<2, LDSB, LDSB, false, VACC>(j, bid, sq, red, false);
     else
-      tn_block<1, LDSB, LDSB, false>(j, bid, sq, red, false);
+      tn_block<1, LDSB, LDSB, false, VACC>(j, bid, sq, red, false);
     return;
   }
   __shared__ int bad[2];
@@ -212,9 +215,9 @@ LRQ_DEV void mid_tn(const GemmArgs& a, int tb, uint32_t want, int readers, uint1
   const bool poison = bad[half] != 0;
   mid_flags_done<256>(a, readers);
   if (a.rp == 32)
-    tn_block<2, LDSB, LDSB, true>(j, bid, sq, red, poison);
+    tn_block<2, LDSB, LDSB, true, VACC>(j, bid, sq, red, poison);
   else
-    tn_block<1, LDSB, LDSB, true>(j, bid, sq, red, poison);
+    tn_block<1, LDSB, LDSB, true, VACC>(j, bid, sq, red, poison);
 }
 
 }  // namespace

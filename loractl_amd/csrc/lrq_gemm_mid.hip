@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(256, 2) k_mid(GemmArgs a, int tiles_m, int til
       if ((int)blockIdx.x >= a.fold_wgs + nunits) {
         static_assert(MID_TN_LDS <= XB * 2, "a weight-gradient block's LDS fits one stage buffer");
         const int nda = a.tn_da >= 0 ? a.tj[a.tn_da].blocks : 0;
-        mid_tn<MID_TN_LDS>(a, (int)blockIdx.x - a.fold_wgs - nunits, want, ntiles + nda, sx0, sx1);
+        mid_tn<MID_TN_LDS, false>(a, (int)blockIdx.x - a.fold_wgs - nunits, want, ntiles + nda, sx0, sx1);
         return;
       }
     }

@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(WNT, 2) k_w8(GemmArgs a, int tiles_m, int tile
         const int wg = (int)blockIdx.x - a.fold_wgs - nunits, w0 = (a.tj[0].blocks + 1) / 2;
         const int tb = wg < w0 ? 2 * wg + half : a.tj[0].blocks + 2 * (wg - w0) + half;
         if (tb < (wg < w0 ? a.tj[0].blocks : a.tn_blocks))
-          mid_tn<W8_TN_LDS>(a, tb, want, ntiles + nda, lt, lt);
+          mid_tn<W8_TN_LDS, true>(a, tb, want, ntiles + nda, lt, lt);
         return;
       }
     }

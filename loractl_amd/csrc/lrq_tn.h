@@ -54,7 +54,7 @@ LRQ_DEV void zero_dev(uint32_t* c) { __hip_atomic_store(c, 0u, __ATOMIC_RELAXED,
 // in the same launch, so it is read at device scope (past the per-XCD L2s;
 // a.ldq a multiple of 8). `poison`: the factor is not trustworthy (a wait
 // for it ran out), so the slice's sums are NaN.
-template <int NJT, int QBYTES, int RBYTES, bool QDEV>
+template <int NJT, int QBYTES, int RBYTES, bool QDEV, bool VACC = false>
 LRQ_DEV void tn_block(const TnArgs& a, int bid, uint16_t* sQ, float* red, bool poison) {
   constexpr int RP = 16 * NJT;
   // combine rounds: RCOLS columns at a time (128 when the buffer holds a
@@ -83,7 +83,7 @@ LRQ_DEV void tn_block(const TnArgs& a, int bid, uint16_t* sQ, float* red, bool p
 #pragma unroll
   for (int q = 0; q < 8; ++q)
 #pragma unroll
-    for (int jt = 0; jt < NJT; ++jt) acc[q][jt] = acc_zero4();
+    for (int jt = 0; jt < NJT; ++jt) acc[q][jt] = VACC ? acc_zero4_v() : acc_zero4();
 
   const int64_t nchunks = (toks + 127) / 128;
   u32x4 pv[2][8];

@@ -3,6 +3,7 @@ compiles to assembly), checked as the other kernel files' are, and
 the wait for the copies before each barrier of its pipelined loop."""
 
 import os
+import re
 import tempfile
 
 import isa_hazards as H
@@ -23,3 +24,6 @@ def test_w8_meets_wait_states():
         total += n
         bad += v + H.check_dpp(k)[0]
     assert total > 0 and not bad, bad[:5]
+    # the side products' registers stay within the tiles': no spills to scratch
+    spills = re.findall(r"^\s*\.vgpr_spill_count:\s*(\d+)", text, flags=re.M)
+    assert spills and not any(int(s) for s in spills), spills
