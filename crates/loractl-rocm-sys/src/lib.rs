@@ -195,7 +195,7 @@ pub mod ffi {
         pub fn lrq_probe_stream_read(ctx: *mut lrq_ctx, data: *const c_void, bytes: i64) -> c_int;
         pub fn lrq_debug_force_wait_timeout(on: c_int) -> c_int;
         pub fn lrq_debug_gemm_path(path: c_int) -> c_int;
-        pub fn lrq_debug_plan(pass: c_int, m: i64, n: i64, k: i64, r: i64, out: *mut i64) -> c_int;
+        pub fn lrq_debug_plan(pass: c_int, format: c_int, m: i64, n: i64, k: i64, r: i64, out: *mut i64) -> c_int;
     }
 }
 

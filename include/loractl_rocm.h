@@ -272,21 +272,24 @@ int lrq_debug_force_wait_timeout(int on);
  * the 64-row x 64-token and the 128-row x 128-token tiles (depth ranges as
  * planned); 4 and 5 the same tiles with at least two depth ranges wherever
  * the depth has two whole rounds of their pipeline; 6 and 7 the 256-row x
- * 128-token tiles likewise. Every path computes the same products; a
+ * 128-token tiles likewise; 8 and 9 the 64-row x 128-token tiles, which run
+ * only backward passes that form the adapter's products in their launch (the
+ * others as planned). Every path computes the same products; a
  * workspace sized by lrq_reserve under one setting grows on the next hot call
  * if another needs more. */
 int lrq_debug_gemm_path(int path);
 
 /* Test hook, no counterpart in the reference; host only, no context: how a
- * call of m tokens at rank r (0: no adapter) would run. pass 0 the forward, 1
+ * call of m tokens at rank r (0: no adapter) on a weight [n, k] of `format`
+ * would run. pass 0 the forward, 1
  * the backward with an input gradient; out[0] = its workspace bytes, and past
  * 16 tokens out[1] = the kernel (0 the 256-token tiles; the mid-size tiles of
- * 1: 64 x 64, 2: 128 x 128, 3: 256 rows x 128 tokens), out[2] = its depth
+ * 1: 64 x 64, 2: 128 x 128, 3: 256 rows x 128 tokens, 4: 64 x 128), out[2] = its depth
  * ranges, out[3] = 1 if it forms the adapter's products in its own launch.
  * pass 2: out[0] = what lrq_reserve takes. pass 3: the forward in the fixed
  * scratch of lrq_lora_fwd_noalloc. out[4] = cost-model evaluations of
  * this process before the call. */
-int lrq_debug_plan(int pass, int64_t m, int64_t n, int64_t k, int64_t r, int64_t* out);
+int lrq_debug_plan(int pass, int format, int64_t m, int64_t n, int64_t k, int64_t r, int64_t* out);
 
 #ifdef __cplusplus
 }

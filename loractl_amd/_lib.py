@@ -92,7 +92,7 @@ SIGNATURES = {
     "lrq_probe_stream_read": (_i32, [_vp, _vp, _i64]),
     "lrq_debug_force_wait_timeout": (_i32, [_i32]),
     "lrq_debug_gemm_path": (_i32, [_i32]),
-    "lrq_debug_plan": (_i32, [_i32, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)]),
+    "lrq_debug_plan": (_i32, [_i32, _i32, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)]),
 }
 
 _lib = None

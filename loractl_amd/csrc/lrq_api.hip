@@ -267,7 +267,7 @@ bool fold_rank(int64_t r) { return r > 0 && r % 8 == 0 && r <= 32; }
 // forward's scratch); the plan is the fastest that fits it, or, if none does,
 // the fastest.
 constexpr size_t WS_GROWS = SIZE_MAX;
-LoraPass plan_fwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, size_t cap = WS_GROWS) {
+LoraPass plan_fwd(int fmt, int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, size_t cap = WS_GROWS) {
   LoraPass p;
   const int rp = (int)round_up(r, 16);
   const bool fold_ok = may_fold && fold_rank(r);
@@ -276,11 +276,11 @@ LoraPass plan_fwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, siz
   p.G = (m + 63) / 64;
   p.fs = (k + MID_FOLD_KT - 1) / MID_FOLD_KT;
   p.fp = round_up(p.fs * p.G * 64 * rp, 64);
-  p.fold = fold_ok && fold_plan(m, n, k, false, rp, left(p.fp * 4), false, &p.g);
+  p.fold = fold_ok && fold_plan(fmt, m, n, k, false, rp, left(p.fp * 4), false, &p.g);
   const size_t lb = p.fold ? 0 : lora_layout(nullptr, m, n, k, rp, false).bytes;
-  if (!p.fold && !gemm_plan(m, n, k, left((int64_t)lb), &p.g)) {
-    p.fold = fold_ok && fold_plan(m, n, k, false, rp, left(p.fp * 4), true, &p.g);
-    if (!p.fold) gemm_plan(m, n, k, PLAN_ANY, &p.g);
+  if (!p.fold && !gemm_plan(fmt, m, n, k, false, left((int64_t)lb), &p.g)) {
+    p.fold = fold_ok && fold_plan(fmt, m, n, k, false, rp, left(p.fp * 4), true, &p.g);
+    if (!p.fold) gemm_plan(fmt, m, n, k, false, PLAN_ANY, &p.g);
   }
   p.ms = p.fold ? p.g.floats : 0;
   p.bytes = p.fold ? (size_t)(p.fp + p.ms) * 4 : lb + (size_t)p.g.floats * 4;
@@ -288,15 +288,15 @@ LoraPass plan_fwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, siz
 }
 
 // gemm: the pass has an input gradient
-LoraPass plan_bwd(int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, bool gemm) {
+LoraPass plan_bwd(int fmt, int64_t m, int64_t n, int64_t k, int64_t r, bool may_fold, bool gemm) {
   LoraPass p;
   const int rp = (int)round_up(r, 16);
   const size_t lb = lora_layout(nullptr, m, n, k, rp, true).bytes;
   p.G = (m + 63) / 64;
   p.fs = (n + MID_FOLD_KT - 1) / MID_FOLD_KT;
-  p.fold = gemm && may_fold && fold_rank(r) && fold_plan(m, k, n, true, rp, PLAN_ANY, false, &p.g);
+  p.fold = gemm && may_fold && fold_rank(r) && fold_plan(fmt, m, k, n, true, rp, PLAN_ANY, false, &p.g);
   if (!p.fold) {
-    if (gemm) gemm_plan(m, k, n, PLAN_ANY, &p.g);
+    if (gemm) gemm_plan(fmt, m, k, n, true, PLAN_ANY, &p.g);
     p.bytes = lb + (size_t)p.g.floats * 4;
     return p;
   }
@@ -326,20 +326,20 @@ size_t few_bwd_bytes(int64_t m, int64_t n, int64_t k, int rp) {
 }
 
 // Workspace of every call of up to m tokens at rank r, and without an
-// adapter. The plans' partials are not monotonic in the token count (fewer
-// tiles, more depth ranges), but within a 64-token group every part grows
-// with it: the largest over the groups' last counts. A call may not fold for
-// its pointers' alignment.
+// adapter, on a weight of any format. The plans' partials are not monotonic in
+// the token count (fewer tiles, more depth ranges), but within a 64-token
+// group every part grows with it: the largest over the groups' last counts. A
+// call may not fold for its pointers' alignment.
 size_t reserve_bytes(int64_t m, int64_t n, int64_t k, int64_t r) {
   const int64_t lr = r > 0 ? r : 16;
   const int rp = (int)round_up(lr, 16);
   size_t need = (size_t)round_up(n * 4, 256);  // the fp8 quantizer's row maxima
   for (int64_t mg = 0; mg < m; mg += 64) {
     const int64_t mm = std::min(mg + 64, m);
-    for (bool fold : {false, true}) {
-      if (fold && !fold_rank(r)) continue;
-      need = std::max(need, std::max(plan_fwd(mm, n, k, lr, fold).bytes, plan_bwd(mm, n, k, lr, fold, true).bytes));
-    }
+    for (int fmt : {LRQ_FMT_INT4, LRQ_FMT_INT8, LRQ_FMT_FP8})
+      for (bool fold : {false, true})
+        if (!fold || fold_rank(r))
+          need = std::max(need, std::max(plan_fwd(fmt, mm, n, k, lr, fold).bytes, plan_bwd(fmt, mm, n, k, lr, fold, true).bytes));
   }
   if (m >= 1) {
     const int64_t mm = m < 16 ? m : 16;
@@ -530,13 +530,14 @@ int lrq_probe_stream_read(lrq_ctx* c, const void* data, int64_t bytes) {
 }
 
 int lrq_debug_gemm_path(int path) {
-  if (path < 0 || path > 7) return LRQ_EINVAL;
+  if (path < 0 || path > 9) return LRQ_EINVAL;
   set_gemm_path(path);
   return LRQ_OK;
 }
 
-int lrq_debug_plan(int pass, int64_t m, int64_t n, int64_t k, int64_t r, int64_t* out) {
-  if (pass < 0 || pass > 3 || m < 1 || n < 1 || k < 1 || r < 0 || r > 64 || !out) return LRQ_EINVAL;
+int lrq_debug_plan(int pass, int format, int64_t m, int64_t n, int64_t k, int64_t r, int64_t* out) {
+  const int fmt = format;
+  if (pass < 0 || pass > 3 || fmt < LRQ_FMT_INT4 || fmt > LRQ_FMT_INT8 || m < 1 || n < 1 || k < 1 || r < 0 || r > 64 || !out) return LRQ_EINVAL;
   for (int i = 0; i < 4; ++i) out[i] = 0;
   out[4] = plans_formed();
   if (pass == 2) {
@@ -551,9 +552,9 @@ int lrq_debug_plan(int pass, int64_t m, int64_t n, int64_t k, int64_t r, int64_t
   }
   LoraPass p;
   if (r > 0) {
-    p = bwd ? plan_bwd(m, n, k, r, true, true) : plan_fwd(m, n, k, r, true, pass == 3 ? SCRATCH_WS_BYTES : WS_GROWS);
+    p = bwd ? plan_bwd(fmt, m, n, k, r, true, true) : plan_fwd(fmt, m, n, k, r, true, pass == 3 ? SCRATCH_WS_BYTES : WS_GROWS);
   } else {
-    gemm_plan(m, bwd ? k : n, bwd ? n : k, PLAN_ANY, &p.g);
+    gemm_plan(fmt, m, bwd ? k : n, bwd ? n : k, bwd, PLAN_ANY, &p.g);
     p.bytes = (size_t)p.g.floats * 4;
   }
   out[0] = (int64_t)p.bytes;
@@ -779,7 +780,7 @@ static int fwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t 
   if (lora) {
     const int rp = (int)round_up(r, 16);
     LRQ_TRY(check_lora_shapes(c, m, w->n, w->k, rp));
-    const LoraPass p = plan_fwd(m, w->n, w->k, r, aligned16(a) && t_out && aligned16(t_out),
+    const LoraPass p = plan_fwd(fmt, m, w->n, w->k, r, aligned16(a) && t_out && aligned16(t_out),
                                 src->scratch ? SCRATCH_WS_BYTES : WS_GROWS);
     plan = p.g;
     LRQ_TRY(acquire_ws(c, src, p.bytes, &ws, &cnt));
@@ -820,7 +821,7 @@ static int fwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t 
     ga.part = reinterpret_cast<float*>(ws + lw.bytes);
     ga.mcnt = cnt;
   } else {
-    gemm_plan(m, w->n, w->k, PLAN_ANY, &plan);
+    gemm_plan(fmt, m, w->n, w->k, false, PLAN_ANY, &plan);
     if (plan.floats > 0) {
       LRQ_TRY(acquire_ws(c, src, (size_t)plan.floats * 4, &ws, &cnt));
       ga.part = reinterpret_cast<float*>(ws);
@@ -907,7 +908,7 @@ static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const ui
       }));
       return LRQ_OK;
     }
-    const LoraPass p = plan_bwd(m, w->n, w->k, r, aligned16(a), dx != nullptr);
+    const LoraPass p = plan_bwd(fmt, m, w->n, w->k, r, aligned16(a), dx != nullptr);
     plan = p.g;
     LRQ_TRY(ensure_ws(c, p.bytes));
     const LoraWs ws = lora_layout(c->ws, m, w->n, w->k, rp, true);
@@ -988,7 +989,7 @@ static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const ui
       return launch_skinny(c->stream, fmt, true, ga, nullptr, sp, part, nullptr, c->cnt, 1.0f, nullptr);
     });
   }
-  gemm_plan(m, wk, wn, PLAN_ANY, &plan);
+  gemm_plan(fmt, m, wk, wn, true, PLAN_ANY, &plan);
   LRQ_TRY(ensure_ws(c, (size_t)plan.floats * 4));
   if (plan.floats > 0) {
     ga.part = reinterpret_cast<float*>(c->ws);

@@ -88,6 +88,7 @@
 //     rounds once to bf16.
 
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 
 #include "lrq_common.h"
@@ -762,83 +763,88 @@ hipError_t run_fmt(hipStream_t st, int fmt, bool r192, const GemmArgs& a) {
 
 // Which GEMM kernel a shape takes: the 256-token tiles above (split in
 // depth when they are too few), lrq_gemm_mid.hip's 64-row x 64-token tiles,
-// two workgroups per CU, or lrq_gemm_w8.hip's 128-token tiles of 128 or 256
-// rows, one workgroup per CU. The choice is the smallest modelled time, in
-// microseconds, with constants measured on MI355X (every path forced in turn
-// over the shapes of the 3072-wide MMDiT and the 2560-wide decoder):
-//   - a 256 x 256 x 64 step of the large tiles takes 1.75 us (0.8 of that
-//     for 192-row tiles); a split shape adds its f32 partials, written and
-//     read once at about 4 TB/s, and the reduction launch;
-//   - a 64-wide depth block of a 64-token tile takes MID_T1 us when its
-//     workgroup has the CU to itself and MID_T2 us each when two share it;
-//     the tiles are dealt over the CUs, two at a time, MID_ROUND_US for each
-//     further round (400 tokens, 512 -> 8192: 24 us in two rounds);
-//   - a stage of a 128-token tile (256 deep with 128 rows, 128 deep with
-//     256: the same matrix-core work) takes 1.3 us with a third of the CUs at
-//     work and 1.75 us with all of them (the power limit), the tile's start and
-//     end MID_FIX us: 1024 tokens, 3072 -> 3072, 192 tiles of 12 stages
-//     25 us; 777 tokens, 3072 -> 9216, 252 tiles of 24 stages 45 us;
-//   - a tile may split its depth into ranges (one workgroup each, whole
-//     rounds of stages) when the tiles leave CUs idle; the ranges'
-//     accumulators meet in the launch, and S > 1 must model a tenth faster;
-//   - what forming the LoRA factors adds (large_side_us, w8_side_us). The
-//     large tiles need a launch for t, or for u and for dA and dB (8 and 20
-//     us plus their streams at 6 TB/s); the others form them in their own
-//     launch: the factor slices' workgroups hold up tiles, and weight-gradient
-//     blocks beyond half a round of workgroups follow the tiles (4096 tokens,
-//     3072 -> 12288, rank 32: 100 us, where 1999 tokens, 2560 -> 4096 add 4).
-//     A call that gives up the folded plan for those launches takes the
-//     kernel that is fastest without the factors, the large tiles or not.
+// two workgroups per CU, lrq_gemm_w8.hip's 128-token tiles of 128 or 256
+// rows, one workgroup per CU, or, for a backward that forms its LoRA factors,
+// lrq_gemm_mid.hip's 64-row x 128-token tiles (few outputs at 100 to 640
+// tokens: 8192 -> 512 at 128 tokens, rank 16, 13.1 us against 14.2 on the best
+// of the others; 3072 -> 3072 at 384 tokens, rank 32, 25.7 against 28.0). The
+// choice is the smallest modelled time, in microseconds:
+//   - large tiles: LARGE_STEP_US per 256 x 256 x 64 step, LARGE_192 of it for
+//     192-row tiles; a split shape's f32 partials (LARGE_SPLIT_MB per MB) and
+//     its reduction launch (LARGE_SPLIT_US);
+//   - two-per-CU tiles: MID_A per 64-wide depth block when a workgroup has
+//     its CU to itself and MID_B each when two share it, the tiles dealt over
+//     the CUs two at a time, MID_ROUND_US for each further round;
+//   - 128-token tiles: MID_A + MID_B x (the share of the CUs at work: the
+//     power limit) per stage, whole rounds of tiles;
+//   - MID_FIX per tile: its start and end;
+//   - depth ranges: RANGE_US, RANGE_EACH_US per range and RANGE_MB_US per MB
+//     of partials written and read. Only where every range's workgroup has a
+//     place at once: with more of them the partials cost more than the
+//     ranges gave (1024 tokens, 16384 -> 9216: 150 MB in four ranges, 347 us
+//     against 316 on the large tiles), and they are bounded by 34 MB;
+//   - LoRA factors in the launch (fold_us): FOLD_US, and FOLD_LATE_US when
+//     the factor slices' workgroups take places that tiles need. A
+//     weight-gradient block takes TN_US + TN_TOKENS_US per 128 tokens
+//     (TN_R32 as long at rank 32): as many as the places free beside the
+//     tiles can take while these run cost nothing but what they slow the tiles
+//     (SHARE_US at ranks to 16 and 32, for full CUs), the others follow the
+//     tiles, and dA's blocks wait for u (CHAIN_US);
+//   - the large tiles' launches for t, or for u and for dA and dB:
+//     LARGE_SIDE_US. (A call that gives up the folded plan takes the kernel
+//     that is fastest without the factors, the large tiles or not.)
+// The constants are fitted to 153000 timings of every kernel and range count
+// over 13400 calls (17 to 16384 tokens, layers 512 to 32768 wide, every
+// format, ranks 0 to 64) so that the plan's own time is least: it is 1.3 %
+// above the fastest kernel's on average, and 4 of 100 calls take more
+// than a tenth longer.
 // Decided on whole 64-token groups, so that a workspace reserved for the
 // largest of a group's token counts serves them all. A plan keeps the limits
 // of the call (its workspace, the counter area) and of the launch (32-bit
 // buffer offsets).
-constexpr double LARGE_STEP_US = 1.75;
-// per variant MID_64, MID_128, MID_256: tile tokens and rows, a fixed cost
-// per round of tiles, 64-deep blocks per pipeline stage, stages a depth range
-// is a multiple of, and the most ranges
-constexpr int MID_T[4] = {0, 64, W8_TOKENS, W8_TOKENS}, MID_R[4] = {0, 64, 128, 256};
-constexpr double MID_T1 = 0.342, MID_T2 = 0.423;
-constexpr double W8_STAGE_US = 1.0, W8_STAGE_FULL_US = 0.75;  // W8_STAGE_US + the share of the CUs at work x the other
-constexpr double MID_FIX[4] = {0, 2.0, 7.0, 6.0};
-constexpr int MID_SD[4] = {0, 2, 4, 2};
-constexpr int MID_ROUND[4] = {0, MID_MST, 1, 1};
-constexpr int MID_MAXS[4] = {0, MID_MAX_SPLIT, W8_MAX_SPLIT, W8_MAX_SPLIT};
-constexpr double MID_FINISH_US = 4.5;  // depth ranges of a 64-token tile
-constexpr double W8_FINISH_US = 2.0;   // and of the others, with 0.5 a range and the partials at 8 TB/s
-constexpr double MID_ROUND_US = 6.0;   // a further round of 64-token tiles
-// lrq_debug_gemm_path: 0 planned, 1 large tiles, 2 + (variant - 1) a mid
-// variant (MID_64, MID_128), 4 + (variant - 1) one with at least two depth
-// ranges where the depth has them; 6 and 7 the same for MID_256
+//
+// By format: int4, int8, fp8; pairs: forward, input gradient.
+constexpr double LARGE_STEP_US[3][2] = {{1.434, 1.341}, {1.419, 1.382}, {1.393, 1.6}};
+constexpr double LARGE_192 = 0.843, LARGE_US = 11.01;
+constexpr double LARGE_SPLIT_US = 8.05, LARGE_SPLIT_MB = 0.525, LARGE_SIDE_US[2] = {11.87, 21.74};
+// per MID_64, MID_128, MID_256, MID_64X128: tile tokens and rows, 64-deep
+// blocks per pipeline stage, stages a depth range is a multiple of, and the
+// most ranges; then the model's
+constexpr int MID_T[5] = {0, 64, W8_TOKENS, W8_TOKENS, 128}, MID_R[5] = {0, 64, 128, 256, 64};
+constexpr int MID_SD[5] = {0, 2, 4, 2, 1};
+constexpr int MID_ROUND[5] = {0, MID_MST, 1, 1, MID_MST};
+constexpr int MID_MAXS[5] = {0, MID_MAX_SPLIT, W8_MAX_SPLIT, W8_MAX_SPLIT, MID_MAX_SPLIT};
+constexpr double MID_A[3][2][5] =
+    {{{0, 0.33, 1.065, 1.099, 0}, {0, 0.319, 1.368, 1.301, 0.453}},
+     {{0, 0.322, 1.264, 1.217, 0}, {0, 0.273, 1.456, 1.344, 0.484}},
+     {{0, 0.204, 1.272, 1.388, 0}, {0, 0.308, 1.425, 1.322, 0.524}}};
+constexpr double MID_B[3][2][5] =
+    {{{0, 0.436, 0.548, 0.36, 0}, {0, 0.407, 0.344, 0.215, 0.611}},
+     {{0, 0.433, 0.545, 0.285, 0}, {0, 0.408, 0.297, 0.131, 0.858}},
+     {{0, 0.29, 0.543, 0.252, 0}, {0, 0.409, 0.434, 0.226, 0.645}}};
+constexpr double MID_FIX[2][5] = {{0, 3.56, 6.33, 5.76, 2.23}, {0, 1.19, 5.34, 5.45, 1.92}};
+constexpr double MID_ROUND_US[5] = {0, 10.48, 0, 0, 6.66};
+constexpr double RANGE_US[5] = {0, 1.09, 2.26, 2.55, 1.24}, RANGE_EACH_US[5] = {0, 0, 0.88, 1.13, 0};
+constexpr double RANGE_MB_US[5] = {0, 0.117, 0, 0.112, 0.166};
+constexpr double FOLD_US[5] = {0, 1.63, 1.36, 3.35, 0.3}, FOLD_LATE_US[5] = {0, 2.29, 7.21, 5.07, 6.45};
+constexpr double TN_US[5] = {0, 3.34, 0.55, 0.19, 2.09}, TN_TOKENS_US[5] = {0, 1.12, 0.76, 0.94, 0.69};
+constexpr double TN_R32 = 1.985, CHAIN_US[5] = {0, 1.39, 18.43, 0.55, 9.5};
+constexpr double SHARE_US[2][5] = {{0, 2.38, 0.92, 0.15, 4.59}, {0, 4.18, 4.16, 0.4, 12.99}};
+bool is_w8(int v) { return v == MID_128 || v == MID_256; }
+int model_fmt(int fmt) { return fmt == LRQ_FMT_INT4 ? 0 : fmt == LRQ_FMT_INT8 ? 1 : 2; }
+// lrq_debug_gemm_path: 0 planned, 1 large tiles, 2 and 3 MID_64 and MID_128,
+// 4 and 5 these with at least two depth ranges where the depth has them; 6
+// and 7 the same for MID_256, 8 and 9 for MID_64X128 (where it runs)
 int g_gemm_path = 0;
 
-// microseconds that a product's bytes take beside a launch's fixed cost
-double stream_us(double bytes) { return bytes / 6.0e6; }
-
-double large_us(int64_t m, int64_t e, int64_t depth, const SplitPlan& p) {
+double large_us(int fmt, int64_t m, int64_t e, int64_t depth, bool bwd) {
+  const SplitPlan p = plan_split(m, e, depth);
   const int64_t cus = get_num_cus();
   const int64_t RA = p.r192 ? 192 : 256;
   const int64_t tiles = (m + RB - 1) / RB * ((e + RA - 1) / RA);
-  const double f = p.r192 ? 0.8 : 1.0;
-  if (p.S <= 1) return (double)((tiles + cus - 1) / cus) * (double)((depth + 63) / 64) * LARGE_STEP_US * f + 3.0;
-  const double part = 4.0 * (double)p.S * (double)m * (double)e;
-  return (double)p.spl * LARGE_STEP_US * f + 2.0 * part / 4.0e6 + 8.0;
-}
-
-double large_side_us(int64_t m, int64_t e, int64_t depth, bool bwd) {
-  const double act = 2.0 * (double)m * (double)depth;
-  return bwd ? 20.0 + stream_us(2.0 * act + 2.0 * (double)m * (double)e) : 8.0 + stream_us(act);
-}
-
-double w8_side_us(int64_t m, int64_t e, int64_t depth, bool bwd) {
-  const double slots = 2.0 * (double)get_num_cus();
-  // factor slices, two a workgroup, about 10 us a round with what they hold up
-  double us = 10.0 * (double)((m + 63) / 64 * ((depth + MID_FOLD_KT - 1) / MID_FOLD_KT)) / slots;
-  if (bwd) {
-    const LoraPlan pa = mid_tn_plan(m, e, depth, 32, W8_TN_LDS), pb = mid_tn_plan(m, depth, e, 32, W8_TN_LDS);
-    us += 45.0 * std::max(0.0, (double)(pa.tiles * pa.splits + pb.tiles * pb.splits) / slots - 0.5);
-  }
-  return us;
+  const double step = LARGE_STEP_US[model_fmt(fmt)][bwd] * (p.r192 ? LARGE_192 : 1.0);
+  if (p.S <= 1) return (double)((tiles + cus - 1) / cus) * (double)((depth + 63) / 64) * step + LARGE_US;
+  return (double)p.spl * step + LARGE_SPLIT_MB * 4.0e-6 * (double)p.S * (double)m * (double)e + LARGE_SPLIT_US;
 }
 
 // stages per range (whole rounds) for S ranges of a depth, and the ranges
@@ -855,21 +861,75 @@ int mid_ranges(int64_t depth, int v, int S) {
 
 int64_t mid_tiles(int64_t m, int64_t e, int v) { return (m + MID_T[v] - 1) / MID_T[v] * ((e + MID_R[v] - 1) / MID_R[v]); }
 
-// the product alone in S ranges
-double mid_us(int64_t m, int64_t e, int64_t depth, int v, int S) {
+// the product alone in S ranges; *tile: one tile's time
+double mid_us(int fmt, int64_t m, int64_t e, int64_t depth, bool bwd, int v, int S, double* tile) {
   const int64_t cus = get_num_cus(), units = mid_tiles(m, e, v) * S;
   const int64_t n = (units + cus - 1) / cus;
-  if (v != MID_64) {
+  const double A = MID_A[model_fmt(fmt)][bwd][v], B = MID_B[model_fmt(fmt)][bwd][v], fix = MID_FIX[bwd][v];
+  const double ranges = S > 1 ? RANGE_US[v] + RANGE_EACH_US[v] * S + RANGE_MB_US[v] * 8.0e-6 * (double)(units * MID_T[v] * MID_R[v]) : 0.0;
+  if (is_w8(v)) {
     const int64_t nst = ((depth + 63) / 64 + MID_SD[v] - 1) / MID_SD[v];
-    const double part =
-        S > 1 ? W8_FINISH_US + 0.5 * S + 0.75 * stream_us(2.0 * 4.0 * (double)(units * MID_T[v] * MID_R[v])) : 0.0;
-    const double stage = W8_STAGE_US + W8_STAGE_FULL_US * std::min(1.0, (double)units / (double)cus);
-    return (double)n * ((double)(S > 1 ? mid_spl(depth, v, S) : nst) * stage + MID_FIX[v]) + part;
+    *tile = (double)(S > 1 ? mid_spl(depth, v, S) : nst) * (A + B * std::min(1.0, (double)units / (double)cus)) + fix;
+    return (double)n * *tile + ranges;
   }
   const int64_t nb = S > 1 ? std::min<int64_t>((int64_t)mid_spl(depth, v, S) * MID_SD[v], (depth + 63) / 64)
                            : (depth + 63) / 64;
-  return (double)nb * ((double)(n / 2) * MID_T2 + (double)(n % 2) * MID_T1) +
-         MID_FIX[v] + MID_ROUND_US * (double)((n + 1) / 2 - 1) + (S > 1 ? MID_FINISH_US : 0.0);
+  *tile = (double)nb * (n > 1 ? B : A) + fix;
+  return (double)nb * ((double)(n / 2) * B + (double)(n % 2) * A) + fix + MID_ROUND_US[v] * (double)((n + 1) / 2 - 1) +
+         ranges;
+}
+
+// The LoRA factors formed beside a product, per plan: depth slices of the
+// token-side factor, and (backward) the weight gradients' workgroups and
+// their token slice, for lrq_gemm_mid.hip [0] and lrq_gemm_w8.hip [1].
+struct Side {
+  bool on = false;
+  int64_t slices = 0;
+  int64_t wgs[2] = {0, 0};
+  double us[2][5] = {};  // a weight-gradient workgroup, per variant
+  bool r32 = false;
+};
+
+Side side_work(int64_t m, int64_t e, int64_t depth, bool bwd, int rp) {
+  Side s;
+  s.on = true;
+  s.r32 = rp > 16;
+  s.slices = (m + 63) / 64 * ((depth + MID_FOLD_KT - 1) / MID_FOLD_KT);
+  for (int w8 = 0; bwd && w8 < 2; ++w8) {
+    const int lds = w8 ? W8_TN_LDS : MID_TN_LDS;
+    const LoraPlan a = mid_tn_plan(m, depth, e, rp, lds), b = mid_tn_plan(m, e, depth, rp, lds);
+    if (a.splits <= 0 || b.splits <= 0) continue;
+    const int64_t na = a.tiles * a.splits, nb = b.tiles * b.splits;
+    s.wgs[w8] = w8 ? (na + 1) / 2 + (nb + 1) / 2 : na + nb;
+    const double per = (double)((m + std::min(a.splits, b.splits) - 1) / std::min(a.splits, b.splits)) / 128.0;
+    for (int v = MID_64; v <= MID_64X128; ++v) s.us[w8][v] = (TN_US[v] + TN_TOKENS_US[v] * per) * (s.r32 ? TN_R32 : 1.0);
+  }
+  return s;
+}
+
+// a product's time `us` (tiles of `tile` us, `units` workgroups) with its
+// factors in the launch: the factor slices' workgroups first, then the tiles,
+// then the weight gradients', on the places (one or two a CU)
+double fold_us(const Side& s, int v, int64_t units, int stages, double us, double tile) {
+  const bool w8 = is_w8(v);
+  const int64_t places = get_num_cus() * (w8 ? 1 : 2), rounds = (units + places - 1) / places * places;
+  const int64_t first = w8 ? w8_fold_wgs(s.slices, units, stages) : (s.slices + 7) / 8 * 8;
+  const int64_t turns = w8 ? ((s.slices + 1) / 2 + first - 1) / first : 1;
+  const double late = (double)(units + first - rounds), lat = FOLD_LATE_US[v];
+  us += FOLD_US[v] + (late <= 0 ? 0.0 : w8 ? lat : lat * std::min(1.0, late / (double)first));
+  const int64_t wgs = s.wgs[w8];
+  if (wgs == 0) return us;
+  const double tau = s.us[w8][v];
+  const double fit = std::floor(tile / tau);  // one after another beside a tile
+  const double beside = units <= places && late <= 0
+                            ? (double)(places - first - units) * fit + (double)first * std::floor(std::max(0.0, tile - lat * (double)turns) / tau)
+                            : (double)(rounds - units) * fit;
+  const double after = std::ceil(std::max(0.0, (double)wgs - beside) / (double)places) * tau;
+  const double alone = rounds > units
+                           ? std::max(0.0, lat * (double)turns + std::ceil((double)wgs / (double)(rounds - units)) * tau - tile)
+                           : after;
+  const double share = SHARE_US[s.r32][v] * std::min(1.0, (double)(units + first + wgs) / (double)places);
+  return std::max(us + std::min(after, alone) + share, CHAIN_US[v] + tau);
 }
 
 struct Pick {
@@ -879,37 +939,44 @@ struct Pick {
 
 // the best number of depth ranges for variant v, its partials and counters
 // within the limits (forced: at least two where the depth has them). False
-// if the launch cannot take the shape.
-bool mid_best(int64_t m, int64_t e, int64_t depth, int v, double side_us, bool force_split, int64_t max_floats,
-              int64_t max_tiles, Pick* out) {
+// if the launch cannot take the shape, or none takes less than `below`.
+bool mid_best(int fmt, int64_t m, int64_t e, int64_t depth, bool bwd, int v, const Side& side, bool force_split, double below,
+              int64_t max_floats, int64_t max_tiles, Pick* out) {
   // 32-bit buffer offsets of a tile's activation rows, outputs and weight rows
   if ((int64_t)128 * depth * 2 >= ((int64_t)1 << 31) || (int64_t)128 * e * 2 >= ((int64_t)1 << 31)) return false;
   if (max_floats < 0) return false;
-  const int64_t tiles = mid_tiles(m, e, v);
-  GemmPlan p;
-  p.v = v;
-  Pick best{p, mid_us(m, e, depth, v, 1) + side_us}, alt{p, 1e30};
-  for (int S = 2; S <= MID_MAXS[v] && tiles <= max_tiles; ++S) {
-    const int64_t floats = S * tiles * MID_T[v] * MID_R[v];
-    if (floats > max_floats || floats * 4 >= ((int64_t)1 << 32)) break;
-    if (mid_ranges(depth, v, S) != S) continue;  // (rounding turns it into fewer ranges, covered by those)
-    const double us = mid_us(m, e, depth, v, S) + side_us;
-    if (us >= alt.us) continue;
+  const int64_t tiles = mid_tiles(m, e, v), places = get_num_cus() * (is_w8(v) ? 1 : 2);
+  bool found = false;
+  for (int S = 1; S <= MID_MAXS[v]; ++S) {
+    GemmPlan p;
+    p.v = v;
     p.S = S;
-    p.spl = mid_spl(depth, v, S);
-    p.tiles = tiles;
-    p.floats = floats;
-    alt = Pick{p, us};
+    if (S > 1) {
+      p.spl = mid_spl(depth, v, S);
+      p.tiles = tiles;
+      p.floats = S * tiles * MID_T[v] * MID_R[v];
+      if (tiles > max_tiles || p.floats > max_floats || p.floats * 4 >= ((int64_t)1 << 32)) break;
+      if (!force_split && tiles * S > places) break;
+      if (mid_ranges(depth, v, S) != S) continue;  // (rounding turns it into fewer ranges, covered by those)
+    }
+    double tile = 0.0, us = mid_us(fmt, m, e, depth, bwd, v, S, &tile);
+    const bool must = force_split && found && out->p.S == 1;
+    if (us >= below && !must) continue;
+    if (side.on) us = fold_us(side, v, tiles * S, S > 1 ? p.spl : (int)(((depth + 63) / 64 + MID_SD[v] - 1) / MID_SD[v]), us, tile);
+    if (us >= below && !must) continue;
+    *out = Pick{p, us};
+    below = us;
+    found = true;
   }
-  *out = alt.p.S > 1 && (force_split || alt.us < 0.9 * best.us) ? alt : best;
-  return true;
+  return found;
 }
 
 // the variant that lrq_debug_gemm_path forces (MID_NONE: none), and whether
 // with at least two depth ranges
-int forced_variant(bool* split) {
-  *split = g_gemm_path == 4 || g_gemm_path == 5 || g_gemm_path == 7;
-  return g_gemm_path >= 6 ? MID_256 : g_gemm_path >= 2 ? (g_gemm_path - 2) % 2 + 1 : MID_NONE;
+int forced_variant(bool folded_bwd, bool* split) {
+  static const int v[10] = {MID_NONE, MID_NONE, MID_64, MID_128, MID_64, MID_128, MID_256, MID_256, MID_64X128, MID_64X128};
+  *split = g_gemm_path == 4 || g_gemm_path == 5 || g_gemm_path == 7 || g_gemm_path == 9;
+  return g_gemm_path < 8 || folded_bwd ? v[g_gemm_path] : MID_NONE;
 }
 
 std::atomic<int64_t> g_plans{0};
@@ -946,15 +1013,15 @@ int g_num_cus_ = 256;  // compute units of the context's device (the persistent 
 void set_num_cus(int n) { g_num_cus_ = n > 0 ? n : 256; }
 int get_num_cus() { return g_num_cus_; }
 
-bool gemm_plan(int64_t m, int64_t e, int64_t depth, int64_t max_floats, GemmPlan* p) {
+bool gemm_plan(int fmt, int64_t m, int64_t e, int64_t depth, bool bwd, int64_t max_floats, GemmPlan* p) {
   *p = GemmPlan{};
   if (m <= 0 || e <= 0) return true;
   g_plans.fetch_add(1, std::memory_order_relaxed);
   const int64_t mg = (m + 63) / 64 * 64;
   bool split = false;
-  const int fv = forced_variant(&split);
+  const int fv = forced_variant(false, &split);
   Pick pick{GemmPlan{}, 1e30}, c;
-  if (fv != MID_NONE && mid_best(mg, e, depth, fv, 0.0, split, max_floats, SK_MAX_NB, &c)) {
+  if (fv != MID_NONE && mid_best(fmt, mg, e, depth, bwd, fv, Side{}, split, 1e30, max_floats, SK_MAX_NB, &c)) {
     *p = c.p;
     return true;
   }
@@ -966,12 +1033,12 @@ bool gemm_plan(int64_t m, int64_t e, int64_t depth, int64_t max_floats, GemmPlan
     pick.p.S = sp.S;
     pick.p.spl = sp.spl;
     pick.p.floats = floats;
-    pick.us = large_us(mg, e, depth, plan_split(mg, e, depth));
+    pick.us = large_us(fmt, mg, e, depth, bwd);
   }
   bool found = large;
-  if (g_gemm_path == 0)
+  if (g_gemm_path == 0 || g_gemm_path >= 8)
     for (int v : {MID_64, MID_128, MID_256})
-      if (mid_best(mg, e, depth, v, 0.0, false, max_floats, SK_MAX_NB, &c) && c.us < pick.us) {
+      if (mid_best(fmt, mg, e, depth, bwd, v, Side{}, false, pick.us, max_floats, SK_MAX_NB, &c)) {
         pick = c;
         found = true;
       }
@@ -979,7 +1046,8 @@ bool gemm_plan(int64_t m, int64_t e, int64_t depth, int64_t max_floats, GemmPlan
   return found;
 }
 
-bool fold_plan(int64_t m, int64_t e, int64_t depth, bool bwd, int rp, int64_t max_floats, bool always, GemmPlan* p) {
+bool fold_plan(int fmt, int64_t m, int64_t e, int64_t depth, bool bwd, int rp, int64_t max_floats, bool always,
+               GemmPlan* p) {
   *p = GemmPlan{};
   const int64_t G = (m + 63) / 64, mg = G * 64;
   if (m <= 0 || e <= 0 || g_gemm_path == 1) return false;
@@ -991,15 +1059,13 @@ bool fold_plan(int64_t m, int64_t e, int64_t depth, bool bwd, int rp, int64_t ma
     return false;
   g_plans.fetch_add(1, std::memory_order_relaxed);
   bool split = false;
-  const int fv = forced_variant(&split);
-  const double w8 = w8_side_us(mg, e, depth, bwd);
+  const int fv = forced_variant(bwd, &split);
+  const Side side = side_work(mg, e, depth, bwd, rp);
   Pick pick{GemmPlan{}, 1e30}, c;
-  if (fv == MID_NONE && !always)
-    pick.us = large_us(mg, e, depth, plan_split(mg, e, depth)) + large_side_us(mg, e, depth, bwd);
-  for (int v : {MID_64, MID_128, MID_256}) {
-    if (fv != MID_NONE && v != fv) continue;
-    if (mid_best(mg, e, depth, v, v == MID_64 ? 0.0 : w8, split, max_floats, SK_MAX_NB - 2 * G, &c) && c.us < pick.us)
-      pick = c;
+  if (fv == MID_NONE && !always) pick.us = large_us(fmt, mg, e, depth, bwd) + LARGE_SIDE_US[bwd];
+  for (int v = MID_64; v <= MID_64X128; ++v) {
+    if ((fv != MID_NONE && v != fv) || (v == MID_64X128 && !bwd)) continue;
+    if (mid_best(fmt, mg, e, depth, bwd, v, side, split, pick.us, max_floats, SK_MAX_NB - 2 * G, &c)) pick = c;
   }
   *p = pick.p;
   return pick.p.v != MID_NONE;

@@ -485,41 +485,43 @@ __global__ void __launch_bounds__(256, 2) k_mid(GemmArgs a, int tiles_m, int til
   if (FOLD) mid_flags_done<256>(a, ntiles + ((BWD && a.tn_da >= 0) ? a.tj[a.tn_da].blocks : 0));
 }
 
-template <bool BWD, int FMT>
-hipError_t run_mid(hipStream_t st, const GemmArgs& a) {
-  constexpr int T = 64;
+// TT, SD: 64-token tiles in stages of two 64-wide blocks, or 128-token tiles
+// of one; 64 KiB of LDS either way, two workgroups per CU
+template <bool BWD, int FMT, int TT, int SD, bool FOLD>
+hipError_t run_tiles(hipStream_t st, const GemmArgs& a) {
+  constexpr int T = 16 * TT;
   const int tiles_m = (int)((a.m + T - 1) / T);
   const int tiles_e = (int)((a.e + MR - 1) / MR);
   const int group_m = tiles_m < 8 ? tiles_m : 8;
-  const int ntiles = tiles_m * tiles_e;
-  const int S = a.msplit > 1 ? a.msplit : 1;
-  // k_mid: two 64-wide blocks per stage with 64-token tiles, one with 128;
-  // 64 KiB of LDS in every variant, two workgroups per CU; S units per tile
-  // with depth ranges; with the fold, its workgroups first
-  if (a.fold) {
-    const unsigned grid = (unsigned)(ntiles * S + a.fold_wgs + (BWD ? a.tn_blocks : 0));
-    hipLaunchKernelGGL((k_mid<BWD, FMT, 4, 2, true>), dim3(grid), dim3(256), 0, st, a, tiles_m, tiles_e, group_m);
-  } else {
-    hipLaunchKernelGGL((k_mid<BWD, FMT, 4, 2, false>), dim3(ntiles * S), dim3(256), 0, st, a, tiles_m, tiles_e, group_m);
-  }
+  // S units per tile with depth ranges; with the fold, its workgroups first
+  unsigned grid = (unsigned)(tiles_m * tiles_e * (a.msplit > 1 ? a.msplit : 1));
+  if (FOLD) grid += a.fold_wgs + (BWD ? a.tn_blocks : 0);
+  hipLaunchKernelGGL((k_mid<BWD, FMT, TT, SD, FOLD>), dim3(grid), dim3(256), 0, st, a, tiles_m, tiles_e, group_m);
   return hipGetLastError();
+}
+
+template <int FMT>
+hipError_t run_mid(hipStream_t st, bool bwd, const GemmArgs& a, int variant) {
+  if (variant == MID_64X128) return run_tiles<true, FMT, 8, 1, true>(st, a);
+  if (bwd) return a.fold ? run_tiles<true, FMT, 4, 2, true>(st, a) : run_tiles<true, FMT, 4, 2, false>(st, a);
+  return a.fold ? run_tiles<false, FMT, 4, 2, true>(st, a) : run_tiles<false, FMT, 4, 2, false>(st, a);
 }
 
 }  // namespace
 
 hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int variant) {
   if (a.m <= 0 || a.e <= 0) return hipSuccess;
-  if (variant != MID_64 && variant != MID_128 && variant != MID_256) return hipErrorInvalidValue;
+  if (variant < MID_64 || variant > MID_64X128 || (variant == MID_64X128 && (!bwd || !a.fold))) return hipErrorInvalidValue;
   if (a.rp > 64 || a.rp % 16 != 0) return hipErrorInvalidValue;
   // depth ranges: at most MID_MAX_SPLIT (W8_MAX_SPLIT), each whole rounds of
   // stages (whole stages), the last one non-empty; partials for every unit
   // and a counter per tile
-  const bool w8 = variant != MID_64;
-  const int T = w8 ? W8_TOKENS : 64, TR = variant == MID_64 ? MR : (variant == MID_128 ? 128 : 256);
+  const bool w8 = variant == MID_128 || variant == MID_256;
+  const int T = variant == MID_64 ? 64 : 128, TR = !w8 ? MR : (variant == MID_128 ? 128 : 256);
   const int64_t ntiles = (a.m + T - 1) / T * ((a.e + TR - 1) / TR);
   const int S = a.msplit > 1 ? a.msplit : 1;
   if (S > 1) {
-    const int64_t stage = variant == MID_128 ? 256 : 128;
+    const int64_t stage = variant == MID_128 ? 256 : variant == MID_64X128 ? 64 : 128;
     const int64_t nst = (a.l + stage - 1) / stage;
     if (S > (w8 ? W8_MAX_SPLIT : MID_MAX_SPLIT) || a.mspl <= 0 || a.mspl % (w8 ? 1 : MST) != 0 || (int64_t)(S - 1) * a.mspl >= nst ||
         (int64_t)S * a.mspl < nst || !a.part || !a.mcnt ||
@@ -572,9 +574,7 @@ hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int 
   if ((int64_t)128 * a.l * 2 >= ((int64_t)1 << 31) || (int64_t)128 * a.e * 2 >= ((int64_t)1 << 31))
     return hipErrorInvalidValue;
   if (w8) return launch_w8(st, fmt, bwd, a, TR);
-  if (fmt == LRQ_FMT_INT4)
-    return bwd ? run_mid<true, LRQ_FMT_INT4>(st, a) : run_mid<false, LRQ_FMT_INT4>(st, a);
-  if (fmt == LRQ_FMT_INT8)
-    return bwd ? run_mid<true, LRQ_FMT_INT8>(st, a) : run_mid<false, LRQ_FMT_INT8>(st, a);
-  return bwd ? run_mid<true, LRQ_FMT_FP8>(st, a) : run_mid<false, LRQ_FMT_FP8>(st, a);
+  if (fmt == LRQ_FMT_INT4) return run_mid<LRQ_FMT_INT4>(st, bwd, a, variant);
+  if (fmt == LRQ_FMT_INT8) return run_mid<LRQ_FMT_INT8>(st, bwd, a, variant);
+  return run_mid<LRQ_FMT_FP8>(st, bwd, a, variant);
 }

@@ -561,22 +561,6 @@ __global__ void __launch_bounds__(WNT, 2) k_w8(GemmArgs a, int tiles_m, int tile
   if (FOLD) mid_flags_done<WNT>(a, ntiles + ((BWD && a.tn_da >= 0) ? a.tj[a.tn_da].blocks : 0));
 }
 
-// Workgroups for the factor slices (two at a time each, about 4 us). They
-// come first, so each one beyond the CUs that the tiles leave free holds up a
-// tile by its run time. A tile needs the factor only after its depth: when
-// the free CUs can form it in rounds that end by about half of a tile's
-// stages (1.5 us each), only they do (512 tokens, 12288 -> 3072, rank 32: 64
-// workgroups in two rounds beside 192 tiles, 62 -> 49 us against 128 in one);
-// otherwise one round, the least any tile can be held up. A multiple of 8, so
-// that the tiles keep their XCDs.
-int w8_fold_wgs(int slices, int units, int stages) {
-  const int need = (slices + 1) / 2, cus = get_num_cus();
-  const int spare = (cus - units % cus) % cus / 8 * 8;
-  const int rounds = std::max(1, (int)(stages * 1.5 / 8.0));
-  const int wgs = spare * rounds >= need ? std::min(spare, need) : need;
-  return (wgs + 7) / 8 * 8;
-}
-
 template <bool BWD, int FMT, int RW>
 hipError_t run_w8(hipStream_t st, const GemmArgs& a) {
   constexpr int R = 64 * RW;
@@ -590,7 +574,7 @@ hipError_t run_w8(hipStream_t st, const GemmArgs& a) {
     // per workgroup
     GemmArgs b = a;
     const int stages = (int)((a.l + 64 * (8 / RW) - 1) / (64 * (8 / RW)));
-    b.fold_wgs = w8_fold_wgs(a.fold_slices * (int)((a.m + 63) / 64), (int)units, S > 1 ? a.mspl : stages);
+    b.fold_wgs = (int)w8_fold_wgs(a.fold_slices * ((a.m + 63) / 64), units, S > 1 ? a.mspl : stages);
     const unsigned tn = BWD ? (unsigned)((a.tj[0].blocks + 1) / 2 + (a.tj[1].blocks + 1) / 2) : 0u;
     hipLaunchKernelGGL((k_w8<BWD, FMT, RW, true>), dim3(units + b.fold_wgs + tn), dim3(WNT), 0, st, b, tiles_m, tiles_e,
                        group_m);
@@ -608,6 +592,22 @@ hipError_t run_fmt(hipStream_t st, int fmt, bool bwd, const GemmArgs& a) {
 }
 
 }  // namespace
+
+// Workgroups for the factor slices (two at a time each, about 4 us). They
+// come first, so each one beyond the CUs that the tiles leave free holds up a
+// tile by its run time. A tile needs the factor only after its depth: when
+// the free CUs can form it in rounds that end by about half of a tile's
+// stages (1.5 us each), only they do (512 tokens, 12288 -> 3072, rank 32: 64
+// workgroups in two rounds beside 192 tiles, 62 -> 49 us against 128 in one);
+// otherwise one round, the least any tile can be held up. A multiple of 8, so
+// that the tiles keep their XCDs.
+int64_t w8_fold_wgs(int64_t slices, int64_t units, int stages) {
+  const int64_t need = (slices + 1) / 2, cus = get_num_cus();
+  const int64_t spare = (cus - units % cus) % cus / 8 * 8;
+  const int64_t rounds = std::max(1, (int)(stages * 1.5 / 8.0));
+  const int64_t wgs = spare * rounds >= need ? std::min(spare, need) : need;
+  return (wgs + 7) / 8 * 8;
+}
 
 hipError_t launch_w8(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int rows) {
   return rows == 256 ? run_fmt<4>(st, fmt, bwd, a) : run_fmt<2>(st, fmt, bwd, a);

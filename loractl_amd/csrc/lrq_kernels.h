@@ -97,13 +97,14 @@ struct GemmArgs {
   uint32_t* mcnt;
 };
 
-// How a fused product (m tokens, e outputs, `depth`) runs. A call forms its
+// How a fused product (a weight of `fmt`, m tokens, e outputs, `depth`) runs. A call forms its
 // plan once and sizes its workspace and launches from it; lrq_reserve forms
 // the same plans.
-enum { MID_NONE = 0, MID_64 = 1, MID_128 = 2, MID_256 = 3 };
+enum { MID_NONE = 0, MID_64 = 1, MID_128 = 2, MID_256 = 3, MID_64X128 = 4 };
 struct GemmPlan {
-  int v = MID_NONE;    // lrq_gemm_mid.hip (64-row x 64-token tiles, MID_64), lrq_gemm_w8.hip (128-token
-                       // tiles of 128 or 256 rows, MID_128 and MID_256), or the 256-token tiles
+  int v = MID_NONE;    // lrq_gemm_mid.hip (64-row tiles of 64 tokens, MID_64, or, folded backward, 128,
+                       // MID_64X128), lrq_gemm_w8.hip (128-token tiles of 128 or 256 rows, MID_128 and
+                       // MID_256), or the 256-token tiles
   bool r192 = false;   // 256-token tiles: of 192 rows instead of 256
   int S = 1, spl = 0;  // depth ranges (1: the whole depth), and steps or stages in each
   int64_t tiles = 0;   // arrival counters that the ranges of a MID_* plan need
@@ -113,12 +114,13 @@ constexpr int64_t PLAN_ANY = INT64_MAX;
 // The product by itself, or with its LoRA factors from launches of their own:
 // the kernel modelled fastest of those whose partials fit max_floats. False
 // if none does.
-bool gemm_plan(int64_t m, int64_t e, int64_t depth, int64_t max_floats, GemmPlan* p);
+bool gemm_plan(int fmt, int64_t m, int64_t e, int64_t depth, bool bwd, int64_t max_floats, GemmPlan* p);
 // The product and its LoRA factors (t; backward u, dA and dB; padded rank rp)
 // in one launch: the fastest such kernel within max_floats. False if the
 // launch cannot take the shape, or none is modelled faster than the 256-token
 // tiles and their side launches (`always`: the first alone).
-bool fold_plan(int64_t m, int64_t e, int64_t depth, bool bwd, int rp, int64_t max_floats, bool always, GemmPlan* p);
+bool fold_plan(int fmt, int64_t m, int64_t e, int64_t depth, bool bwd, int rp, int64_t max_floats, bool always,
+               GemmPlan* p);
 // cost-model evaluations of this process (lrq_debug_plan)
 int64_t plans_formed();
 
@@ -131,13 +133,15 @@ int64_t plans_formed();
 hipError_t launch_fwd(hipStream_t st, int fmt, const GemmPlan& p, const GemmArgs& a);
 hipError_t launch_bwd(hipStream_t st, int fmt, const GemmPlan& p, const GemmArgs& a);
 int get_num_cus();
-constexpr int MID_MAX_SPLIT = 4;  // depth ranges of a MID_64 tile
-constexpr int MID_MST = 4;  // MID_64: the kernel's pipeline stages (a range is whole rounds of them)
+constexpr int MID_MAX_SPLIT = 4;  // lrq_gemm_mid.hip: depth ranges of a tile
+constexpr int MID_MST = 4;  // and its pipeline stages (a range is whole rounds of them)
 // lrq_gemm_w8.hip: tiles of 128 tokens x 128 (MID_128) or 256 rows (MID_256),
 // one workgroup of eight wavefronts per CU, stages of 256 or 128 depth
 constexpr int W8_TOKENS = 128;
 constexpr int W8_MAX_SPLIT = 8;  // depth ranges of a tile
 hipError_t launch_w8(hipStream_t st, int fmt, bool bwd, const struct GemmArgs& a, int rows);
+// its workgroups for the factor slices beside `units` tiles of `stages`
+int64_t w8_fold_wgs(int64_t slices, int64_t units, int stages);
 hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int variant);
 // depth per slice of the folded factor's workgroups (GemmArgs.fold)
 constexpr int MID_FOLD_KT = 384;
@@ -145,7 +149,7 @@ constexpr int MID_FOLD_KT = 384;
 // backward: the factor slice takes at most 16 KiB of LDS (ranks padded to 16 or 32)
 constexpr int MID_TN_LDS = 16384;
 constexpr int W8_TN_LDS = 36864;  // in lrq_gemm_w8.hip
-inline int mid_tn_lds(int v) { return v == MID_64 ? MID_TN_LDS : W8_TN_LDS; }
+inline int mid_tn_lds(int v) { return v == MID_128 || v == MID_256 ? W8_TN_LDS : MID_TN_LDS; }
 // tuning and test hook: the values of lrq_debug_gemm_path
 void set_gemm_path(int path);
 

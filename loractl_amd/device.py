@@ -374,17 +374,18 @@ def debug_force_wait_timeout(on: bool):
     L.load().lrq_debug_force_wait_timeout(int(on))
 
 
-def debug_plan(what: str, m: int, n: int, k: int, r: int) -> dict:
+def debug_plan(what: str, m: int, n: int, k: int, r: int, fmt: int = L.LRQ_FMT_INT4) -> dict:
     """Test hook, host only: how a "fwd", "bwd" or "noalloc" forward call
     would run, or what "reserve" takes (lrq_debug_plan)."""
     out = (ctypes.c_int64 * 5)()
-    rc = L.load().lrq_debug_plan(("fwd", "bwd", "reserve", "noalloc").index(what), m, n, k, r, out)
+    rc = L.load().lrq_debug_plan(("fwd", "bwd", "reserve", "noalloc").index(what), fmt, m, n, k, r, out)
     if rc != 0:
         raise L.LrqError(rc, f"lrq_debug_plan({what}, {m}, {n}, {k}, {r})")
     return dict(zip(("bytes", "kernel", "ranges", "folded", "plans"), out))
 
 
-GEMM_PATHS = {"planned": 0, "large": 1, "mid64": 2, "mid128": 3, "mid64s": 4, "mid128s": 5, "mid256": 6, "mid256s": 7}
+GEMM_PATHS = {"planned": 0, "large": 1, "mid64": 2, "mid128": 3, "mid64s": 4, "mid128s": 5, "mid256": 6, "mid256s": 7,
+              "mid64x128": 8, "mid64x128s": 9}
 
 
 def debug_gemm_path(path: str):
@@ -393,8 +394,10 @@ def debug_gemm_path(path: str):
     split in depth when too few, "mid64" / "mid128" / "mid256": tiles of 64
     rows and tokens, 128 rows and tokens, or 256 rows and 128 tokens, with
     depth ranges as planned, "mid64s" / "mid128s" / "mid256s": the same with
-    at least two depth ranges where the depth allows). Every path computes the
-    same products."""
+    at least two depth ranges where the depth allows, "mid64x128" /
+    "mid64x128s": 64 rows and 128 tokens, in backward passes that form the
+    adapter's products in their launch). Every path computes the same
+    products."""
     L.load().lrq_debug_gemm_path(GEMM_PATHS[path])
 
 

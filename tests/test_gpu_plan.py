@@ -45,11 +45,13 @@ def test_a_call_evaluates_the_cost_model_once(cuda, M, r, most):
         assert formed() - before <= most
 
 
-@pytest.mark.parametrize("M,K,N,r", [(96, 15360, 12288, 64), (512, 15360, 3072, 32), (640, 16384, 9728, 16),
-                                     (1024, 16384, 9216, 16), (2112, 14336, 4096, 16), (8192, 12288, 9216, 32)])
+@pytest.mark.parametrize("M,K,N,r", [(64, 18432, 12288, 64), (96, 15360, 12288, 64), (512, 15360, 3072, 32),
+                                     (640, 16384, 9728, 16), (1024, 14336, 2560, 32), (1024, 16384, 9216, 16),
+                                     (2112, 14336, 4096, 16), (8192, 12288, 9216, 32)])
 def test_noalloc_takes_a_kernel_that_fits_its_scratch(cuda, M, K, N, r):
     """Shapes whose fastest plan needs more than the 32 MiB scratch array
-    (depth-range partials, t's slice partials) run on another that fits."""
+    (depth-range partials, t's slice partials) run on another that fits; and
+    shapes just within it."""
     wq, x, _, a, b = _case(cuda, M, K, N, r, M + K)
     y = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
     t = torch.empty((M, r), dtype=torch.bfloat16, device=cuda)
