@@ -318,7 +318,10 @@ __global__ void __launch_bounds__(WNT, 2) k_w8(GemmArgs a, int tiles_m, int tile
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) fa[0][i] = wfrag(b ^ 1, i, 0);
-    __syncthreads();  // the next stage has landed, and this one's reads are done
+    // the next stage's copies have landed (said here: the compiler does not
+    // carry them over the loop's back edge), and this one's reads are done
+    __builtin_amdgcn_s_waitcnt(0xf70);  // vmcnt(0)
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < 4; ++j) fb[0][j] = xfrag(nxt, j, 0);
   };
@@ -326,6 +329,7 @@ __global__ void __launch_bounds__(WNT, 2) k_w8(GemmArgs a, int tiles_m, int tile
   dma(sx0, 0, 0, XL);
 #pragma unroll
   for (int i = 0; i < 2; ++i) fa[0][i] = wfrag(0, i, 0);
+  __builtin_amdgcn_s_waitcnt(0xf70);  // vmcnt(0)
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < 4; ++j) fb[0][j] = xfrag(sx0, j, 0);

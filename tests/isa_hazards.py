@@ -322,6 +322,30 @@ def stage_waits(k: Kernel) -> list:
     return out
 
 
+def unwaited_copies(k: Kernel) -> list:
+    """(copy, barrier) index pairs: a copy of global memory into LDS and an
+    s_barrier that some path reaches from it without an s_waitcnt vmcnt(0)
+    in between."""
+    succ, out = _successors(k), []
+    for i, ins in enumerate(k.insns):
+        if not _lds_copy(ins):
+            continue
+        stack, seen = list(succ[i]), set()
+        while stack:
+            j = stack.pop()
+            if j in seen:
+                continue
+            seen.add(j)
+            nxt = k.insns[j]
+            if nxt.mnem == "s_barrier":
+                out.append((i, j))
+                continue
+            m = _VMCNT.search(nxt.text) if nxt.mnem == "s_waitcnt" else None
+            if not (m and int(m.group(1)) == 0):
+                stack.extend(succ[j])
+    return out
+
+
 def compile_asm(src: str, include: str, out_dir: str) -> str:
     """Device assembly of one HIP source for gfx950, with the library's flags."""
     out = os.path.join(out_dir, os.path.splitext(os.path.basename(src))[0] + ".s")
