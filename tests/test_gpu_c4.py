@@ -98,9 +98,44 @@ def _steps(cfg, cuda, runs):
     return out
 
 
+def _rounding_flips(ref, got, tol):
+    """Whether what exceeds ``tol`` (of the peak) is bf16 roundings that went
+    the other way, at a site of one token: its dA is x^T u and its dB t^T dy
+    with u and dy rounded to bf16, so a value that the noise carries over a
+    rounding boundary moves its column of the gradient, each entry by one bf16
+    ulp (at most 2^-7 of it). A column past the bound is such a one, and few
+    are: near the peak, and next to a boundary."""
+    d, big = np.abs(got - ref), np.maximum(np.abs(got), np.abs(ref))
+    over = d > tol * np.abs(ref).max()
+    cols = over.any(0)
+    return bool((d[over] <= 2.0**-7 * (1 + 2.0**-6) * big[over]).all()) and cols.sum() <= max(2, cols.size // 100)
+
+
+def test_rounding_flips_are_single_ulps_of_few_columns():
+    """The check of the one-token sites takes one column an ulp off, and
+    neither two ulps, nor part of an entry's column in error, nor many."""
+    g = np.random.Generator(np.random.PCG64(3))
+    t, dy = g.standard_normal((32, 1)).astype(np.float32), O.bf16_round(g.standard_normal((1, 400)).astype(np.float32))
+    dy[0, 7] = 4.0
+    ref = t * dy
+
+    def moved(cols, ulps):
+        d = dy.copy()
+        d[0, cols] = (d[0, cols].view(np.uint32) + (ulps << 16)).view(np.float32)
+        return t * d
+
+    assert _rounding_flips(ref, moved([7], 1), 1e-3)
+    assert not _rounding_flips(ref, moved([7], 2), 1e-3)
+    assert not _rounding_flips(ref, moved(np.abs(dy[0]) > 0.5, 1), 1e-3)
+    worse = ref.copy()
+    worse[3, 7] *= 1.02
+    assert not _rounding_flips(ref, worse, 1e-3)
+
+
 def _compare(cfg, ref, got, tol):
     """Every adapter gradient of ``got`` within ``tol(path)`` of ``ref``
-    (peak-normalized), and the dead branch exactly zero."""
+    (peak-normalized; a modulation site's up to single bf16 roundings), and
+    the dead branch exactly zero."""
     paths = cfg.site_paths()
     assert len(ref) == len(got) == 2 * len(paths)
     last = cfg.layers - 1
@@ -117,7 +152,8 @@ def _compare(cfg, ref, got, tol):
         rn, gn = r.cpu().numpy(), g.cpu().numpy()
         dev = O.rel_deviation(gn, rn)
         worst = max(worst, dev)
-        assert dev <= tol(i) and O.cosine(gn, rn) >= 0.9999, (path, dev, tol(i))
+        ok = dev <= tol(i) or (path.endswith(".mod") and tol(i) >= 1e-3 and _rounding_flips(rn, gn, tol(i)))
+        assert ok and O.cosine(gn, rn) >= 0.9999, (path, dev, tol(i))
     return worst
 
 
@@ -139,20 +175,15 @@ def test_c4_width_checkpointed_step_matches_monolithic(cuda, monkeypatch):
 def test_c4_width_checkpointed_step_with_atomic_attention(cuda):
     """The same with the step's own attention kernels: the loss is equal (the
     forward kernels are deterministic); the gradients differ from the
-    monolithic step's by no more than two monolithic steps differ from each
-    other (the attention backward's atomic reduction order), or 1e-3."""
+    monolithic step's by no more than four times what two monolithic steps
+    differ from each other (the attention backward's atomic reduction order),
+    or 1e-3, or at the one-token sites by single bf16 roundings (seen: 1/231
+    of the peak, the ulp of 231, in 2 of 13 steps)."""
     cfg = MmditConfig(layers=2)
     (loss_m, gm), (loss_m2, gm2), (loss_c, gc) = _steps(cfg, cuda, ["monolithic", "monolithic", "checkpointed"])
     assert loss_c == loss_m == loss_m2
     noise = [0.0 if r is None else O.rel_deviation(g.cpu().numpy(), r.cpu().numpy()) for r, g in zip(gm, gm2)]
-    # A modulation site has one token: its dA is x^T u and its dB t^T dy with u
-    # and dy rounded to bf16, so a value that the noise carries over a rounding
-    # boundary moves a whole column of the gradient by one bf16 ulp. At the
-    # peak that is up to 2^-7 of it, whatever the other pair of steps shows
-    # (seen: 1/231 of the peak, the ulp of 231, in 2 of 13 steps). Sites with
-    # more tokens average such steps out.
-    ulp = [2.0**-7 if p.endswith(".mod") else 0.0 for p in cfg.site_paths()]
-    worst = _compare(cfg, gm, gc, lambda i: max(1e-3, 4.0 * noise[i], ulp[i // 2]))
+    worst = _compare(cfg, gm, gc, lambda i: max(1e-3, 4.0 * noise[i]))
     print(f"worst gradient deviation {worst:.3e}; monolithic-to-monolithic up to {max(noise):.3e}")
 
 
