@@ -15,6 +15,7 @@ missing library or symbol raises.
 from __future__ import annotations
 
 import ctypes
+import numbers
 import os
 from typing import Tuple
 
@@ -63,8 +64,9 @@ def rope_tables(L: int, head_dim: int, device, theta: float = 10000.0) -> Tuple[
     """(cos, sin) f32 ``[L, head_dim / 2]``: pair (2j, 2j+1) of position p
     turns by ``p * theta^(-2j / head_dim)``; the angles are formed in f64
     (on a GPU by one kernel on the current stream)."""
-    dev = torch.device(device)
-    if dev.type == "cuda" and head_dim > 0:
+    dev = None if device is None else torch.device(device)
+    counts = isinstance(L, numbers.Integral) and isinstance(head_dim, numbers.Integral)
+    if dev is not None and dev.type == "cuda" and counts and head_dim > 0:
         cos = torch.empty((L, (head_dim + 1) // 2), device=dev, dtype=torch.float32)
         sin = torch.empty_like(cos)
         with torch.cuda.device(cos.device):

@@ -61,3 +61,7 @@ def test_rope_tables_kernel_takes_what_the_host_takes(cuda):
     for got, ref in zip(rope_tables(70, 64, cuda, theta), rope_tables(70, 64, "cpu", theta)):
         assert float((got.cpu() - ref).abs().max()) <= 2.0**-24
     assert rope_tables(3, 0, cuda)[0].shape == rope_tables(3, 0, "cpu")[0].shape
+    # no device (the host's), and sizes that are whole but not integers
+    for got in (rope_tables(5, 64, None), rope_tables(5.0, 64.0, cuda), rope_tables(np.int64(5), np.int32(64), cuda)):
+        for t, ref in zip(got, rope_tables(5, 64, "cpu")):
+            assert t.shape == ref.shape and float((t.cpu() - ref).abs().max()) <= 2.0**-24
