@@ -29,8 +29,9 @@ def _weight(cuda, w, group=64):
 @pytest.mark.parametrize(
     "M,K,N,path",
     [(4, 3072, 12288, "planned"), (4, 1024, 4096, "planned"), (192, 1024, 1536, "mid64"), (256, 1152, 1024, "mid128"),
-     (200, 3072, 2560, "mid64s")],
-    ids=["whole-depth", "splits", "mid64-fold", "mid128-fold", "mid64-ranges-fold"],
+     (200, 3072, 2560, "mid64s"), (256, 1152, 1024, "mid256"), (256, 2304, 1024, "mid256s"), (200, 3072, 2560, "mid64x128")],
+    ids=["whole-depth", "splits", "mid64-fold", "mid128-fold", "mid64-ranges-fold", "mid256-fold", "mid256-ranges-fold",
+         "mid64x128-fold"],
 )
 def test_few_token_wait_timeout_is_reported_and_cleared(cuda, M, K, N, path):
     r = 16

@@ -195,14 +195,15 @@ def test_bias_epilogue(cuda):
     check("y+bias", y, y_ref)
 
 
-@pytest.mark.parametrize("path", ["large", "mid64", "mid128", "mid64s", "mid128s"])
+@pytest.mark.parametrize("path", ["large", "mid64", "mid128", "mid256", "mid64s", "mid128s", "mid256s"])
 @pytest.mark.parametrize("fmt,per_channel", [("int4", True), ("fp8", True), ("fp8", False), ("int8", True)])
 def test_split_depth_bias_and_scales(cuda, fmt, per_channel, path):
     """Few output tiles (M = 200, d_out = 3072). On the large tiles the depth
     is split into ranges whose f32 partials a reduction sums, and the bias
     and the forward fp8 channel scales (or the scalar) are applied there,
-    once; the mid-size tiles run the whole depth ("mid64s", "mid128s": in
-    depth ranges summed in the launch) and apply them in their epilogue."""
+    once; the mid-size tiles run the whole depth ("mid64s", "mid128s",
+    "mid256s": in depth ranges summed in the launch) and apply them in their
+    epilogue."""
     M, K, N, r = 200, 3072, 3072, 16
     g = torch.Generator(device=cuda).manual_seed(7)
     w = torch.randn(N, K, device=cuda, generator=g) * 0.02
@@ -244,7 +245,7 @@ def test_fp8_mid_forward_repeats(cuda, per_channel):
     b = (torch.randn(r, N, device=cuda, generator=g) * 1e-2).to(torch.bfloat16)
     xf = x.float()
     y_ref = (xf @ wdq.t() + 0.5 * (xf @ a.float()) @ b.float()).cpu().numpy()
-    for path in ("mid64", "mid128", "mid64s", "mid128s"):
+    for path in ("mid64", "mid128", "mid256", "mid64s", "mid128s", "mid256s"):
         outs = []
         for _ in range(3):
             with gemm_path(path):
@@ -405,16 +406,18 @@ PATH_SHAPES = [(37, 96, 72, 32), (130, 192, 520, 64), (300, 320, 264, 64), (513,
 
 
 @pytest.mark.parametrize("r", [33, 32, 24, 16, 8])
-@pytest.mark.parametrize("path", ["large", "mid64", "mid128", "mid64s", "mid128s"])
+@pytest.mark.parametrize("path", ["large", "mid64", "mid128", "mid256", "mid64s", "mid128s", "mid256s", "mid64x128",
+                                  "mid64x128s"])
 @pytest.mark.parametrize("fmt,per_channel", [("int4", True), ("int8", True), ("fp8", True), ("fp8", False)])
 @pytest.mark.parametrize("M,K,N,g", PATH_SHAPES)
 def test_gemm_paths_against_oracle(cuda, M, K, N, g, fmt, per_channel, path, r):
     """Every kernel path of m > 16 (the 256-token tiles, split in depth where
-    they are few, and the 64-row tiles of 64 or 128 tokens) on the same
-    inputs: y (with bias), t, dx, dA and dB of the fused site, and the plain
-    product and its input gradient, against the f64 oracle. At ranks 8, 16,
-    24 and 32 the 64-row tiles form t, u, dA and dB in their own launches; "mid64s"
-    and "mid128s" split their depth into ranges where it allows."""
+    they are few, the 64-token tiles, the 128-token tiles of 128 and 256 rows,
+    and, for backwards that form their factors, of 64) on the same inputs: y
+    (with bias), t, dx, dA and dB of the fused site, and the plain product and
+    its input gradient, against the f64 oracle. At ranks 8, 16, 24 and 32 all
+    but the 256-token tiles form t, u, dA and dB in their own launches; "...s"
+    split their depth into ranges where it allows."""
     w, x, a, b, dy = case_inputs(M, K, N, r, seed=7 * M + N + g)
     wq, wdq = _weight(w, fmt, g, cuda, per_channel)
     bias = np.linspace(-0.5, 0.5, N).astype(np.float32)

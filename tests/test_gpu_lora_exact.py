@@ -12,8 +12,9 @@ test checks that the last chunk contributes to a large share of them.
 Each case selects one kernel path of the library (256 CUs): the few-token
 kernels (m <= 16), the split-depth GEMM with 192-row tiles (m = 256, forced
 onto the large tiles), the tiled GEMM with 192-row and 256-row tiles
-(m = 4096), and the mid-size tiles of 64 and 128 tokens (forced, with a
-ragged token count), forward and backward. Ranks 16, 32, 33, 48 and 64
+(m = 4096), and the mid-size tiles of 64 and 128 tokens (of 128 and 256 rows,
+and the backward's of 64; forced, with a ragged token count), forward and
+backward. Ranks 16, 32, 33, 48 and 64
 cover one to four rank chunks and a padded chunk.
 """
 
@@ -42,6 +43,10 @@ PATHS = [
     ("mid 128-token tiles", 300, 1088, 1032, "mid128"),
     ("mid 64-token tiles, depth ranges", 200, 3072, 2560, "mid64s"),
     ("mid 128-token tiles, depth ranges", 256, 2560, 9728, "mid128s"),
+    ("mid 256-row tiles", 300, 1088, 1032, "mid256"),
+    ("mid 256-row tiles, depth ranges", 256, 2560, 9728, "mid256s"),
+    ("mid 64 x 128 backward", 300, 1088, 1032, "mid64x128"),
+    ("mid 64 x 128 backward, depth ranges", 200, 3072, 2560, "mid64x128s"),
 ]
 RANKS = [16, 32, 33, 48, 64]
 

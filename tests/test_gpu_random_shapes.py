@@ -99,8 +99,8 @@ def test_random_shape_base_bias_and_noalloc(cuda, M, K, N, r, fmt, grp):
     y = x W^T + bias (quant_matmul_t, crates/loractl-core/src/quant.rs's
     QuantBackend::quant_matmul_t), dx = dy W (its backward), and the LoRA
     forward with the bias through lrq_lora_fwd_noalloc, bit-identical to
-    lrq_lora_fwd where its fixed scratch holds the shape's workspace (else
-    it refuses the shape with LRQ_EINVAL)."""
+    lrq_lora_fwd where its fixed scratch holds that call's workspace (every
+    shape here; a larger one may run on another kernel)."""
     from loractl_amd._lib import LrqError
 
     g = torch.Generator(device=cuda).manual_seed(M * 137 + K * 5 + N + r)
@@ -168,14 +168,15 @@ def test_large_token_counts(cuda, M, K, N, r, fmt, grp):
     check("dB", db, (tb.t() @ dyf).cpu().numpy())
 
 
-@pytest.mark.parametrize("M,path", [(5, "planned"), (300, "mid64"), (300, "mid128"), (200, "mid64s"), (2048, "large")])
+@pytest.mark.parametrize("M,path", [(5, "planned"), (300, "mid64"), (300, "mid128"), (300, "mid256"), (300, "mid64x128"),
+                                    (200, "mid64s"), (200, "mid256s"), (2048, "large")])
 @pytest.mark.parametrize("grp", [256, 512])
 @pytest.mark.parametrize("fmt", ["int4", "int8"])
 def test_large_quant_blocks(cuda, fmt, grp, M, path):
     """Quant blocks of 256 and 512 (any power of two >= 32 that divides d_in
     is accepted; crates/loractl-core/src/quant.rs's group argument): the
     device quantization and dequantization are bit-exact against the oracle
-    (Q4S / Q8S with that block), and every kernel path (few-token, both
+    (Q4S / Q8S with that block), and every kernel path (few-token, the
     mid-size tiles, depth ranges, large tiles) gives y, t, dx, dA and dB
     within the tolerance. A block then spans four or eight of the kernels'
     64-deep steps, and in the transposed section four or eight 64-row
@@ -212,7 +213,8 @@ def test_large_quant_blocks(cuda, fmt, grp, M, path):
     check("dB", db, (tb.t() @ dyf).cpu().numpy())
 
 
-@pytest.mark.parametrize("path", ["mid64", "mid128", "mid64s", "mid128s", "large"])
+@pytest.mark.parametrize("path", ["mid64", "mid128", "mid256", "mid64x128", "mid64s", "mid128s", "mid256s", "mid64x128s",
+                                  "large"])
 @pytest.mark.parametrize("fmt", FORMATS)
 def test_mid_paths_repeat_bit_identical(cuda, fmt, path):
     """The mid-size tiles' pipelines count their copies per stage (one load

@@ -72,3 +72,38 @@ def test_factor_slices_in_rounds(cuda, path):
     t_ref = x.float() @ a.float()
     check("t", t, t_ref.cpu().numpy())
     check("y", y, (x.float() @ D.dequant(wq).t() + t_ref @ b.float()).cpu().numpy())
+
+
+@pytest.mark.parametrize("path", ["mid64s", "mid128s", "mid256s", "mid64x128s"])
+@pytest.mark.parametrize("fmt", ["int4", "fp8"])
+def test_depth_ranges_of_more_tiles_than_cus(cuda, path, fmt):
+    """Forced ranges where the tiles alone fill the CUs: ranges of a tile run
+    in different rounds, and the last to arrive sums them all."""
+    from loractl_amd import device as D
+
+    M, K, N, r = 1100, 4096, 4096, 16
+    g = torch.Generator(device=cuda).manual_seed(9)
+    w = torch.randn(N, K, device=cuda, generator=g) * 0.02
+    wq = D.compute_weight(D.quantize_int4(w, 64) if fmt == "int4" else D.quantize_fp8(w, True))
+    bf = torch.bfloat16
+    x, dy = (torch.randn(M, d, device=cuda, generator=g).to(bf) for d in (K, N))
+    a = (torch.randn(K, r, device=cuda, generator=g) * 0.01).to(bf)
+    b = (torch.randn(r, N, device=cuda, generator=g) * 0.1).to(bf)
+
+    def run():
+        y, t = D.lora_fwd(x, wq, a, b, 1.0)
+        return (y, t) + tuple(D.lora_bwd(x, dy, wq, a, b, 1.0, t))
+
+    with gemm_path(path):
+        got, again = run(), run()
+        plan = D.debug_plan("bwd", M, N, K, r, wq.fmt)
+    rows = {1: 64, 2: 128, 3: 256, 4: 64}[plan["kernel"]]
+    assert plan["ranges"] > 1 and plan["folded"]
+    assert -(-M // (64 if path == "mid64s" else 128)) * -(-K // rows) * plan["ranges"] > 256 * (2 if rows == 64 else 1)
+    for u, v in zip(got, again):
+        assert torch.equal(u, v)
+    W, xf, dyf, af, bff = D.dequant(wq), x.float(), dy.float(), a.float(), b.float()
+    t, u = xf @ af, dyf @ bff.t()
+    refs = (xf @ W.t() + t @ bff, t, dyf @ W + u @ af.t(), xf.t() @ u, t.t() @ dyf)
+    for name, v, ref in zip(("y", "t", "dx", "dA", "dB"), got, refs):
+        check(name, v, ref.cpu().numpy())
