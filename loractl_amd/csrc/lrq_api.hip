@@ -789,7 +789,6 @@ static int fwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, int64_t 
       // fold's)
       ga.fold = force_wait_timeout() ? -1 : 1;
       ga.fold_slices = (int)p.fs;
-      ga.fold_wgs = (int)round_up(p.fs * p.G, 8);
       ga.fpart = reinterpret_cast<float*>(ws);
       ga.fcnt = cnt;
       ga.part = p.ms > 0 ? ga.fpart + p.fp : nullptr;
@@ -918,7 +917,6 @@ static int bwd_impl(lrq_ctx* c, const lrq_weight* w, const uint16_t* x, const ui
       // launch
       ga.fold = force_wait_timeout() ? -1 : 1;
       ga.fold_slices = (int)p.fs;
-      ga.fold_wgs = (int)round_up(p.fs * p.G, 8);
       ga.fpart = tail;
       ga.fcnt = c->cnt;
       ga.lact = b;

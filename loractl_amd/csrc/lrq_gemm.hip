@@ -955,7 +955,7 @@ bool mid_best(int fmt, int64_t m, int64_t e, int64_t depth, bool bwd, int v, con
       p.spl = mid_spl(depth, v, S);
       p.tiles = tiles;
       p.floats = S * tiles * MID_T[v] * MID_R[v];
-      if (tiles > max_tiles || p.floats > max_floats || p.floats * 4 >= ((int64_t)1 << 32)) break;
+      if (tiles > max_tiles || p.floats > max_floats || p.floats * 4 > (int64_t)LRQ_OOB) break;
       if (!force_split && tiles * S > places) break;
       if (mid_ranges(depth, v, S) != S) continue;  // (rounding turns it into fewer ranges, covered by those)
     }

@@ -1,6 +1,6 @@
 // The two GEMMs of the quantized LoRA linear for mid token counts (the
 // token count that leaves the 256 x 256 tiles of lrq_gemm.hip too few to
-// fill the CUs), without splitting the depth:
+// fill the CUs), over the whole depth or a few ranges finished in the launch:
 //
 //   forward   y[m, n]  = x[m, k]  . bf16(dq(w))[n, k]^T (+bias) + t[m, :] . B[:, n]
 //   backward  dx[m, k] = dy[m, n] . bf16(dq(w))[n, k]            + u[m, :] . A[k, :]^T
@@ -10,10 +10,10 @@
 // kernels, as for the large tiles.)
 //
 // "Rows" are the output columns (n forward, k backward), "depth" the
-// reduction index. A tile is 64 rows x 64 tokens (T = 16 TT) over the whole
-// depth, one workgroup of four wavefronts, two workgroups per CU (its
-// 128-token tiles gave way to lrq_gemm_w8.hip's: 1024 tokens, 3072 -> 3072,
-// rank 16, forward 39 -> 29 us):
+// reduction index. A tile is 64 rows x 64 tokens (T = 16 TT; in backwards
+// that form their factors also 128), one workgroup of four wavefronts, two
+// workgroups per CU (elsewhere the 128-token tiles are lrq_gemm_w8.hip's: 1024
+// tokens, 3072 -> 3072, rank 16, forward 39 -> 29 us):
 //   - wavefront w owns rows 16w .. 16w+15 of the tile for all T tokens, so
 //     each weight element is dequantized once per tile and each dequantized
 //     fragment feeds TT matrix-core steps (v_mfma_f32_16x16x32_bf16, weight
@@ -494,9 +494,14 @@ hipError_t run_tiles(hipStream_t st, const GemmArgs& a) {
   const int tiles_e = (int)((a.e + MR - 1) / MR);
   const int group_m = tiles_m < 8 ? tiles_m : 8;
   // S units per tile with depth ranges; with the fold, its workgroups first
+  // (one per factor slice, a multiple of 8, so that the tiles keep their XCDs)
   unsigned grid = (unsigned)(tiles_m * tiles_e * (a.msplit > 1 ? a.msplit : 1));
-  if (FOLD) grid += a.fold_wgs + (BWD ? a.tn_blocks : 0);
-  hipLaunchKernelGGL((k_mid<BWD, FMT, TT, SD, FOLD>), dim3(grid), dim3(256), 0, st, a, tiles_m, tiles_e, group_m);
+  GemmArgs b = a;
+  if (FOLD) {
+    b.fold_wgs = (int)((a.fold_slices * ((a.m + 63) / 64) + 7) / 8 * 8);
+    grid += b.fold_wgs + (BWD ? a.tn_blocks : 0);
+  }
+  hipLaunchKernelGGL((k_mid<BWD, FMT, TT, SD, FOLD>), dim3(grid), dim3(256), 0, st, b, tiles_m, tiles_e, group_m);
   return hipGetLastError();
 }
 
@@ -525,18 +530,17 @@ hipError_t launch_mid(hipStream_t st, int fmt, bool bwd, const GemmArgs& a, int 
     const int64_t nst = (a.l + stage - 1) / stage;
     if (S > (w8 ? W8_MAX_SPLIT : MID_MAX_SPLIT) || a.mspl <= 0 || a.mspl % (w8 ? 1 : MST) != 0 || (int64_t)(S - 1) * a.mspl >= nst ||
         (int64_t)S * a.mspl < nst || !a.part || !a.mcnt ||
-        (int64_t)S * ntiles * T * TR * 4 >= ((int64_t)1 << 32))
+        (int64_t)S * ntiles * T * TR * 4 > (int64_t)LRQ_OOB)
       return hipErrorInvalidValue;
   }
-  // the fold: ranks 8 to 32 (multiples of 8, padded to 16 or 32), both raw factors, its output, partials and
-  // counters (groups' arrivals and flags within the counter area), and
-  // enough factor workgroups, whole groups of eight
+  // the fold: ranks 8 to 32 (multiples of 8, padded to 16 or 32), both raw
+  // factors, its output, partials and counters (groups' arrivals and flags
+  // within the counter area)
   if (a.fold) {
     const int64_t G = (a.m + 63) / 64;
     if ((a.rp != 16 && a.rp != 32) || a.r % 8 != 0 || a.r > a.rp || a.r <= a.rp - 16 || !a.lact || !a.lw ||
         !a.fout || a.fout_ld % 8 != 0 || a.fout_ld < a.r || a.fout_ld > a.rp || !a.fpart || !a.fcnt ||
-        2 * G > SK_MAX_NB || a.fold_wgs % 8 != 0 ||
-        a.fold_slices != (int)((a.l + MID_FOLD_KT - 1) / MID_FOLD_KT) || a.fold_wgs < a.fold_slices * G ||
+        2 * G > SK_MAX_NB || a.fold_slices != (int)((a.l + MID_FOLD_KT - 1) / MID_FOLD_KT) ||
         a.m * a.l * 2 > (int64_t)LRQ_OOB || a.m * a.fout_ld * 2 > (int64_t)LRQ_OOB ||
         (int64_t)a.fold_slices * G * 64 * a.rp * 4 > (int64_t)LRQ_OOB)
       return hipErrorInvalidValue;

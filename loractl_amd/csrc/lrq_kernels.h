@@ -64,9 +64,10 @@ struct GemmArgs {
   uint16_t* out;         // [m, e]
   float* part;           // depth ranges' partials: lrq_gemm.hip [S][m][e]; the mid-size tiles' own layout; or null
   int splits, spl;       // set by lrq_gemm.hip: depth ranges and steps per range
-  // lrq_gemm_mid.hip with the token-side LoRA factor formed in the same
-  // launch (fold != 0, rank 8 to 32, a multiple of 8): the first fold_wgs workgroups (a
-  // multiple of 8) form bf16(fscale . act . F) for 64-token groups over
+  // The mid-size tiles with the token-side LoRA factor formed in the same
+  // launch (fold != 0, rank 8 to 32, a multiple of 8): the first fold_wgs
+  // workgroups (a multiple of 8, set by the launch) form
+  // bf16(fscale . act . F) for 64-token groups over
   // fold_slices depth slices of MID_FOLD_KT (F = lact: forward A [l, r],
   // backward B [r, l]), sum the slices in order, store it to fout
   // [m][fout_ld] and publish a stamped ready flag per group; the tiles read
@@ -88,18 +89,18 @@ struct GemmArgs {
   // the counter area past the fold's [0, 2 G).
   TnArgs tj[2];
   int tn_blocks, tn_da;
-  // lrq_gemm_mid.hip with depth ranges (msplit in 2 .. MID_MAX_SPLIT): each
-  // tile's depth in msplit ranges of mspl stages (a multiple of 4; the last
+  // The mid-size tiles with depth ranges (msplit > 1): each tile's depth in
+  // msplit ranges of mspl stages (lrq_gemm_mid.hip: a multiple of 4; the last
   // range to the end), one workgroup each; their f32 accumulators go to
-  // `part` (msplit x tiles x tokens x 64), mcnt holds one arrival counter per
-  // tile (zero on entry and exit). Set by lrq_gemm.hip's planner.
+  // `part` (msplit x tiles x tokens x rows), mcnt holds one arrival counter per
+  // tile (zero on entry and exit). Set from the plan.
   int msplit, mspl;
   uint32_t* mcnt;
 };
 
-// How a fused product (a weight of `fmt`, m tokens, e outputs, `depth`) runs. A call forms its
-// plan once and sizes its workspace and launches from it; lrq_reserve forms
-// the same plans.
+// How a fused product (a weight of `fmt`, m tokens, e outputs, `depth`) runs.
+// A call forms its plan once and sizes its workspace and launches from it;
+// lrq_reserve forms the same plans.
 enum { MID_NONE = 0, MID_64 = 1, MID_128 = 2, MID_256 = 3, MID_64X128 = 4 };
 struct GemmPlan {
   int v = MID_NONE;    // lrq_gemm_mid.hip (64-row tiles of 64 tokens, MID_64, or, folded backward, 128,
@@ -217,7 +218,7 @@ LoraPlan lora_plan_nt(int64_t M, int64_t C, int rp);
 LoraPlan lora_plan_tn(int64_t M, int64_t C, int rp, int64_t other_c = 0);
 // tn slices that fit the mid-size backward's LDS (`lds` bytes for the factor
 // slice, mid_tn_lds): as few token slices as that allows, but in lrq_gemm_w8.hip
-// as many as keep this job's and the other's (other_c columns) within TN_BLOCKS
+// as many as keep this job's and the other's (other_c columns) within a block a CU
 LoraPlan mid_tn_plan(int64_t M, int64_t C, int64_t other_c, int rp, int lds);
 // out = bf16(s * sum over slices of p[m, c] * q(j, c)) as [M, rp] (columns
 // >= r zero) and/or [M, r], with q(j, c) = q[j * ldq + c] when qrow (B [r, n]),

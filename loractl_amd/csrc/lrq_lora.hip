@@ -325,10 +325,6 @@ LoraPlan lora_plan_nt(int64_t M, int64_t C, int rp) {
   return p;
 }
 
-// weight-gradient blocks of a mid-size backward on the 128-token tiles, at
-// most (two a workgroup, one workgroup a CU)
-constexpr int64_t TN_BLOCKS = 256;
-
 // tn: token slices (multiples of 128) so that the column tiles of every job
 // in the launch (this job's C and other_c, 0 when it runs alone) times the
 // slices fill at most the 512 workgroup slots (two resident per CU): a
@@ -355,7 +351,10 @@ LoraPlan mid_tn_plan(int64_t M, int64_t C, int64_t other_c, int rp, int lds) {
   const int64_t m = M > 0 ? M : 1;
   p.tiles = cdiv(C, 128);
   int64_t S = cdiv(m, cap);
-  if (lds > MID_TN_LDS) S = std::max(S, std::max(TN_BLOCKS / (p.tiles + cdiv(other_c, 128)), TN_BLOCKS / 2 / p.tiles));
+  // on the 128-token tiles a block per CU at most: two a workgroup, so that
+  // they take half of a round
+  const int64_t blocks = get_num_cus();
+  if (lds > MID_TN_LDS) S = std::max(S, std::max(blocks / (p.tiles + cdiv(other_c, 128)), blocks / 2 / p.tiles));
   p.per = 128 * cdiv(cdiv(m, std::max<int64_t>(S, 1)), 128);
   p.splits = (int)cdiv(m, p.per);
   return p;
